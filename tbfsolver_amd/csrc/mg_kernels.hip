@@ -1658,106 +1658,6 @@ __global__ void __launch_bounds__(1024) k_tail_lds(const TailPlan<T>* __restrict
     for (int t = threadIdx.x; t < n0; t += blockDim.x) gp[t] = p0[t];
 }
 
-// Dense bottom operator: G = (M + c 1 1^T)^-1 (I - 1 1^T / n) (-V), with
-// M = -V A the V-scaled symmetric matrix of poissMat.f90:746-763.  x = G q is the
-// Lagrange-constrained exact solve (poissMat.f90:246-259,467-503, sum x = 0).
-// Gauss-Jordan on the symmetric positive definite M + c 1 1^T, one workgroup.
-// A, B: the n x n work matrices, in HBM (W) or in LDS (bottoms of at most
-// kDenseLdsCells cells); int indices (n <= 512).
-template <class T, class PA>
-__device__ void dense_setup_body(const LevelDev<double>& L, const T* __restrict__ beta_t,
-                                 const double* __restrict__ vol, double* __restrict__ bet, PA A, PA B,
-                                 double* __restrict__ G)
-{
-    const int nx = L.nx, ny = L.ny, nz = L.nz;
-    const int nb = nx * ny * nz;
-    const int nn = nb * nb;
-    __shared__ double s_trace;
-    for (int t = threadIdx.x; t < nb; t += blockDim.x) bet[t] = (double)beta_t[t];
-    for (int t = threadIdx.x; t < nn; t += blockDim.x) {
-        A[t] = 0.0;
-        B[t] = ((t / nb) == (t % nb)) ? 1.0 : 0.0;
-    }
-    __syncthreads();
-    // rows of M: for each face with neighbour nb != c: M[c][nb] -= V a_f, M[c][c] += V a_f
-    for (int c = threadIdx.x; c < nb; c += blockDim.x) {
-        const int i = c % nx, r = c / nx, j = r % ny, k = r / ny;
-        int cc, e, w, n, s, f, b;
-        neighbours(i, j, k, nx, ny, nz, cc, e, w, n, s, f, b);
-        Coef<double> a = coefs<double>(L, bet, i, j, k, cc, e, w, n, s, f, b);
-        const double v = vol[c];
-        const int nbr[6] = {e, w, n, s, f, b};
-        const double af[6] = {a.aR, a.aL, a.aT, a.aB, a.aF, a.aK};
-        for (int q = 0; q < 6; ++q) {
-            if (nbr[q] == cc) continue;
-            A[c * nb + nbr[q]] -= v * af[q];
-            A[c * nb + c] += v * af[q];
-        }
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double tr = 0.0;
-        for (int c = 0; c < nb; ++c) tr += A[c * nb + c];
-        s_trace = (tr > 0.0 ? tr : 1.0) / ((double)nb * nb);
-    }
-    __syncthreads();
-    const double cshift = s_trace;
-    for (int t = threadIdx.x; t < nn; t += blockDim.x) A[t] += cshift;
-    __syncthreads();
-    // Gauss-Jordan without pivoting (SPD)
-    for (int piv = 0; piv < nb; ++piv) {
-        const double inv = 1.0 / A[piv * nb + piv];
-        __syncthreads();
-        for (int c = threadIdx.x; c < nb; c += blockDim.x) {
-            A[piv * nb + c] *= inv;
-            B[piv * nb + c] *= inv;
-        }
-        __syncthreads();
-        for (int t = threadIdx.x; t < nn; t += blockDim.x) {
-            const int r = t / nb, c = t - r * nb;
-            if (r == piv) continue;
-            const double fct = A[r * nb + piv];
-            if (c != piv) A[t] -= fct * A[piv * nb + c];
-            B[t] -= fct * B[piv * nb + c];
-        }
-        __syncthreads();
-        for (int r = threadIdx.x; r < nb; r += blockDim.x)
-            if (r != piv) A[r * nb + piv] = 0.0;
-        __syncthreads();
-    }
-    // G[i][j] = -V_j (B[i][j] - rowmean_i(B))
-    for (int r = threadIdx.x; r < nb; r += blockDim.x) {
-        double s = 0.0;
-        for (int c = 0; c < nb; ++c) s += B[r * nb + c];
-        s /= (double)nb;
-        for (int c = 0; c < nb; ++c) G[(size_t)r * nb + c] = -vol[c] * (B[r * nb + c] - s);
-    }
-}
-
-template <class T>
-__global__ void __launch_bounds__(1024) k_dense_setup(LevelDev<double> L, const T* __restrict__ beta_t,
-                                                     const double* __restrict__ vol, double* __restrict__ W,
-                                                     double* __restrict__ G)
-{
-    const int nb = L.nx * L.ny * L.nz;
-    double* A = W;                        // n x n: M + c 1 1^T, reduced to the identity
-    double* B = W + (size_t)nb * nb;      // n x n: identity, becomes the inverse
-    dense_setup_body<T>(L, beta_t, vol, W + 2 * (size_t)nb * nb, A, B, G);
-}
-
-// the same with A and B in LDS (dynamic, 16 n^2 bytes)
-constexpr int kDenseLdsCells = 63;
-template <class T>
-__global__ void __launch_bounds__(1024) k_dense_setup_lds(LevelDev<double> L, const T* __restrict__ beta_t,
-                                                         const double* __restrict__ vol, double* __restrict__ W,
-                                                         double* __restrict__ G)
-{
-    extern __shared__ double dense_smem[];
-    const int nb = L.nx * L.ny * L.nz;
-    const lds_ptr<double> A = (lds_ptr<double>)dense_smem;
-    dense_setup_body<T>(L, beta_t, vol, W + 2 * (size_t)nb * nb, A, A + nb * nb, G);
-}
-
 // ------------------------------------------------------------ host launches
 
 namespace {
@@ -2077,20 +1977,6 @@ int launch_tail(const TailPlan<T>* plan_dev, const int* done, size_t lds_bytes, 
     return TBFG_OK;
 }
 
-template <class T>
-int launch_dense_setup(const LevelDev<double>& L, const T* beta, const double* vol, double* work, double* G,
-                       void* stream)
-{
-    const int nb = L.nx * L.ny * L.nz;
-    if (nb <= kDenseLdsCells)
-        hipLaunchKernelGGL(k_dense_setup_lds<T>, dim3(1), dim3(1024), (size_t)nb * nb * 2 * sizeof(double), S(stream),
-                           L, beta, vol, work, G);
-    else
-        hipLaunchKernelGGL(k_dense_setup<T>, dim3(1), dim3(1024), 0, S(stream), L, beta, vol, work, G);
-    TBFG_HIP(hipGetLastError());
-    return TBFG_OK;
-}
-
 // explicit instantiations
 template int launch_pcg_dots<double>(size_t, const double*, const double*, const double*, int, PcgState*,
                                      const Reducer&, void*);
@@ -2148,9 +2034,5 @@ size_t tail_lds_capacity()
 }
 template size_t tail_lds_capacity<float>();
 template size_t tail_lds_capacity<double>();
-template int launch_dense_setup<double>(const LevelDev<double>&, const double*, const double*, double*, double*,
-                                        void*);
-template int launch_dense_setup<float>(const LevelDev<double>&, const float*, const double*, double*, double*,
-                                       void*);
 
 }  // namespace tbfg

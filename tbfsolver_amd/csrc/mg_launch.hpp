@@ -114,8 +114,5 @@ int launch_tail(const TailPlan<T>* plan_dev, const int* done, size_t lds_bytes, 
 // dynamic LDS the LDS-resident tail kernel may use on the current device (0: none)
 template <class T>
 size_t tail_lds_capacity();
-template <class T>
-int launch_dense_setup(const LevelDev<double>& L, const T* beta, const double* vol, double* work, double* G,
-                       void* stream);
 
 }  // namespace tbfg

@@ -21,6 +21,7 @@
 #include <type_traits>
 #include <utility>
 
+#include "dense.hpp"
 #include "mg_launch.hpp"
 
 using namespace tbfg;
@@ -411,7 +412,7 @@ int pcg_create(const tbfg_grid_desc* g, const tbfg_pcg_params* prm_in, tbfg_pcg*
     const HostLevel& B = h->hl[ntot - 1];
     const size_t nbc = B.cells();
     TBFG_TRY(h->G.alloc(nbc * nbc * 8));
-    TBFG_TRY(h->dwork.alloc((2 * nbc * nbc + nbc + 16) * 8));
+    TBFG_TRY(h->dwork.alloc(dense_work_doubles(nbc) * 8));
     {
         std::vector<double> vol(nbc);
         for (int k = 1; k <= B.n[2]; ++k)
