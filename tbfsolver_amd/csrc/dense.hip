@@ -312,6 +312,75 @@ __global__ void __launch_bounds__(256)
     for (int c = lane; c < n; c += 64) G[(size_t)r * n + c] = -vol[c] * (row[c] - s);
 }
 
+// x = G q, one wavefront per row, q staged in LDS.  Bound by reading G once (from
+// the MALL after the first application): 1152 cells, 10.6 MB.
+__global__ void __launch_bounds__(256)
+    k_dense_apply(int n, const double* __restrict__ G, const double* __restrict__ q, double* __restrict__ x,
+                  const int* done)
+{
+    __shared__ double sq[kDenseDirectCells];
+    if (done && *done) return;
+    for (int c = threadIdx.x; c < n; c += 256) sq[c] = q[c];
+    __syncthreads();
+    const int lane = threadIdx.x & 63, r = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (r >= n) return;
+    const double* row = G + (size_t)r * n;
+    double acc = 0.0;
+#pragma unroll 8
+    for (int c = lane; c < n; c += 64) acc += row[c] * sq[c];
+    for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+    if (lane == 0) x[r] = acc;
+}
+
+// The diagnostics of one such solve (tbfg_pcg_coarse_stats): the V-weighted norm of
+// its residual over that of the right-hand side projected onto the range of A
+// (q - (sum V q) / (n V)), counted as one inner iteration; a zero right-hand side
+// counts no call.  One workgroup, at most two cells per thread.
+__global__ void __launch_bounds__(1024)
+    k_dense_check(LevelDev<double> L, const double* __restrict__ beta, const double* __restrict__ vol,
+                  const double* __restrict__ q, const double* __restrict__ x, PcgState* st, const int* done)
+{
+    __shared__ double lds[32 * 2];
+    __shared__ double s_shift;
+    if (done && *done) return;
+    const int n = L.nx * L.ny * L.nz;
+    double v[2], qc[2], ax[2], sum[1] = {0.0};
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int c = (int)threadIdx.x + u * 1024;
+        v[u] = qc[u] = ax[u] = 0.0;
+        if (c < n) {
+            const OpRow o = op_row(L, beta, vol, c);
+            v[u] = vol[c];
+            qc[u] = q[c];
+            double a = 0.0;
+#pragma unroll
+            for (int f = 0; f < 6; ++f) a += o.va[f] * (x[o.nb[f]] - x[c]);
+            ax[u] = a / v[u];
+            sum[0] += v[u] * qc[u];
+        }
+    }
+    block_sum<1>(sum, lds);
+    if (threadIdx.x == 0) s_shift = sum[0] / (double)n;
+    __syncthreads();
+    double rr[2] = {0.0, 0.0};
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+        if ((int)threadIdx.x + u * 1024 < n) {
+            const double r0 = qc[u] - s_shift / v[u], r = r0 - ax[u];
+            rr[0] += v[u] * r0 * r0;
+            rr[1] += v[u] * r * r;
+        }
+    block_sum<2>(rr, lds);
+    if (threadIdx.x == 0 && rr[0] > 0.0) {
+        st->coarse_calls += 1;
+        st->coarse_iters += 1;
+        if (st->coarse_iters_max < 1) st->coarse_iters_max = 1;
+        const double rel = sqrt(rr[1] / rr[0]);
+        if (rel > st->coarse_res_max) st->coarse_res_max = rel;
+    }
+}
+
 int padded(int n) { return (n + kTile - 1) / kTile * kTile; }
 
 }  // namespace
@@ -346,6 +415,21 @@ int launch_dense_setup(const LevelDev<double>& L, const T* beta, const double* v
     TBFG_HIP(hipGetLastError());
     return TBFG_OK;
 }
+int launch_dense_solve(const LevelDev<double>& L, const double* beta, const double* vol, const double* G,
+                       const double* q, double* x, PcgState* st, const int* done, void* stream)
+{
+    hipStream_t s = (hipStream_t)stream;
+    const int n = L.nx * L.ny * L.nz;
+    if (n > kDenseDirectCells) {
+        set_error("launch_dense_solve: %d cells (at most %d)", n, kDenseDirectCells);
+        return TBFG_EINVAL;
+    }
+    hipLaunchKernelGGL(k_dense_apply, dim3(ceil_div(n, 4)), dim3(256), 0, s, n, G, q, x, done);
+    hipLaunchKernelGGL(k_dense_check, dim3(1), dim3(1024), 0, s, L, beta, vol, q, x, st, done);
+    TBFG_HIP(hipGetLastError());
+    return TBFG_OK;
+}
+
 template int launch_dense_setup<double>(const LevelDev<double>&, const double*, const double*, double*, double*,
                                         void*);
 template int launch_dense_setup<float>(const LevelDev<double>&, const float*, const double*, double*, double*,

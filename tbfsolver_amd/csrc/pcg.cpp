@@ -331,9 +331,23 @@ int pcg_create(const tbfg_grid_desc* g, const tbfg_pcg_params* prm_in, tbfg_pcg*
     if (prm.coarse_max_iter > 0 && ntot > h->nuser && level_cells(h->nuser - 1) > inner_lim &&
         !std::getenv("TBFG_INNER_IN_TAIL"))
         h->kin = h->nuser - 1;
+    // An FP64 coarsest level of at most kDenseDirectCells cells that the caller wants
+    // solved to round-off-like accuracy (a target of 1e-8 or less and the iterations
+    // to reach it: the defaults are 1e-10 and 40) is solved by its dense inverse,
+    // formed once per solve, instead of an inner CG in one workgroup: 1152 cells took
+    // 22 iterations of 50 us per application.  A looser target or fewer iterations ask
+    // for an inexact solve, which the inner CG still gives.
+    h->direct = prm.coarse_max_iter >= 40 && h->prm.coarse_tol <= 1e-8 && !h->mixed && ntot > h->nuser &&
+                h->kin < 0 && level_cells(h->nuser - 1) <= (size_t)kDenseDirectCells &&
+                level_cells(h->nuser - 1) <= tail_lim && prm.preconditioner == TBFG_PRECOND_MG &&
+                !std::getenv("TBFG_INNER_IN_TAIL");
+    if (h->direct) {
+        ntot = h->nuser;
+        h->ntot = ntot;
+    }
     const int t_cap = prm.coarse_max_iter > 0 && h->kin < 0 ? h->nuser - 1 : ntot - 1;
     int t0 = t_cap;
-    for (int l = h->kin >= 0 ? h->kin + 1 : 1; l < t_cap; ++l) {
+    for (int l = h->kin >= 0 ? h->kin + 1 : 1; l < t_cap && !h->direct; ++l) {
         size_t cells = 1;
         for (int a = 0; a < 3; ++a) cells *= (size_t)(g->n[a] >> l);
         if (cells <= tail_lim) {
@@ -423,7 +437,7 @@ int pcg_create(const tbfg_grid_desc* g, const tbfg_pcg_params* prm_in, tbfg_pcg*
         TBFG_TRY(upload(h->vol, vol.data(), nbc * 8));
     }
     // inner CG vectors and cell volumes of the coarsest user level
-    if (prm.coarse_max_iter > 0) {
+    if (prm.coarse_max_iter > 0 && !h->direct) {
         const HostLevel& U = h->hl[h->nuser - 1];
         const size_t nu = U.cells();
         TBFG_TRY(h->cx.alloc(nu * es));
@@ -688,10 +702,15 @@ static int vcycle(tbfg_pcg* h, const T0* r0, T** z, const T0* beta0, const int* 
                 TBFG_TRY(launch_resid_restrict<T, T>(geo<T>(h, l), b, q, cur[l], h->q[l + 1].as<T>(), done, stream));
             }
         }
-        if (h->kin >= 0)
+        if (h->kin >= 0) {
             TBFG_TRY(inner_solve<T>(h, stream));
-        else
+        } else if (std::is_same<T, double>::value && h->direct) {
+            TBFG_TRY(launch_dense_solve(h->tabd[t0]->view, h->beta[t0].as<double>(), h->vol.as<double>(),
+                                        h->G.as<double>(), h->q[t0].as<double>(), h->p[t0].as<double>(),
+                                        h->st.as<PcgState>(), done, stream));
+        } else {
             TBFG_TRY(launch_tail<T>(h->plan.as<TailPlan<T>>(), done, h->tail_lds, stream));
+        }
         for (int l = t0 - 1; l >= 0; --l) {
             const T* pc = (l + 1 < t0) ? cur[l + 1] : h->p[l + 1].as<T>();
             TBFG_TRY(launch_prolong_add<T>(geo<T>(h, l), pc, cur[l], done, stream));

@@ -15,6 +15,7 @@ struct tbfg_pcg {
     int ntot = 0;    // reference levels + sub-levels of the coarsest-solve hierarchy
     int t0 = 0;      // first level run by the tail kernel
     int kin = -1;    // coarsest user level when its solve runs as multi-workgroup kernels (too large for the tail)
+    bool direct = false;  // the coarsest user level is the last one, solved by its dense inverse
     size_t n0 = 0;   // finest cells
 
     std::vector<tbfg::HostLevel> hl;

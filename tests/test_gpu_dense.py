@@ -50,3 +50,32 @@ def test_dense_bottom_matches_oracle(torch_gpu, n, stretch, bottom):
     e = rel(to_host(z), zr)
     print("  rel error", e, flush=True)
     assert e < 1e-11
+
+
+@pytest.mark.parametrize("n,nlev,cells", [((48, 32, 48), 4, 144), ((48, 40, 48), 3, 1440), ((128, 64, 128), 4, 2048)])
+def test_direct_coarsest_solve_matches_inner_cg(torch_gpu, monkeypatch, n, nlev, cells):
+    """The reference algorithm with its coarsest level solved by the dense inverse and by
+    the inner CG (TBFG_INNER_IN_TAIL): the same outer iterations within one, pressures to
+    1e-12 residual equal to 1e-10; a looser coarse_tol or fewer iterations keep the CG."""
+    print("case direct coarsest", n, cells, flush=True)
+    g, go, q, beta = setup(n, 1)
+    b, r = to_dev(beta, torch_gpu), to_dev(q, torch_gpu)
+
+    def solve(**kw):
+        s = T.PCG(g, nLevels=nlev, tolPCG=1e-12, maxIterPCG=200, flexible=1, **kw)
+        psi = torch_gpu.zeros_like(r)
+        s.solvePCG(psi, b, r)
+        out = (s.iterations, s.coarse_stats(), to_host(psi))
+        assert s.converged
+        s.close()
+        return out
+
+    it, cs, psi = solve()
+    assert cs["calls"] >= it and cs["iters_max"] == 1 and cs["iters"] == cs["calls"] and cs["res_max"] <= 1e-10
+    assert solve(coarse_tol=1e-3)[1]["iters_max"] > 1
+    assert solve(coarse_max_iter=39)[1]["iters_max"] > 1
+    monkeypatch.setenv("TBFG_INNER_IN_TAIL", "1")
+    it_cg, cs_cg, psi_cg = solve()
+    print("  iterations", it, it_cg, cs, cs_cg, flush=True)
+    assert cs_cg["iters_max"] > 1 and abs(it - it_cg) <= 1
+    assert rel(psi, psi_cg) < 1e-10
