@@ -7,6 +7,7 @@
 // Staggered layout: ux, uz hold nx*ny*nz faces (face i between cells i and i+1,
 // face 0 == face nx by periodicity); uy holds nx*(ny+1)*nz faces, j = 0..ny,
 // with the walls at j = 0 and j = ny.
+#include <algorithm>
 #include <cstring>
 #include <map>
 #include <mutex>
@@ -163,114 +164,231 @@ __global__ void k_project_mg(FieldGeo G, double alpha_dt, const double* __restri
     }
 }
 
-// old-pressure level, absent on the first steps (then zero)
-__device__ __forceinline__ double old_level(const double* __restrict__ a, size_t i) { return a ? a[i] : 0.0; }
+// Old levels of the FAST splitting (poissonEqn.f90:255-301): psi^n (p1), psi^(n-1) (p2)
+// and the surface-tension levels st^n, st^(n-1), three staggered components each laid
+// out like the velocity.  A level, or a component, may be absent (then zero): its
+// pointer is that of another array and its bit in `has` is clear, so that every load is
+// unconditional (a branch around each load made the compiler wait for it there).
+struct OldLevels {
+    const double* p[2];     // psi^n, psi^(n-1)
+    const double* st[2][3]; // st^n, st^(n-1)
+    unsigned has;           // bit l: p[l]; bit 2 + 3 l + c: st[l][c]
+};
+// which levels a kernel reads: none, pressure, pressure and surface tension
+enum { kNoLevels = 0, kPsiLevels = 1, kAllLevels = 2 };
 
-// extrapolated old-pressure difference across a face: (2 (psi1_b - psi1_a) - (psi2_b - psi2_a)) / dc
-__device__ __forceinline__ double old_grad(const double* __restrict__ psi1, const double* __restrict__ psi2, size_t a,
-                                           size_t b, double dc)
+template <int MODE>
+__device__ __forceinline__ double old_psi(const OldLevels& o, int l, size_t i)
 {
-    return (2.0 * (old_level(psi1, b) - old_level(psi1, a)) - (old_level(psi2, b) - old_level(psi2, a))) / dc;
+    if (MODE == kNoLevels) return 0.0;
+    const double v = o.p[l][i];
+    return (o.has >> l) & 1u ? v : 0.0;
 }
 
-// Old surface-tension levels st^n (1) and st^(n-1) (2), three staggered
-// components laid out like the velocity; a NULL component is zero.
-struct StLevels {
-    const double* x1;
-    const double* y1;
-    const double* z1;
-    const double* x2;
-    const double* y2;
-    const double* z2;
+template <int MODE>
+__device__ __forceinline__ double old_st(const OldLevels& o, int l, int comp, size_t f)
+{
+    if (MODE != kAllLevels) return 0.0;
+    const double v = o.st[l][comp][f];
+    return (o.has >> (2 + 3 * l + comp)) & 1u ? v : 0.0;
+}
+
+// the face value G_f = (2 d psi^n - d psi^(n-1)) / dc - 2 st^n_f + st^(n-1)_f
+// (poissonEqn.f90:255-301, momentumEqn.f90:1104-1121), in the reference's order of
+// operations; a*, b* the values of the two levels on either side of the face
+template <int MODE>
+__device__ __forceinline__ double old_grad(double a1, double b1, double a2, double b2, double dc, double s1, double s2)
+{
+    if (MODE == kNoLevels) return 0.0;
+    const double g = (2.0 * (b1 - a1) - (b2 - a2)) / dc;
+    return MODE == kPsiLevels ? g : g - 2.0 * s1 + s2;
+}
+
+// Launch of the column kernels below: a thread owns the column (i, j) of a chunk of kc
+// planes and marches through it, so the values of the plane before and after stay in
+// registers (read once per chunk instead of once per z neighbour: at 192x128x192 a
+// plane of the up to 16 arrays is 3 MB, and the z neighbours fell out of the L2), and
+// the loads of the next plane are in flight while one is computed.  The in-plane
+// neighbours come from the tile's own rows (L1).  Tiles of 64 x 4 columns, or 32 x 8
+// where those leave fewer lanes idle; chunks for one resident round of workgroups
+// (three per CU by registers: 768), since a second, partly filled one costs as much as
+// a full one.  192x128x192 with every level, in a step: source 211 -> 145 us, projection
+// 153 -> 139 us (their bytes at the copy rate: 96 and 118 us).
+struct ColGrid {
+    dim3 blk;
+    unsigned nblocks;
+    int tiles_x, ntiles, kc;
 };
 
-// the face value G_f = old_grad - 2 st^n_f + st^(n-1)_f (poissonEqn.f90:255-301,
-// momentumEqn.f90:1104-1121), in the reference's order of operations
-__device__ __forceinline__ double with_st(double grad, const double* __restrict__ s1, const double* __restrict__ s2,
-                                          size_t f)
+static ColGrid column_grid(int nx, int ny, int nz)
 {
-    return grad - 2.0 * old_level(s1, f) + old_level(s2, f);
+    ColGrid c;
+    const bool wide = (nx + 63) / 64 * 64 <= (nx + 31) / 32 * 32;
+    c.blk = wide ? dim3(64, 4) : dim3(32, 8);
+    c.tiles_x = (int)ceil_div(nx, c.blk.x);
+    c.ntiles = c.tiles_x * (int)ceil_div(ny, c.blk.y);
+    const int chunks = std::max(1, std::min(nz, 768 / c.ntiles));
+    c.kc = (nz + chunks - 1) / chunks;
+    c.nblocks = (unsigned)c.ntiles * ceil_div(nz, c.kc);
+    return c;
+}
+
+// consecutive tiles of a chunk of planes on one XCD, as row_cell
+__device__ __forceinline__ void column_cell(int kc, int tiles_x, int ntiles, int nz, int& i, int& j, int& k0, int& k1)
+{
+    const unsigned nb = gridDim.x;
+    unsigned id = blockIdx.x;
+    if ((nb & 7u) == 0) id = (id & 7u) * (nb >> 3) + (id >> 3);
+    const int tile = (int)(id % (unsigned)ntiles);
+    k0 = (int)(id / (unsigned)ntiles) * kc;
+    k1 = min(nz, k0 + kc);
+    i = (tile % tiles_x) * (int)blockDim.x + (int)threadIdx.x;
+    j = (tile / tiles_x) * (int)blockDim.y + (int)threadIdx.y;
 }
 
 // FAST computeSource + computeOldPressDiv with two old levels (poissonEqn.f90:193-305):
 // s = rho0/(alpha dt) div u* + div[(1 - rho0 (1/rho)_f) G_f], G_f the face gradient of
 // 2 psi^n - psi^(n-1) minus 2 st^n_f - st^(n-1)_f; (1/rho)_f the arithmetic face mean.
 // The face after a cell reads the st values of the cell's own face index, the face
-// before it those of the previous face (in y the wall faces 0 and ny included).
-__global__ void k_source_fast(FieldGeo G, double r_adt, double rho0, const double* __restrict__ rho,
-                              const double* __restrict__ ux, const double* __restrict__ uy,
-                              const double* __restrict__ uz, const double* __restrict__ psi1,
-                              const double* __restrict__ psi2, StLevels st, double* __restrict__ s)
+// before it those of the previous face (in y the wall faces 0 and ny included).  The
+// flux and the velocity of the face after a cell in z are those of the face before the
+// next one: carried along the march.
+template <int MODE>
+__global__ void __launch_bounds__(256)
+    k_source_fast(FieldGeo G, double r_adt, double rho0, const double* __restrict__ rho,
+                  const double* __restrict__ ux, const double* __restrict__ uy, const double* __restrict__ uz,
+                  OldLevels o, double* __restrict__ s, int kc, int tiles_x, int ntiles)
 {
-    int i, j, k;
-    row_cell(G.nx, G.ny, i, j, k);
+    int i, j, k0, k1;
+    column_cell(kc, tiles_x, ntiles, G.nz, i, j, k0, k1);
     const int nx = G.nx, ny = G.ny, nz = G.nz;
-    if (i >= nx) return;
+    if (i >= nx || j >= ny) return;
     const size_t plane = (size_t)nx * ny;
-    const size_t c = i + (size_t)nx * j + plane * k;
-    const size_t e = (i + 1 < nx ? i + 1 : 0) + (size_t)nx * j + plane * k;
-    const size_t w = (i > 0 ? i - 1 : nx - 1) + (size_t)nx * j + plane * k;
-    const size_t n = i + (size_t)nx * (j + 1 < ny ? j + 1 : j) + plane * k;  // wall ghost = the cell
-    const size_t so = i + (size_t)nx * (j > 0 ? j - 1 : j) + plane * k;
-    const size_t f = i + (size_t)nx * j + plane * (k + 1 < nz ? k + 1 : 0);
-    const size_t b = i + (size_t)nx * j + plane * (k > 0 ? k - 1 : nz - 1);
-    const size_t yt = i + (size_t)nx * ((j + 1) + (size_t)(ny + 1) * k);  // y face after the cell
-    const size_t yb = yt - nx;                                             // y face before it
+    const size_t oc = i + (size_t)nx * j;
+    const size_t oe = (i + 1 < nx ? i + 1 : 0) + (size_t)nx * j;
+    const size_t ow = (i > 0 ? i - 1 : nx - 1) + (size_t)nx * j;
+    const size_t on = i + (size_t)nx * (j + 1 < ny ? j + 1 : j);  // wall ghost = the cell
+    const size_t os = i + (size_t)nx * (j > 0 ? j - 1 : j);
     const double dxf = G.df[0][0], dzf = G.df[2][0], dyf = G.df[1][j];
     const double dxc = G.dcn[0][0], dzc = G.dcn[2][0];
     const double dycp = G.dcn[1][j], dycm = G.dcn[1][j > 0 ? j - 1 : 0];
-    const double sv = div_cell(G, ux, uy, uz, i, j, k) * r_adt * rho0;
-    const double ic = 1.0 / rho[c];
-    const double apx = 1.0 - rho0 * 0.5 * (1.0 / rho[e] + ic);
-    const double amx = 1.0 - rho0 * 0.5 * (1.0 / rho[w] + ic);
-    const double apy = 1.0 - rho0 * 0.5 * (1.0 / rho[n] + ic);
-    const double amy = 1.0 - rho0 * 0.5 * (1.0 / rho[so] + ic);
-    const double apz = 1.0 - rho0 * 0.5 * (1.0 / rho[f] + ic);
-    const double amz = 1.0 - rho0 * 0.5 * (1.0 / rho[b] + ic);
-    const double gxp = with_st(old_grad(psi1, psi2, c, e, dxc), st.x1, st.x2, c);
-    const double gxm = with_st(old_grad(psi1, psi2, w, c, dxc), st.x1, st.x2, w);
-    const double gyp = with_st(old_grad(psi1, psi2, c, n, dycp), st.y1, st.y2, yt);
-    const double gym = with_st(old_grad(psi1, psi2, so, c, dycm), st.y1, st.y2, yb);
-    const double gzp = with_st(old_grad(psi1, psi2, c, f, dzc), st.z1, st.z2, c);
-    const double gzm = with_st(old_grad(psi1, psi2, b, c, dzc), st.z1, st.z2, b);
-    const double dx = (apx * gxp - amx * gxm) / dxf;
-    const double dy = (apy * gyp - amy * gym) / dyf;
-    const double dz = (apz * gzp - amz * gzm) / dzf;
-    s[c] = sv + dx + dy + dz;
+    // 1 - rho0 (1/rho)_f of the face between inverses a and b
+    auto weight = [&](double a, double b) { return 1.0 - rho0 * 0.5 * (b + a); };
+    const size_t pb = plane * (size_t)(k0 > 0 ? k0 - 1 : nz - 1), p0 = plane * k0 + oc;
+    double ic = 1.0 / rho[p0], c1 = old_psi<MODE>(o, 0, p0), c2 = old_psi<MODE>(o, 1, p0);
+    double fzm = weight(1.0 / rho[pb + oc], ic) *
+                 old_grad<MODE>(old_psi<MODE>(o, 0, pb + oc), c1, old_psi<MODE>(o, 1, pb + oc), c2, dzc,
+                                old_st<MODE>(o, 0, 2, pb + oc), old_st<MODE>(o, 1, 2, pb + oc));
+    double uzm = uz[pb + oc];
+    // the loads of a plane, issued while the plane before is computed
+    struct Plane {
+        double rf, re, rw, rn, rs;                            // density behind the faces (z-: the plane before)
+        double f1, f2, e1, e2, w1, w2, n1, n2, s1, s2;         // the two old pressures there
+        double uxc, uxw, uyt, uyb, uzc;
+        double x1, x2, m1, m2, t1, t2, b1, b2, z1, z2;         // surface tension: x+, x-, y+, y-, z+
+    };
+    auto load = [&](Plane& v, int k) {
+        const size_t pk = plane * k, f = plane * (size_t)(k + 1 < nz ? k + 1 : 0) + oc;
+        const size_t yt = i + (size_t)nx * ((j + 1) + (size_t)(ny + 1) * k);  // y face after the cell
+        const size_t yb = yt - nx;                                             // y face before it
+        const size_t c = pk + oc, e = pk + oe, w = pk + ow, n = pk + on, so = pk + os;
+        v.rf = rho[f], v.re = rho[e], v.rw = rho[w], v.rn = rho[n], v.rs = rho[so];
+        v.f1 = old_psi<MODE>(o, 0, f), v.f2 = old_psi<MODE>(o, 1, f);
+        v.e1 = old_psi<MODE>(o, 0, e), v.e2 = old_psi<MODE>(o, 1, e);
+        v.w1 = old_psi<MODE>(o, 0, w), v.w2 = old_psi<MODE>(o, 1, w);
+        v.n1 = old_psi<MODE>(o, 0, n), v.n2 = old_psi<MODE>(o, 1, n);
+        v.s1 = old_psi<MODE>(o, 0, so), v.s2 = old_psi<MODE>(o, 1, so);
+        v.uxc = ux[c], v.uxw = ux[w], v.uyt = uy[yt], v.uyb = uy[yb], v.uzc = uz[c];
+        v.x1 = old_st<MODE>(o, 0, 0, c), v.x2 = old_st<MODE>(o, 1, 0, c);
+        v.m1 = old_st<MODE>(o, 0, 0, w), v.m2 = old_st<MODE>(o, 1, 0, w);
+        v.t1 = old_st<MODE>(o, 0, 1, yt), v.t2 = old_st<MODE>(o, 1, 1, yt);
+        v.b1 = old_st<MODE>(o, 0, 1, yb), v.b2 = old_st<MODE>(o, 1, 1, yb);
+        v.z1 = old_st<MODE>(o, 0, 2, c), v.z2 = old_st<MODE>(o, 1, 2, c);
+    };
+    Plane v;
+    load(v, k0);
+    for (int k = k0; k < k1; ++k) {
+        Plane nxt;
+        load(nxt, min(k + 1, k1 - 1));
+        __builtin_amdgcn_sched_barrier(0);
+        const double div = (v.uxc - v.uxw) / dxf + (v.uyt - v.uyb) / dyf + (v.uzc - uzm) / dzf;
+        const double gxp = old_grad<MODE>(c1, v.e1, c2, v.e2, dxc, v.x1, v.x2);
+        const double gxm = old_grad<MODE>(v.w1, c1, v.w2, c2, dxc, v.m1, v.m2);
+        const double gyp = old_grad<MODE>(c1, v.n1, c2, v.n2, dycp, v.t1, v.t2);
+        const double gym = old_grad<MODE>(v.s1, c1, v.s2, c2, dycm, v.b1, v.b2);
+        const double gzp = old_grad<MODE>(c1, v.f1, c2, v.f2, dzc, v.z1, v.z2);
+        const double jf = 1.0 / v.rf;
+        const double fzp = weight(ic, jf) * gzp;
+        const double dx = (weight(1.0 / v.re, ic) * gxp - weight(1.0 / v.rw, ic) * gxm) / dxf;
+        const double dy = (weight(1.0 / v.rn, ic) * gyp - weight(1.0 / v.rs, ic) * gym) / dyf;
+        const double dz = (fzp - fzm) / dzf;
+        s[plane * k + oc] = div * r_adt * rho0 + dx + dy + dz;
+        ic = jf, c1 = v.f1, c2 = v.f2;
+        fzm = fzp;
+        uzm = v.uzc;
+        v = nxt;
+    }
 }
 
 // FAST makeVelocityDivFree + computeOldPressGrad (momentumEqn.f90:999-1127):
 // u_f -= alpha dt [(1/rho0) d psi + ((1/rho)_f - 1/rho0) G_f] on the periodic x/z
-// faces and the interior y faces.
-__global__ void k_project_fast(FieldGeo G, double alpha_dt, double rho0, const double* __restrict__ rho,
-                               const double* __restrict__ psi, const double* __restrict__ psi1,
-                               const double* __restrict__ psi2, StLevels st, double* __restrict__ ux,
-                               double* __restrict__ uy, double* __restrict__ uz)
+// faces and the interior y faces.  The plane after a cell's is its own on the next
+// step of the march.
+template <int MODE>
+__global__ void __launch_bounds__(256)
+    k_project_fast(FieldGeo G, double alpha_dt, double rho0, const double* __restrict__ rho,
+                   const double* __restrict__ psi, OldLevels o, double* __restrict__ ux, double* __restrict__ uy,
+                   double* __restrict__ uz, int kc, int tiles_x, int ntiles)
 {
-    int i, j, k;
-    row_cell(G.nx, G.ny, i, j, k);
+    int i, j, k0, k1;
+    column_cell(kc, tiles_x, ntiles, G.nz, i, j, k0, k1);
     const int nx = G.nx, ny = G.ny, nz = G.nz;
-    if (i >= nx) return;
+    if (i >= nx || j >= ny) return;
     const size_t plane = (size_t)nx * ny;
-    const size_t c = i + (size_t)nx * j + plane * k;
-    const size_t e = (i + 1 < nx ? i + 1 : 0) + (size_t)nx * j + plane * k;
-    const size_t f = i + (size_t)nx * j + plane * (k + 1 < nz ? k + 1 : 0);
-    const double dxc = G.dcn[0][0], dzc = G.dcn[2][0];
+    const size_t oc = i + (size_t)nx * j;
+    const size_t oe = (i + 1 < nx ? i + 1 : 0) + (size_t)nx * j;
+    const size_t on = j + 1 < ny ? oc + nx : oc;
+    const double dxc = G.dcn[0][0], dzc = G.dcn[2][0], dyc = G.dcn[1][j];
     const double inv0 = 1.0 / rho0;
-    const double ic = 1.0 / rho[c];
-    double inv = 0.5 * (1.0 / rho[e] + ic);
-    ux[c] = ux[c] - alpha_dt * (inv0 * ((psi[e] - psi[c]) / dxc) +
-                                (inv - inv0) * with_st(old_grad(psi1, psi2, c, e, dxc), st.x1, st.x2, c));
-    inv = 0.5 * (1.0 / rho[f] + ic);
-    uz[c] = uz[c] - alpha_dt * (inv0 * ((psi[f] - psi[c]) / dzc) +
-                                (inv - inv0) * with_st(old_grad(psi1, psi2, c, f, dzc), st.z1, st.z2, c));
-    if (j + 1 < ny) {
-        const size_t n = c + nx;
+    // the correction of a face between inverses ia, ib and pressures pa, pb, with the old levels' G_f
+    auto face = [&](double ia, double ib, double pa, double pb, double g, double dc) {
+        const double inv = 0.5 * (ib + ia);
+        return alpha_dt * (inv0 * ((pb - pa) / dc) + (inv - inv0) * g);
+    };
+    const size_t p0 = plane * k0 + oc;
+    double ic = 1.0 / rho[p0], pc = psi[p0], c1 = old_psi<MODE>(o, 0, p0), c2 = old_psi<MODE>(o, 1, p0);
+    struct Plane {
+        double rf, re, rn, pf, pe, pn, f1, f2, e1, e2, n1, n2, vx, vy, vz, x1, x2, y1, y2, z1, z2;
+    };
+    auto load = [&](Plane& v, int k) {
+        const size_t pk = plane * k, f = plane * (size_t)(k + 1 < nz ? k + 1 : 0) + oc;
+        const size_t c = pk + oc, e = pk + oe, n = pk + on;
         const size_t yf = i + (size_t)nx * ((j + 1) + (size_t)(ny + 1) * k);
-        const double dyc = G.dcn[1][j];
-        inv = 0.5 * (1.0 / rho[n] + ic);
-        uy[yf] = uy[yf] - alpha_dt * (inv0 * ((psi[n] - psi[c]) / dyc) +
-                                      (inv - inv0) * with_st(old_grad(psi1, psi2, c, n, dyc), st.y1, st.y2, yf));
+        v.rf = rho[f], v.re = rho[e], v.rn = rho[n];
+        v.pf = psi[f], v.pe = psi[e], v.pn = psi[n];
+        v.f1 = old_psi<MODE>(o, 0, f), v.f2 = old_psi<MODE>(o, 1, f);
+        v.e1 = old_psi<MODE>(o, 0, e), v.e2 = old_psi<MODE>(o, 1, e);
+        v.n1 = old_psi<MODE>(o, 0, n), v.n2 = old_psi<MODE>(o, 1, n);
+        v.vx = ux[c], v.vy = uy[yf], v.vz = uz[c];
+        v.x1 = old_st<MODE>(o, 0, 0, c), v.x2 = old_st<MODE>(o, 1, 0, c);
+        v.y1 = old_st<MODE>(o, 0, 1, yf), v.y2 = old_st<MODE>(o, 1, 1, yf);
+        v.z1 = old_st<MODE>(o, 0, 2, c), v.z2 = old_st<MODE>(o, 1, 2, c);
+    };
+    Plane v;
+    load(v, k0);
+    for (int k = k0; k < k1; ++k) {
+        Plane nxt;
+        load(nxt, min(k + 1, k1 - 1));  // (each face belongs to one thread and plane: none is read after its update)
+        __builtin_amdgcn_sched_barrier(0);
+        const size_t c = plane * k + oc;
+        const double jf = 1.0 / v.rf;
+        ux[c] = v.vx - face(ic, 1.0 / v.re, pc, v.pe, old_grad<MODE>(c1, v.e1, c2, v.e2, dxc, v.x1, v.x2), dxc);
+        uz[c] = v.vz - face(ic, jf, pc, v.pf, old_grad<MODE>(c1, v.f1, c2, v.f2, dzc, v.z1, v.z2), dzc);
+        if (j + 1 < ny)
+            uy[i + (size_t)nx * ((j + 1) + (size_t)(ny + 1) * k)] =
+                v.vy - face(ic, 1.0 / v.rn, pc, v.pn, old_grad<MODE>(c1, v.n1, c2, v.n2, dyc, v.y1, v.y2), dyc);
+        ic = jf, pc = v.pf, c1 = v.f1, c2 = v.f2;
+        v = nxt;
     }
 }
 
@@ -473,11 +591,25 @@ int beta_dev(const tbfg_grid_desc* g, double alpha_dt, const double* rho, double
     return TBFG_OK;
 }
 
-// a NULL level, or a NULL component of one, is zero
-static StLevels st_levels(const double* const st1[3], const double* const st2[3])
+// a NULL level, or a NULL component of one, is zero (`any` stands in for its address);
+// mode: the levels that are there
+static OldLevels old_levels(const double* psi1, const double* psi2, const double* const st1[3],
+                            const double* const st2[3], const double* any_cell, const double* any_y, int& mode)
 {
-    return StLevels{st1 ? st1[0] : nullptr, st1 ? st1[1] : nullptr, st1 ? st1[2] : nullptr,
-                    st2 ? st2[0] : nullptr, st2 ? st2[1] : nullptr, st2 ? st2[2] : nullptr};
+    OldLevels o{};
+    const double* p[2] = {psi1, psi2};
+    const double* const* st[2] = {st1, st2};
+    for (int l = 0; l < 2; ++l) {
+        o.p[l] = p[l] ? p[l] : any_cell;
+        if (p[l]) o.has |= 1u << l;
+        for (int c = 0; c < 3; ++c) {
+            const double* a = st[l] ? st[l][c] : nullptr;
+            o.st[l][c] = a ? a : (c == 1 ? any_y : any_cell);
+            if (a) o.has |= 1u << (2 + 3 * l + c);
+        }
+    }
+    mode = (o.has >> 2) ? kAllLevels : (o.has ? kPsiLevels : kNoLevels);
+    return o;
 }
 
 int source_fast_dev(const tbfg_grid_desc* g, double alpha_dt, double rho0, const double* rho, const double* ux,
@@ -498,10 +630,14 @@ int source_fast_dev(const tbfg_grid_desc* g, double alpha_dt, double rho0, const
         set_error("tbfg_source_fast_dev: x and z must be uniform (FAST_MODE)");
         return TBFG_EINVAL;
     }
-    const StLevels st = st_levels(st1, st2);
-    dim3 blk = row_block(G.nx);
-    hipLaunchKernelGGL(k_source_fast, dim3(ceil_div(G.nx, blk.x) * G.ny * G.nz), blk, 0, (hipStream_t)stream, G,
-                       1.0 / alpha_dt, rho0, rho, ux, uy, uz, psi1, psi2, st, s);
+    int mode = 0;
+    const OldLevels o = old_levels(psi1, psi2, st1, st2, rho, uy, mode);
+    const ColGrid cg = column_grid(G.nx, G.ny, G.nz);
+    auto k = mode == kAllLevels   ? k_source_fast<kAllLevels>
+             : mode == kPsiLevels ? k_source_fast<kPsiLevels>
+                                  : k_source_fast<kNoLevels>;
+    hipLaunchKernelGGL(k, dim3(cg.nblocks), cg.blk, 0, (hipStream_t)stream, G, 1.0 / alpha_dt, rho0, rho, ux, uy, uz, o,
+                       s, cg.kc, cg.tiles_x, cg.ntiles);
     TBFG_HIP(hipGetLastError());
     return TBFG_OK;
 }
@@ -524,10 +660,14 @@ int project_fast_dev(const tbfg_grid_desc* g, double alpha_dt, double rho0, cons
         set_error("tbfg_project_fast_dev: x and z must be uniform (FAST_MODE)");
         return TBFG_EINVAL;
     }
-    const StLevels st = st_levels(st1, st2);
-    dim3 blk = row_block(G.nx);
-    hipLaunchKernelGGL(k_project_fast, dim3(ceil_div(G.nx, blk.x) * G.ny * G.nz), blk, 0, (hipStream_t)stream, G,
-                       alpha_dt, rho0, rho, psi, psi1, psi2, st, ux, uy, uz);
+    int mode = 0;
+    const OldLevels o = old_levels(psi1, psi2, st1, st2, rho, uy, mode);
+    const ColGrid cg = column_grid(G.nx, G.ny, G.nz);
+    auto k = mode == kAllLevels   ? k_project_fast<kAllLevels>
+             : mode == kPsiLevels ? k_project_fast<kPsiLevels>
+                                  : k_project_fast<kNoLevels>;
+    hipLaunchKernelGGL(k, dim3(cg.nblocks), cg.blk, 0, (hipStream_t)stream, G, alpha_dt, rho0, rho, psi, o, ux, uy, uz,
+                       cg.kc, cg.tiles_x, cg.ntiles);
     TBFG_HIP(hipGetLastError());
     return TBFG_OK;
 }

@@ -382,3 +382,43 @@ def test_poisson_eqn_fast_steps_rotate_old_levels(torch_gpu):
         for got, want in zip(eq.st_old_[0] + eq.st_old_[1], t1 + t2):
             assert np.array_equal(to_host(got), want), step
     eq.close()
+
+
+@pytest.mark.parametrize("n", [(36, 7, 2), (96, 33, 18), (162, 24, 50), (64, 1, 4)])
+@pytest.mark.parametrize("levels", ["psi1", "psi2+y", "all"])
+def test_fast_source_and_projection_ragged_and_partial_levels(torch_gpu, n, levels):
+    """The column kernels at remainders of their tiles and chunks, and with levels or
+    components that are absent: one old pressure only, psi^(n-1) with the y component of
+    st^n only, everything.  Bounds as in the test at full levels (1e-13 and 1e-12)."""
+    print("case fast columns", n, levels, flush=True)
+    g, go = grids(n, 1)
+    nx, ny, nz = n
+    r = np.random.default_rng(8)
+    ux, uy, uz = F.make_velocity(g, 4)
+    rho = np.asfortranarray(r.uniform(0.05, 1.0, n))
+    psi, psi1, psi2 = (np.asfortranarray(r.standard_normal(n)) for _ in range(3))
+    st1, st2 = random_st(n, walls=False), random_st(n, walls=False)
+    zero = tuple(np.zeros_like(a) for a in st1)
+    if levels == "psi1":
+        psi2, st1, st2 = None, None, None
+    elif levels == "psi2+y":
+        psi1, st2 = None, None
+        st1 = (zero[0], st1[1], zero[2])
+    z3 = np.zeros(n, order="F")
+    full = [z3 if psi1 is None else psi1, z3 if psi2 is None else psi2, zero if st1 is None else st1,
+            zero if st2 is None else st2]
+    adt, rho0 = 1e-3, 0.05
+    s_ref = O.source_fast(go, adt, rho0, rho, ux, uy, uz, *full)
+    dev = lambda a: None if a is None else to_dev(a, torch_gpu)  # noqa: E731
+    d1 = None if st1 is None else tuple(dev(a) if a.any() else None for a in st1)
+    d2 = None if st2 is None else tuple(dev(a) for a in st2)
+    du = [dev(a) for a in (ux, uy, uz)]
+    s = torch_gpu.zeros_like(dev(rho))
+    F.computeSourceFast(g, adt, rho0, dev(rho), *du, s, dev(psi1), dev(psi2), d1, d2)
+    torch_gpu.cuda.synchronize()
+    assert rel(to_host(s), s_ref) < 1e-13
+    ref = O.project_fast(go, adt, rho0, rho, psi, full[0], full[1], ux, uy, uz, full[2], full[3])
+    F.makeVelocityDivFreeFast(g, adt, rho0, dev(rho), dev(psi), *du, dev(psi1), dev(psi2), d1, d2)
+    torch_gpu.cuda.synchronize()
+    for a, b in zip(du, ref):
+        assert rel(to_host(a), b) < 1e-12 or not b.any()
