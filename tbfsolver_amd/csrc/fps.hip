@@ -471,7 +471,7 @@ __global__ void __launch_bounds__(kFftThreads)
 
 // ------------------------------------------- two-level passes, N = N1 x N2
 //
-// Lines of N = N1 * N2 points (N1, N2 in {4, 8, 12, 16}; tl_split) skip the
+// Lines of N = N1 * N2 points (N1, N2 of 4 to 18; tl_split) skip the
 // Stockham passes in LDS.  With n = N2 n1 + n2 and k = k1 + N1 k2,
 //   X[k1 + N1 k2] = sum_n2 W_N2^(n2 k2) [ W_N^(n2 k1) sum_n1 x[N2 n1 + n2] W_N1^(n1 k1) ].
 // Step A: thread n2 of a line holds x[N2 n1 + n2], n1 = 0..N1-1, in registers
@@ -501,49 +501,58 @@ struct TlShape {
     static_assert(LINE >= N + 1, "the x passes' lines of N + 1 fit in a Y line");
 };
 
-// cos and sin of 2 pi e / 48 for e = 0..12 (a quarter turn; the W_R of every
-// supported factor R divides 48)
-constexpr double kW48c[13] = {1.0, 0.991444861373810411144558, 0.965925826289068286749743,
-                              0.923879532511286756128183, 0.866025403784438646763723, 0.793353340291235164579777,
-                              0.707106781186547524400844, 0.608761429008720639416098, 0.5,
-                              0.382683432365089771728460, 0.258819045102520762348899, 0.130526192220051591548406,
-                              0.0};
+// cos and sin of 2 pi e / 144 for e = 0..36 (a quarter turn; the W_R of every
+// supported factor R divides 144)
+constexpr double kW144c[37] = {1.0, 0.999048221581857762403716, 0.996194698091745532295010,
+                               0.991444861373810411144558, 0.984807753012208059366743, 0.976296007119933365970886,
+                               0.965925826289068286749743, 0.953716950748226921143847, 0.939692620785908384054109,
+                               0.923879532511286756128183, 0.906307787036649963242553, 0.887010833178221701054610,
+                               0.866025403784438646763723, 0.843391445812885701272857, 0.819152044288991789684488,
+                               0.793353340291235164579777, 0.766044443118978035202393, 0.737277336810124041384293,
+                               0.707106781186547524400844, 0.675590207615660244348339, 0.642787609686539326322643,
+                               0.608761429008720639416098, 0.573576436351046096108032, 0.537299608346823831840786,
+                               0.5, 0.461748613235033930562931, 0.422618261740699436186978,
+                               0.382683432365089771728460, 0.342020143325668733044100, 0.300705799504273121622547,
+                               0.258819045102520762348899, 0.216439613938102879759554, 0.173648177666930348851717,
+                               0.130526192220051591548406, 0.087155742747658173558064, 0.043619387365335999781753,
+                               0.0};
 
-// a * W_R^e, W_R = exp(SIGN 2 pi i / R); R divides 48; e a constant once the
+// a * W_R^e, W_R = exp(SIGN 2 pi i / R); R divides 144; e a constant once the
 // caller's loops are unrolled, so the table reads and branches fold away
 template <class T, int SIGN, int R>
 __device__ __forceinline__ C2<T> twr_mul(C2<T> a, int e)
 {
-    const int e48 = (e % R) * (48 / R);
-    const int q = e48 / 12, r = e48 % 12;
-    if (e48 == 0) return a;
+    static_assert(144 % R == 0, "W_R is not in the table");
+    const int e144 = (e % R) * (144 / R);
+    const int q = e144 / 36, r = e144 % 36;
+    if (e144 == 0) return a;
     if (r == 0) {  // a quarter, half or three-quarter turn
         if (q == 2) return C2<T>{-a.x, -a.y};
         const bool minus_i = (q == 1) == (SIGN < 0);  // W = -i: forward quarter, backward three-quarter
         return minus_i ? C2<T>{a.y, -a.x} : C2<T>{-a.y, a.x};
     }
-    // cos and sin of the angle q * 90 + r * 7.5 degrees
-    const double c = q == 0 ? kW48c[r] : (q == 1 ? -kW48c[12 - r] : (q == 2 ? -kW48c[r] : kW48c[12 - r]));
-    const double s = q == 0 ? kW48c[12 - r] : (q == 1 ? kW48c[r] : (q == 2 ? -kW48c[12 - r] : -kW48c[r]));
+    // cos and sin of the angle q * 90 + r * 2.5 degrees
+    const double c = q == 0 ? kW144c[r] : (q == 1 ? -kW144c[36 - r] : (q == 2 ? -kW144c[r] : kW144c[36 - r]));
+    const double s = q == 0 ? kW144c[36 - r] : (q == 1 ? kW144c[r] : (q == 2 ? -kW144c[36 - r] : -kW144c[r]));
     const T wr = (T)c, wi = (T)(SIGN * s);
     return C2<T>{a.x * wr - a.y * wi, a.x * wi + a.y * wr};
 }
 
-// R-point DFT in registers, natural order in and out: R = 2, 3, 4 directly,
-// R = 8, 12, 16 as 4 x (R/4) Cooley-Tukey
+// R-point DFT in registers, natural order in and out: R = 2, 3, 4 directly, other
+// multiples of 4 as 4 x (R/4) and of 3 as 3 x (R/3) Cooley-Tukey
 template <class T, int SIGN, int R>
 struct DftReg {
     static __device__ __forceinline__ void run(C2<T>* v)
     {
-        static_assert(R % 4 == 0 && R > 4 && R <= 16, "supported: 2, 3, 4, 8, 12, 16");
-        constexpr int P = 4, Q = R / 4;  // n = Q n1 + n2, k = k1 + P k2
+        static_assert((R % 4 == 0 || R % 3 == 0) && R > 4 && R <= 18, "factors of 2 and 3 up to 18");
+        constexpr int P = R % 4 == 0 ? 4 : 3, Q = R / P;  // n = Q n1 + n2, k = k1 + P k2
         C2<T> a[Q][P];
 #pragma unroll
         for (int n2 = 0; n2 < Q; ++n2) {
             C2<T> t[P];
 #pragma unroll
             for (int n1 = 0; n1 < P; ++n1) t[n1] = v[Q * n1 + n2];
-            dft4<T, SIGN>(t);
+            DftReg<T, SIGN, P>::run(t);
 #pragma unroll
             for (int k1 = 0; k1 < P; ++k1) a[n2][k1] = twr_mul<T, SIGN, R>(t[k1], n2 * k1);
         }
@@ -614,8 +623,10 @@ __device__ __forceinline__ void tl_store_y(C2<T>* Y, const C2<T>* twl, int l, in
     for (int k1 = 1; k1 < N1; ++k1) y[k1 * S::ROW] = tw_apply<T, SIGN>(v[k1], twl[k1 * N2 + n2]);
 }
 
-// K2, two-level: A[kx][j][:] -> B[kx][kz][j]
-template <class T, int N1, int N2>
+// K2, two-level: A[kx][j][:] -> B[kx][kz][j].  PART (here and below): the last
+// workgroup of a row holds fewer lines than the others (lines past the last one are
+// read as the last one and not stored); without it the guards cost fast_64 2 %
+template <class T, int N1, int N2, bool PART>
 __global__ void __launch_bounds__((TlShape<N1, N2>::NT))
     k_zfwd_tl(int ny, const C2<T>* __restrict__ tw, const C2<T>* __restrict__ A, C2<T>* __restrict__ B)
 {
@@ -623,7 +634,7 @@ __global__ void __launch_bounds__((TlShape<N1, N2>::NT))
     constexpr int N = S::N;
     __shared__ C2<T> Y[S::LDS];
     C2<T>* twl = Y + kTlLines * S::LINE;
-    const unsigned id = xcd_block(), gj = (unsigned)(ny / kTlLines);
+    const unsigned id = xcd_block(), gj = (unsigned)((ny + (PART ? kTlLines - 1 : 0)) / kTlLines);
     const int m = (int)(id / gj);
     const int j0 = (int)(id % gj) * kTlLines;
     const int tid = threadIdx.x;
@@ -634,7 +645,8 @@ __global__ void __launch_bounds__((TlShape<N1, N2>::NT))
         const int l = tid / N2, n2 = tid - l * N2;  // lanes along the line
         const bool act = tid < kTlLines * N2;
         // unconditional loads (idle threads read line 0), so no branch waits for them
-        const C2<T>* src = A + ((size_t)m * ny + j0 + (act ? l : 0)) * N + n2;
+        const int jl = j0 + (act ? l : 0);
+        const C2<T>* src = A + ((size_t)m * ny + (PART ? min(jl, ny - 1) : jl)) * N + n2;
         C2<T> v[N1];
 #pragma unroll
         for (int n1 = 0; n1 < N1; ++n1) v[n1] = src[N2 * n1];
@@ -653,14 +665,16 @@ __global__ void __launch_bounds__((TlShape<N1, N2>::NT))
 #pragma unroll
         for (int n2 = 0; n2 < N2; ++n2) v[n2] = y[n2];
         DftReg<T, -1, N2>::run(v);
-        C2<T>* dst = B + ((size_t)m * N + k1) * ny + j0 + l;
+        if (!PART || j0 + l < ny) {
+            C2<T>* dst = B + ((size_t)m * N + k1) * ny + j0 + l;
 #pragma unroll
-        for (int k2 = 0; k2 < N2; ++k2) dst[(size_t)N1 * k2 * ny] = v[k2];
+            for (int k2 = 0; k2 < N2; ++k2) dst[(size_t)N1 * k2 * ny] = v[k2];
+        }
     }
 }
 
 // K4, two-level: B[kx][kz][j] -> A[kx][j][:]
-template <class T, int N1, int N2>
+template <class T, int N1, int N2, bool PART>
 __global__ void __launch_bounds__((TlShape<N1, N2>::NT))
     k_zinv_tl(int ny, const C2<T>* __restrict__ tw, const C2<T>* __restrict__ B, C2<T>* __restrict__ A)
 {
@@ -668,7 +682,7 @@ __global__ void __launch_bounds__((TlShape<N1, N2>::NT))
     constexpr int N = S::N;
     __shared__ C2<T> Y[S::LDS];
     C2<T>* twl = Y + kTlLines * S::LINE;
-    const unsigned id = xcd_block(), gj = (unsigned)(ny / kTlLines);
+    const unsigned id = xcd_block(), gj = (unsigned)((ny + (PART ? kTlLines - 1 : 0)) / kTlLines);
     const int m = (int)(id / gj);
     const int j0 = (int)(id % gj) * kTlLines;
     const int tid = threadIdx.x;
@@ -678,7 +692,7 @@ __global__ void __launch_bounds__((TlShape<N1, N2>::NT))
     {
         const int l = tid & (kTlLines - 1), n2 = tid / kTlLines;  // lanes across lines
         const bool act = tid < kTlLines * N2;
-        const C2<T>* src = B + ((size_t)m * N + (act ? n2 : 0)) * ny + j0 + l;
+        const C2<T>* src = B + ((size_t)m * N + (act ? n2 : 0)) * ny + (PART ? min(j0 + l, ny - 1) : j0 + l);
         C2<T> v[N1];
 #pragma unroll
         for (int n1 = 0; n1 < N1; ++n1) v[n1] = src[(size_t)N2 * n1 * ny];
@@ -697,15 +711,17 @@ __global__ void __launch_bounds__((TlShape<N1, N2>::NT))
 #pragma unroll
         for (int n2 = 0; n2 < N2; ++n2) v[n2] = y[n2];
         DftReg<T, +1, N2>::run(v);
-        C2<T>* dst = A + ((size_t)m * ny + j0 + l) * N + k1;
+        if (!PART || j0 + l < ny) {
+            C2<T>* dst = A + ((size_t)m * ny + j0 + l) * N + k1;
 #pragma unroll
-        for (int k2 = 0; k2 < N2; ++k2) dst[N1 * k2] = v[k2];
+            for (int k2 = 0; k2 < N2; ++k2) dst[N1 * k2] = v[k2];
+        }
     }
 }
 
 // K1, two-level: s(:, j, k0..k0+15) -> A[kx][j][k], kx = 0..N/2 (line l packs
 // the real lines k0+2l and k0+2l+1 into one complex line, as k_xfwd)
-template <class T, class TIN, int N1, int N2>
+template <class T, class TIN, int N1, int N2, bool PART>
 __global__ void __launch_bounds__((TlShape<N1, N2>::NT))
     k_xfwd_tl(int ny, int nz, const C2<T>* __restrict__ tw, const TIN* __restrict__ s, C2<T>* __restrict__ A)
 {
@@ -722,7 +738,8 @@ __global__ void __launch_bounds__((TlShape<N1, N2>::NT))
         const int l = tid / N2, n2 = tid - l * N2;  // lanes along the line
         const bool act = tid < kTlLines * N2;
         const size_t plane = (size_t)N * ny;
-        const TIN* s0 = s + n2 + (size_t)N * (j + (size_t)ny * (k0 + 2 * (act ? l : 0)));
+        const int kl = k0 + 2 * (act ? l : 0);
+        const TIN* s0 = s + n2 + (size_t)N * (j + (size_t)ny * (PART ? min(kl, nz - 2) : kl));
         C2<T> v[N1];
 #pragma unroll
         for (int n1 = 0; n1 < N1; ++n1) v[n1] = C2<T>{(T)s0[N2 * n1], (T)s0[N2 * n1 + plane]};
@@ -762,13 +779,13 @@ __global__ void __launch_bounds__((TlShape<N1, N2>::NT))
             val = C2<T>{(T)0.5 * (Z.x + Zn.x), (T)0.5 * (Z.y - Zn.y)};  // (Z + conj Zn)/2
         else
             val = C2<T>{(T)0.5 * (Z.y + Zn.y), (T)0.5 * (Zn.x - Z.x)};  // (Z - conj Zn)/(2i)
-        A[((size_t)m * ny + j) * nz + k0 + kk] = val;
+        if (!PART || k0 + kk < nz) A[((size_t)m * ny + j) * nz + k0 + kk] = val;
     }
 }
 
 // K5, two-level: A[kx][j][k0..k0+15] -> p(:, j, k) scaled by 1/(nx nz);
 // mode 0: p = val; mode 1: p = p + val - shift[0] (as k_xinv)
-template <class T, int N1, int N2>
+template <class T, int N1, int N2, bool PART>
 __global__ void __launch_bounds__((TlShape<N1, N2>::NT))
     k_xinv_tl(int ny, int nz, const C2<T>* __restrict__ tw, const C2<T>* __restrict__ A, double* __restrict__ p,
               int mode, const double* __restrict__ shift)
@@ -791,7 +808,7 @@ __global__ void __launch_bounds__((TlShape<N1, N2>::NT))
         for (int u = 0; u < kB; ++u) {
             const int t = min(t0 + u * S::NT, nh * L - 1);
             const int m = t / L, l = t - m * L;
-            const size_t o = ((size_t)m * ny + j) * nz + k0 + 2 * l;
+            const size_t o = ((size_t)m * ny + j) * nz + (PART ? min(k0 + 2 * l, nz - 2) : k0 + 2 * l);
             const C2<T> a = A[o], b = A[o + 1];
             x1r[u] = a.x;
             x1i[u] = a.y;
@@ -829,6 +846,7 @@ __global__ void __launch_bounds__((TlShape<N1, N2>::NT))
     __syncthreads();
     if (tid >= kTlLines * N1) return;
     const int l = tid / N1, k1 = tid - l * N1;  // lanes along the line
+    if (PART && k0 + 2 * l >= nz) return;
     const C2<T>* y = Y + l * S::LINE + k1 * S::ROW;
     C2<T> v[N2];
 #pragma unroll
@@ -861,37 +879,43 @@ __global__ void __launch_bounds__((TlShape<N1, N2>::NT))
 
 // (N1, N2) of the two-level passes for a line length, or {0, 0} for the
 // Stockham passes; N1 (the step-A DFT, held in registers per thread) takes the
-// larger factor
+// larger factor.  The lengths of channel axes up to 256 points; f is called with
+// integral_constants, so the lengths' kernels are instantiated where it uses them.
+// Against the Stockham passes at 144 x 99 x 108 (FP64): 17-19 us per pass to 9-10 us,
+// the solve 76.5 to 44.7 us.
 struct TlSplit {
     int n1, n2;
 };
-static TlSplit tl_split(int n)
-{
-    switch (n) {
-        case 32: return {8, 4};
-        case 64: return {8, 8};
-        case 96: return {12, 8};
-        case 128: return {16, 8};
-        case 192: return {16, 12};
-        case 256: return {16, 16};
-        default: return {0, 0};
-    }
-}
-
-// f(integral_constant<N1>, integral_constant<N2>) for a length tl_split accepts
 template <class F>
-static void tl_dispatch(int n, F&& f)
+static bool tl_dispatch(int n, F&& f)
 {
     using std::integral_constant;
+#define TBFG_TL_CASE(N, N1, N2) \
+    case N: f(integral_constant<int, N1>{}, integral_constant<int, N2>{}); return true;
     switch (n) {
-        case 32: f(integral_constant<int, 8>{}, integral_constant<int, 4>{}); break;
-        case 64: f(integral_constant<int, 8>{}, integral_constant<int, 8>{}); break;
-        case 96: f(integral_constant<int, 12>{}, integral_constant<int, 8>{}); break;
-        case 128: f(integral_constant<int, 16>{}, integral_constant<int, 8>{}); break;
-        case 192: f(integral_constant<int, 16>{}, integral_constant<int, 12>{}); break;
-        case 256: f(integral_constant<int, 16>{}, integral_constant<int, 16>{}); break;
-        default: break;
+        TBFG_TL_CASE(32, 8, 4)
+        TBFG_TL_CASE(36, 6, 6)
+        TBFG_TL_CASE(48, 8, 6)
+        TBFG_TL_CASE(54, 9, 6)
+        TBFG_TL_CASE(64, 8, 8)
+        TBFG_TL_CASE(72, 9, 8)
+        TBFG_TL_CASE(96, 12, 8)
+        TBFG_TL_CASE(108, 12, 9)
+        TBFG_TL_CASE(128, 16, 8)
+        TBFG_TL_CASE(144, 12, 12)
+        TBFG_TL_CASE(162, 18, 9)
+        TBFG_TL_CASE(192, 16, 12)
+        TBFG_TL_CASE(216, 18, 12)
+        TBFG_TL_CASE(256, 16, 16)
+        default: return false;
     }
+#undef TBFG_TL_CASE
+}
+static TlSplit tl_split(int n)
+{
+    TlSplit s{0, 0};
+    tl_dispatch(n, [&](auto a, auto b) { s = TlSplit{decltype(a)::value, decltype(b)::value}; });
+    return s;
 }
 
 // ------------------------------------------------------------ K3 y-solve
@@ -1423,13 +1447,12 @@ int fps_create(const tbfg_grid_desc* g, const tbfg_fps_opts* o, tbfg_fps** out)
     h->ot.ap = h->tt.ap;
     h->ot.vol_y = tb + o_vy;
     h->inv_vg = 1.0 / (ly * L.ax[0].df(1) * nx * L.ax[2].df(1) * nz);
-    // two-level passes where the line length splits (tl_split) and the
-    // workgroup's lines tile the other axis (TBFG_FFT_TWO_LEVEL=0 keeps
-    // fft_lines: an A/B switch)
+    // two-level passes where the line length splits (tl_split; a last workgroup may
+    // hold fewer lines).  TBFG_FFT_TWO_LEVEL=0 keeps fft_lines: an A/B switch
     const char* tl_env = std::getenv("TBFG_FFT_TWO_LEVEL");
     const bool tl_on = !(tl_env && tl_env[0] == '0');
-    h->tlx = tl_on && tl_split(nx).n1 > 0 && nz % (2 * kTlLines) == 0;
-    h->tlz = tl_on && tl_split(nz).n1 > 0 && ny % kTlLines == 0;
+    h->tlx = tl_on && tl_split(nx).n1 > 0;
+    h->tlz = tl_on && tl_split(nz).n1 > 0;
     TBFG_TRY(h->precision == TBFG_PREC_MIXED ? set_stockham_lds<float, double>(h.get())
                                              : set_stockham_lds<double, double>(h.get()));
     // twiddles in FP64 and rounded to FP32.  fft_lines: entry Ns-1 + (r-1)*Ns + k
@@ -1516,8 +1539,9 @@ static int spectral_solve(tbfg_fps* h, const TIN* in, double* p, int mode, hipSt
     if (h->tlx)
         tl_dispatch(nx, [&](auto a, auto b) {
             constexpr int N1 = decltype(a)::value, N2 = decltype(b)::value;
-            hipLaunchKernelGGL((k_xfwd_tl<T, TIN, N1, N2>), dim3(nz / (2 * kTlLines), ny), dim3(TlShape<N1, N2>::NT), 0,
-                               s, ny, nz, twx, in, A);
+            auto k = nz % (2 * kTlLines) ? k_xfwd_tl<T, TIN, N1, N2, true> : k_xfwd_tl<T, TIN, N1, N2, false>;
+            hipLaunchKernelGGL(k, dim3(ceil_div(nz, 2 * kTlLines), ny), dim3(TlShape<N1, N2>::NT), 0, s, ny, nz, twx,
+                               in, A);
         });
     else
         hipLaunchKernelGGL((k_xfwd<T, TIN>), dim3(nz / h->KT, ny), dim3(kFftThreads), ldx, s, nx, ny, nz, h->KT, h->px,
@@ -1525,8 +1549,8 @@ static int spectral_solve(tbfg_fps* h, const TIN* in, double* p, int mode, hipSt
     if (h->tlz)
         tl_dispatch(nz, [&](auto a, auto b) {
             constexpr int N1 = decltype(a)::value, N2 = decltype(b)::value;
-            hipLaunchKernelGGL((k_zfwd_tl<T, N1, N2>), dim3((ny / kTlLines) * nh), dim3(TlShape<N1, N2>::NT), 0, s, ny,
-                               twz, A, B);
+            auto k = ny % kTlLines ? k_zfwd_tl<T, N1, N2, true> : k_zfwd_tl<T, N1, N2, false>;
+            hipLaunchKernelGGL(k, dim3(ceil_div(ny, kTlLines) * nh), dim3(TlShape<N1, N2>::NT), 0, s, ny, twz, A, B);
         });
     else
         hipLaunchKernelGGL((k_zfwd<T>), dim3((ny / h->JT) * nh), dim3(kFftThreads), ldz, s, ny, nz, h->JT, h->pz, twz,
@@ -1542,8 +1566,8 @@ static int spectral_solve(tbfg_fps* h, const TIN* in, double* p, int mode, hipSt
     if (h->tlz)
         tl_dispatch(nz, [&](auto a, auto b) {
             constexpr int N1 = decltype(a)::value, N2 = decltype(b)::value;
-            hipLaunchKernelGGL((k_zinv_tl<T, N1, N2>), dim3((ny / kTlLines) * nh), dim3(TlShape<N1, N2>::NT), 0, s, ny,
-                               twz, B, A);
+            auto k = ny % kTlLines ? k_zinv_tl<T, N1, N2, true> : k_zinv_tl<T, N1, N2, false>;
+            hipLaunchKernelGGL(k, dim3(ceil_div(ny, kTlLines) * nh), dim3(TlShape<N1, N2>::NT), 0, s, ny, twz, B, A);
         });
     else
         hipLaunchKernelGGL((k_zinv<T>), dim3((ny / h->JT) * nh), dim3(kFftThreads), ldz, s, ny, nz, h->JT, h->pz, twz,
@@ -1551,8 +1575,9 @@ static int spectral_solve(tbfg_fps* h, const TIN* in, double* p, int mode, hipSt
     if (h->tlx)
         tl_dispatch(nx, [&](auto a, auto b) {
             constexpr int N1 = decltype(a)::value, N2 = decltype(b)::value;
-            hipLaunchKernelGGL((k_xinv_tl<T, N1, N2>), dim3(nz / (2 * kTlLines), ny), dim3(TlShape<N1, N2>::NT), 0, s,
-                               ny, nz, twx, A, p, mode, h->mean.as<double>());
+            auto k = nz % (2 * kTlLines) ? k_xinv_tl<T, N1, N2, true> : k_xinv_tl<T, N1, N2, false>;
+            hipLaunchKernelGGL(k, dim3(ceil_div(nz, 2 * kTlLines), ny), dim3(TlShape<N1, N2>::NT), 0, s, ny, nz, twx, A,
+                               p, mode, h->mean.as<double>());
         });
     else
         hipLaunchKernelGGL((k_xinv<T>), dim3(nz / h->KT, ny), dim3(kFftThreads), ldx, s, nx, ny, nz, h->KT, h->px, twx,

@@ -422,3 +422,28 @@ def test_fast_source_and_projection_ragged_and_partial_levels(torch_gpu, n, leve
     torch_gpu.cuda.synchronize()
     for a, b in zip(du, ref):
         assert rel(to_host(a), b) < 1e-12 or not b.any()
+
+
+@pytest.mark.parametrize("n", [(36, 7, 48), (48, 9, 54), (54, 13, 72), (72, 3, 36), (108, 99, 144), (144, 1, 108),
+                               (162, 5, 216), (216, 33, 162), (64, 20, 18), (18, 17, 64), (32, 8, 6)])
+@pytest.mark.parametrize("precision,bound", [("fp64", 1e-13), ("mixed", 1e-5)])
+def test_two_level_passes_of_factors_of_three_and_remainders(torch_gpu, monkeypatch, n, precision, bound):
+    """Lengths with factors of three, and line counts that leave the last workgroup of a
+    pass partly filled, against the Stockham passes of the same solve (the bounds of the
+    test of the other lengths)."""
+    print("case two-level remainders", n, precision, flush=True)
+    g, _ = grids(n, 1)
+    q = np.random.default_rng(6).standard_normal(n)
+    out = []
+    for tl in ("1", "0"):
+        monkeypatch.setenv("TBFG_FFT_TWO_LEVEL", tl)
+        s = T.FastPoissonSolver(g, precision=precision, refine_sweeps=0)
+        d = to_dev(q, torch_gpu)
+        p = torch_gpu.zeros_like(d)
+        s.solveFPS(p, d)
+        torch_gpu.cuda.synchronize()
+        out.append(to_host(p))
+        s.close()
+    e = rel(out[0], out[1])
+    print("  rel", e, flush=True)
+    assert e < bound
