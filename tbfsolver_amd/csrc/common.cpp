@@ -1,6 +1,10 @@
 // common.cpp -- status handling, grid geometry and per-level device tables.
 #include "common.hpp"
 
+#include <algorithm>
+
+#include "hostio.hpp"
+
 #include <cmath>
 #include <mutex>
 #include <cstdarg>
@@ -166,6 +170,64 @@ int upload(DevBuf& d, const void* src, size_t bytes)
 {
     TBFG_TRY(d.alloc(bytes));
     return copy_sync(d.p, src, bytes, hipMemcpyHostToDevice);
+}
+
+// ------------------------------------------------------------ pinned rings
+
+namespace {
+std::mutex g_ring_mu;
+// the idle ones (never destroyed: at exit the runtime may be gone before statics)
+std::vector<std::unique_ptr<HostRing>>& g_rings = *new std::vector<std::unique_ptr<HostRing>>();
+int g_ring_users = 0;                            // live solver handles
+}  // namespace
+
+HostRing::~HostRing()
+{
+    for (hipEvent_t e : ev)
+        if (e) (void)hipEventDestroy(e);
+    if (pin) (void)hipHostFree(pin);
+}
+
+int host_ring_take(const int32_t* n, std::unique_ptr<HostRing>& out)
+{
+    const size_t need = std::max(HostRing::kSlotBytes / 8, (size_t)n[0] * n[1]);
+    int dev = 0;
+    TBFG_HIP(hipGetDevice(&dev));
+    {
+        std::lock_guard<std::mutex> lk(g_ring_mu);
+        for (auto& r : g_rings)
+            if (r->dev == dev && r->slot >= need) {
+                out = std::move(r);
+                r = std::move(g_rings.back());
+                g_rings.pop_back();
+                return TBFG_OK;
+            }
+    }
+    std::unique_ptr<HostRing> r(new HostRing());
+    r->dev = dev;
+    r->slot = need;
+    TBFG_HIP(hipHostMalloc((void**)&r->pin, HostRing::kSlots * need * 8, hipHostMallocDefault));
+    for (hipEvent_t& e : r->ev) TBFG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    out = std::move(r);
+    return TBFG_OK;
+}
+
+void host_ring_give(std::unique_ptr<HostRing> r)
+{
+    std::lock_guard<std::mutex> lk(g_ring_mu);
+    if (g_ring_users > 0 && g_rings.size() < (size_t)kHostRingsKept) g_rings.push_back(std::move(r));
+}
+
+HostRingUser::HostRingUser()
+{
+    std::lock_guard<std::mutex> lk(g_ring_mu);
+    ++g_ring_users;
+}
+
+HostRingUser::~HostRingUser()
+{
+    std::lock_guard<std::mutex> lk(g_ring_mu);
+    if (--g_ring_users == 0) g_rings.clear();
 }
 
 template <class T>

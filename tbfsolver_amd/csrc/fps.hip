@@ -26,6 +26,7 @@
 #include <vector>
 
 #include "fps.hpp"
+#include "hostio.hpp"
 #include "reduce.hpp"
 
 namespace tbfg {
@@ -1283,6 +1284,8 @@ struct tbfg_fps {
     DevBuf tabf;               // am, ap, dyf (float)
     DevBuf twx, twz, twxf, twzf;
     DevBuf r, partials, counter, mean;
+    DevBuf hs, hp;             // host-array entry point, mixed precision: s and p
+    HostRingUser ring_user;    // keeps the process's pinned staging
     TriTables tt{};
     OpTables ot{};
     double inv_vg = 0;
@@ -1619,6 +1622,23 @@ int fps_apply_operator_dev(tbfg_fps* h, const double* p, double* q, void* stream
 void fps_destroy(tbfg_fps* h) { delete h; }
 
 const tbfg_grid_desc* fps_grid(const tbfg_fps* h) { return &h->g; }
+
+// In FP64 both live in the spectral array B, which holds at least as many bytes and
+// is free before the z pass writes it and after the inverse one has read it.  The
+// refinement sweeps of mixed precision read s and p again.
+int fps_host_fields(tbfg_fps* h, double** s, double** p)
+{
+    const size_t bytes = (size_t)h->nx * h->ny * h->nz * 8;
+    if (h->precision == TBFG_PREC_FP64) {
+        *s = *p = h->B.as<double>();
+        return TBFG_OK;
+    }
+    if (!h->hs.p) TBFG_TRY(h->hs.alloc(bytes));
+    if (!h->hp.p) TBFG_TRY(h->hp.alloc(bytes));
+    *s = h->hs.as<double>();
+    *p = h->hp.as<double>();
+    return TBFG_OK;
+}
 
 int64_t fps_footprint(const tbfg_fps* h) { return h ? h->footprint : 0; }
 

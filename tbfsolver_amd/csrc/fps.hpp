@@ -12,5 +12,7 @@ void fps_destroy(tbfg_fps* h);
 const tbfg_grid_desc* fps_grid(const tbfg_fps* h);
 // the constant-coefficient operator the FFT solver inverts (q = L p), FP64
 int fps_apply_operator_dev(tbfg_fps* h, const double* p, double* q, void* stream);
+// device fields of the host-array entry point
+int fps_host_fields(tbfg_fps* h, double** s, double** p);
 int64_t fps_footprint(const tbfg_fps* h);
 }  // namespace tbfg

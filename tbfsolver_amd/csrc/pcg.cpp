@@ -50,7 +50,6 @@ tbfg_pcg::~tbfg_pcg()
     if (hring) (void)hipHostFree(hring);
     for (hipEvent_t e : hev)
         if (e) (void)hipEventDestroy(e);
-    if (hstage) (void)hipHostFree(hstage);
     if (hin) (void)hipHostFree(hin);
     if (hmg) (void)hipHostFree(hmg);
     if (fps) tbfg::fps_destroy(fps);

@@ -4,6 +4,7 @@
 #include <memory>
 
 #include "fps.hpp"
+#include "hostio.hpp"
 #include "mg_launch.hpp"
 
 struct tbfg_pcg {
@@ -48,7 +49,7 @@ struct tbfg_pcg {
     tbfg::PcgState* hst = nullptr;      // pinned mirror of the device state (final, after a solve)
     tbfg::PcgState* hring = nullptr;    // pinned copies of the state after consecutive iterations
     hipEvent_t hev[2] = {nullptr, nullptr};
-    double* hstage = nullptr;           // pinned staging (3 * n0 doubles)
+    tbfg::HostRingUser ring_user;       // keeps the process's pinned staging
     int64_t footprint = 0;
 
     // kernel timing (tbfg_pcg_profile_begin/end)

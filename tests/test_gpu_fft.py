@@ -447,3 +447,26 @@ def test_two_level_passes_of_factors_of_three_and_remainders(torch_gpu, monkeypa
     e = rel(out[0], out[1])
     print("  rel", e, flush=True)
     assert e < bound
+
+
+@pytest.mark.parametrize("n,precision,halo", [((96, 64, 144), "fp64", 2), ((36, 5, 6), "mixed", 1), ((64, 48, 36), "fp64", 0)])
+def test_host_arrays_in_chunks_equal_device_solve(torch_gpu, n, precision, halo):
+    """Host arrays that pass through several staging chunks (85 planes each at 96x64) and
+    halos of other widths: the interior equals the device solve bit for bit; the halo is
+    the wall row in y (first layer), then the periodic image in x and z; layers of y
+    beyond the first are left as they were."""
+    print("case host chunks", n, precision, halo, flush=True)
+    g, _ = grids(n, 1)
+    s = np.random.default_rng(3).standard_normal(n)
+    fs = T.FastPoissonSolver(g, precision=precision)
+    pd = torch_gpu.zeros_like(to_dev(s, torch_gpu))
+    fs.solveFPS(pd, to_dev(s, torch_gpu))
+    torch_gpu.cuda.synchronize()
+    p = np.full([v + 2 * halo for v in n], 7.0, order="F")
+    for _ in range(2):
+        fs.solveFPS(p, np.asfortranarray(np.pad(s, halo)))
+    ref = np.pad(to_host(pd), ((0, 0), (min(halo, 1),) * 2, (0, 0)), mode="edge")
+    ref = np.pad(ref, ((0, 0), (halo - min(halo, 1),) * 2, (0, 0)), constant_values=7.0)
+    ref = np.pad(np.pad(ref, ((halo, halo), (0, 0), (0, 0)), mode="wrap"), ((0, 0), (0, 0), (halo, halo)), mode="wrap")
+    assert np.array_equal(p, ref)
+    fs.close()
