@@ -694,19 +694,17 @@ __device__ __forceinline__ void rbgs_cell(const LV& L, PB __restrict__ beta, PQ 
     const int i = ((COLOUR + j + k + 1) & 1) + 2 * h;
     typename IdxOf<LV>::type c, e, w, n, s, f, b;
     neighbours(i, j, k, nx, ny, nz, c, e, w, n, s, f, b);
-    Coef<T> a = coefs<T>(L, beta, i, j, k, c, e, w, n, s, f, b);
-    const T den = a.aR + a.aL + a.aT + a.aB + a.aF + a.aK;
-    const T qc = (T)q[c];
-    T num;
-    if (FIRST && COLOUR == RED) {
-        num = -qc;
-    } else {
+    const Around<T> bs = {(T)beta[e], (T)beta[w], (T)beta[n], (T)beta[s], (T)beta[f], (T)beta[b]};
+    const T half = (T)0.5;
+    constexpr bool ZERO = FIRST && COLOUR == RED;
+    Around<T> ps = {};
+    if (!ZERO) {
         const T self = FIRST ? (T)0 : p[c];
-        const T pn = (n == c) ? self : p[n];
-        const T ps = (s == c) ? self : p[s];
-        num = -qc + (a.aR * p[e] + a.aL * p[w]) + (a.aT * pn + a.aB * ps) + (a.aF * p[f] + a.aK * p[b]);
+        ps = {p[e], p[w], (n == c) ? self : p[n], (s == c) ? self : p[s], p[f], p[b]};
     }
-    p[c] = smooth_div(num, den);
+    p[c] = smooth_cell<T, ZERO>((T)q[c], (T)beta[c], bs, half * L.a[0].ip[i], half * L.a[0].im[i],
+                                               half * L.a[1].ip[j], half * L.a[1].im[j], half * L.a[2].ip[k],
+                                               half * L.a[2].im[k], ps);
 }
 
 template <class T, class TQ, int COLOUR, bool FIRST>

@@ -62,20 +62,32 @@ struct SweepDots {
 struct KernelEvents {
     hipEvent_t start, stop;
 };
+// (TB: the storage type of beta, T or, on the finest level, bf16s)
+// a march along z; sweep_supported: a tile shape of k_sweep divides the level
 template <class T>
 bool sweep_supported(const LevelDev<T>& L);
-// one full red/black sweep of a small level, out of place, from bricks staged
-// in LDS (levels whose dimensions the brick divides)
+// sweep_named: TBFG_SWEEP_SHAPE or the tuning table asks for one (plain: for the sweep
+// from a non-zero start without the dot products)
 template <class T>
-bool brick_supported(const LevelDev<T>& L);
-template <class T, class TQ>
-int launch_brick_sweep(const LevelDev<T>& L, const T* beta, const TQ* q, const T* pin, T* pout, bool first,
-                       const int* done, void* stream);
-// (TB: the storage type of beta, T or, on the finest level, bf16s)
+bool sweep_named(const LevelDev<T>& L, bool plain);
 template <class T, class TQ, class TB = T>
 int launch_sweep(const LevelDev<T>& L, const TB* beta, const TQ* q, const T* pin, T* pout, bool first,
                  const int* done, void* stream, const SweepDots* dots = nullptr, unsigned* nblocks_out = nullptr,
                  const KernelEvents* kev = nullptr);
+// the march with whole rows in a wavefront (nx a multiple of 4, 16..256)
+template <class T>
+bool row_supported(const LevelDev<T>& L);
+template <class T, class TQ, class TB = T>
+int launch_row_sweep(const LevelDev<T>& L, const TB* beta, const TQ* q, const T* pin, T* pout, bool first,
+                     const int* done, void* stream, const SweepDots* dots = nullptr, unsigned* nblocks_out = nullptr,
+                     const KernelEvents* kev = nullptr);
+// a thread per pair of cells (any even nx, nz)
+template <class T>
+bool point_supported(const LevelDev<T>& L);
+template <class T, class TQ>
+int launch_point_sweep(const LevelDev<T>& L, const T* beta, const TQ* q, const T* pin, T* pout, bool first,
+                       const int* done, void* stream, const SweepDots* dots = nullptr,
+                       unsigned* nblocks_out = nullptr);
 // solveMG's stop test after V-cycle cyc: sets PcgState::mg_stop
 // (T0: the storage type of the finest level's beta and q)
 template <class T, class T0>

@@ -385,16 +385,24 @@ int pcg_create(const tbfg_grid_desc* g, const tbfg_pcg_params* prm_in, tbfg_pcg*
         TBFG_TRY(h->p[l].alloc(n * es));
         if (l > 0) TBFG_TRY(h->q[l].alloc(n * es));
         if (l < (h->kin >= 0 ? h->kin : t0)) {
-            h->fused[l] = h->mixed ? sweep_supported<float>(h->tabf[l]->view) : sweep_supported<double>(h->tabd[l]->view);
-            // below ~1M cells a plane march of a few steps per workgroup is
-            // latency bound and the two half-sweep launches are quicker
-            size_t min_cells = (size_t)1 << 20;
-            if (const char* e = std::getenv("TBFG_SWEEP_MIN_CELLS")) min_cells = (size_t)std::atoll(e);
-            if (n < min_cells || std::getenv("TBFG_HALF_SWEEPS")) h->fused[l] = 0;
-            // below that, one launch per sweep from bricks staged in LDS
-            if (!h->fused[l] && !std::getenv("TBFG_HALF_SWEEPS") && !std::getenv("TBFG_NO_BRICKS") &&
-                (h->mixed ? brick_supported<float>(h->tabf[l]->view) : brick_supported<double>(h->tabd[l]->view)))
-                h->fused[l] = 2;
+            auto can = [&](auto f, auto d) { return h->mixed ? f(h->tabf[l]->view) : d(h->tabd[l]->view); };
+            const bool half = std::getenv("TBFG_HALF_SWEEPS") != nullptr;  // A/B switch: half-sweep launches
+            // one launch per sweep: the marches where their chunks of planes fill the chip
+            // (A/B switch TBFG_SWEEP_MIN_CELLS: from that many cells), a thread per pair
+            // below.  k_sweep's tiles and with them the bf16 storage from 1 M cells; the
+            // rows of k_row_sweep overtake the pairs at about 0.3 M (FP32: 196 K cells
+            // 5.9 us in pairs, 7.3 in rows; 1.6 M 23 and 8.6.  FP64: 262 K 7.6 and 7.4,
+            // 590 K 14.5 and 10)
+            size_t march = (size_t)1 << 20, rows = h->mixed ? (size_t)3 << 17 : (size_t)1 << 18;
+            if (const char* e = std::getenv("TBFG_SWEEP_MIN_CELLS")) march = rows = (size_t)std::atoll(e);
+            if (!half) {
+                if (n >= march && can(sweep_supported<float>, sweep_supported<double>))
+                    h->fused[l] = 1;
+                else if (n >= rows && can(row_supported<float>, row_supported<double>))
+                    h->fused[l] = 3;
+                else if (can(point_supported<float>, point_supported<double>))
+                    h->fused[l] = 2;
+            }
             if (h->fused[l]) TBFG_TRY(h->palt[l].alloc(n * es));
         }
         // bf16 storage of the finest level's q and beta: where the plane march smooths it
@@ -543,15 +551,22 @@ static int smooth(tbfg_pcg* h, int l, const T0* b, const T0* q, T*& p, T*& alt, 
             std::swap(p, alt);
         } else if (h->fused[l] == 2) {
             ProfScope ps(h, l == 0 ? 0 : -1, stream);
-            TBFG_TRY(launch_brick_sweep<T, T>(L, b, q, p, alt, f0, done, stream));
+            const bool last = s == nsweeps - 1;
+            TBFG_TRY(launch_point_sweep<T, T>(L, b, q, p, alt, f0, done, stream, last ? last_dots : nullptr,
+                                              last ? nb_out : nullptr));
             std::swap(p, alt);
         } else if (h->fused[l]) {
             const bool last = s == nsweeps - 1;
             // the timed finest-level sweep: from a non-zero start, without the dot products
             const bool plain = l == 0 && !f0 && !(last && last_dots);
             ProfScope ps(h, plain ? 0 : -1, stream, true);
-            TBFG_TRY(launch_sweep<T, T>(L, b, q, p, alt, f0, done, stream, last ? last_dots : nullptr,
-                                        last ? nb_out : nullptr, ps.events()));
+            // by rows, except where a tile shape is asked for, and under bf16 storage: the
+            // residual cut to 8 bits there turns a last bit of FP32 into a few 1e-9 of the
+            // solution (1 % of its error), so those levels keep k_sweep's order of sums
+            const bool tiles = h->fused[l] == 1 && (h->b16 || !row_supported<T>(L) || sweep_named<T>(L, !f0 && !(last && last_dots)));
+            auto go = tiles ? launch_sweep<T, T, T> : launch_row_sweep<T, T, T>;
+            TBFG_TRY(go(L, b, q, p, alt, f0, done, stream, last ? last_dots : nullptr, last ? nb_out : nullptr,
+                        ps.events()));
             std::swap(p, alt);
         } else {
             ProfScope ps(h, l == 0 ? 0 : -1, stream);
@@ -667,7 +682,9 @@ static int vcycle(tbfg_pcg* h, const T0* r0, T** z, const T0* beta0, const int* 
     // products are not folded into a sweep
     const bool tol_mode = h->prm.mg_tol > 0.0;
     const int ncycles = tol_mode ? h->prm.mg_max_iter : h->prm.mg_cycles;
-    const bool want_dots = !tol_mode && dots_init >= 0 && h->fused[0] == 1 && h->prm.n_post > 0 && h->t0 > 0;
+    // (a thread per pair leaves a partial per 512 cells: the separate pass from 1 M cells)
+    const bool want_dots = !tol_mode && dots_init >= 0 && h->prm.n_post > 0 && h->t0 > 0 &&
+                           (h->fused[0] == 1 || h->fused[0] == 3 || (h->fused[0] == 2 && h->n0 <= ((size_t)1 << 20)));
     SweepDots sd;
     if (want_dots) {
         sd.r = h->r.as<double>();

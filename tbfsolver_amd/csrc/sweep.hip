@@ -1,21 +1,24 @@
 // sweep.hip -- one full red/black Gauss-Seidel sweep per launch (rbgs.f90:205-259:
 // the red half-sweep, then the black one), out of place: pin holds the level's
 // values before the sweep and is only read, pout receives the values after it.
+// Three kernels, chosen per level (pcg_create, smooth):
+//   k_row_sweep    marches along z with whole rows of up to 256 cells in a wavefront
+//   k_sweep        marches along z with tiles staged in LDS: rows longer than that, bf16
+//                  storage, and the tile shapes a tuning table names
+//   k_point_sweep  no march, a thread per pair of cells: small levels and odd row lengths
+// The values a workgroup needs from beyond its cells are recomputed from pin, so
+// no workgroup waits on another and the result equals the two half-sweep launches up to
+// the rounding of fused multiply-adds.
 //
-// A workgroup owns a TX x TY tile of cells in the (x, y) plane and a chunk of
+// k_sweep: a workgroup owns a TX x TY tile of cells in the (x, y) plane and a chunk of
 // planes in z, and marches through the chunk one plane at a time.  At plane
 // step k it computes the red cells of plane k over the tile plus a one-cell
 // ring and then the black cells of plane k-1 over the tile, which need the new
-// red values of planes k-2, k-1, k.  The ring and the two extra red planes at
-// the chunk ends are recomputed by every workgroup that needs them, from the
-// old values in pin, so no workgroup waits on another and the result equals
-// the two half-sweep launches exactly.
-//
-// Every input plane is staged once in LDS (p and beta with a two-cell ring, q
-// with a one-cell ring), loaded into registers one step ahead so that the HBM
-// latency of plane k+2 overlaps the arithmetic of plane k.  HBM traffic per
-// cell: p in, beta, q, p out -- once per sweep, where two half-sweep launches
-// stream every array twice.
+// red values of planes k-2, k-1, k.  Every input plane is staged once in LDS (p and
+// beta with a two-cell ring, q with a one-cell ring), loaded into registers one step
+// ahead so that the HBM latency of plane k+2 overlaps the arithmetic of plane k.  HBM
+// traffic per cell: p in, beta, q, p out -- once per sweep, where two half-sweep
+// launches stream every array twice.
 #include "mg_kernels.hpp"
 #include "mg_launch.hpp"
 #include "reduce.hpp"
@@ -24,9 +27,11 @@
 
 #include <hip/hip_ext.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cstdio>
 #include <cstdlib>
+#include <type_traits>
 
 namespace tbfg {
 
@@ -444,188 +449,474 @@ __global__ void __launch_bounds__(NT)
     if (DOTS) block_partial<5>(acc, dots.red);
 }
 
-// One full red/black sweep of a small level per launch (rbgs.f90:205-259),
-// out of place like k_sweep.  A workgroup stages a BX x BY x BZ brick of p and
-// beta with a two-cell ring and of q with a one-cell ring in LDS (a level this
-// small stays in L2, so the ring's re-reads cost little), computes the red
-// cells of the brick and its one-cell ring, then the black cells of the brick,
-// and writes the brick.  Ring cells are recomputed from pin by every workgroup
-// that needs them, so the launch equals the red and the black half-sweep
-// launches, with the same arithmetic as rbgs_cell.  Where a plane march would
-// take a few steps per workgroup (latency bound), all of a brick's planes load
-// at once.
-constexpr int kBrickThreads = 256;
-
-template <class T, class TQ, int BX, int BY, int BZ, bool FIRST>
-__global__ void __launch_bounds__(kBrickThreads)
-    k_brick_sweep(LevelDev<T> L, const T* __restrict__ beta, const TQ* __restrict__ q, const T* __restrict__ pin,
-                  T* __restrict__ pout, const int* done)
+// One full red/black sweep of a level per launch (rbgs.f90:205-259) without any
+// exchange between threads, out of place like k_sweep: a thread owns the red and the
+// black cell of an x pair and computes from pin, beside its own red cell, the five
+// other red cells its black cell reads -- seven cell updates instead of two, from 25
+// values of beta, 19 of p and 7 of q that all load at once (the neighbours' loads hit
+// in L1).  On small levels the time is the chain of one round of loads, two dependent
+// updates and the launch itself; staging a brick in LDS added its index arithmetic, two
+// barriers and the serial rounds of its cells.  Any even nx, nz; any ny.  Per launch,
+// bricks -> this: FP32 196 K cells 6.7 -> 5.9 us, 25 K 6.3 -> 4.6; FP64 262 K 8.4 -> 7.5,
+// 74 K 6.6 -> 5.5; two half-sweeps at 20 K (72x40x56's level 1) 8.1 -> 4.6.
+// DOTS: the sums of k_pcg_dots as in k_sweep, one partial per workgroup.
+template <class T, class TQ, bool FIRST, bool DOTS>
+__global__ void __launch_bounds__(256)
+    k_point_sweep(LevelDev<T> L, const T* __restrict__ beta, const TQ* __restrict__ q, const T* __restrict__ pin,
+                  T* __restrict__ pout, uint32_t m_hx, uint32_t m_ny, int npairs, const int* done, SweepDots dots)
 {
-    constexpr int NT = kBrickThreads;
-    constexpr int PX = BX + 4, PY = BY + 4, PZ = BZ + 4, PS = PX * PY * PZ;
-    constexpr int QX = BX + 2, QY = BY + 2, QZ = BZ + 2, QS = QX * QY * QZ;
-    static_assert(BX % 2 == 0, "cell pairs along x");
-    __shared__ T sP[FIRST ? 1 : PS];
-    __shared__ T sB[PS];
-    __shared__ T sQ[QS];
-    __shared__ T sR[QS];  // new red values, brick + one-cell ring
-    __shared__ T sT[2 * (QX + QY + QZ)];  // face factors ip, im of the ring-1 rows/columns/planes
-
     if (done && *done) return;
+    unsigned id = blockIdx.x;  // consecutive blocks on one XCD
+    if ((gridDim.x & 7u) == 0) id = (id & 7u) * (gridDim.x >> 3) + (id >> 3);
+    const int tp = (int)(id * 256u + threadIdx.x);
+    const bool own = tp < npairs;  // (the last block's idle threads follow the last pair)
+    const int t = own ? tp : npairs - 1;
     const int nx = L.nx, ny = L.ny, nz = L.nz;
-    const int nbx = nx / BX, nby = ny / BY;
-    const int bid = (int)blockIdx.x;
-    const int x0 = (bid % nbx) * BX, y0 = ((bid / nbx) % nby) * BY, z0 = (bid / (nbx * nby)) * BZ;
-    const size_t plane = (size_t)nx * ny;
+    const int hx = nx >> 1;
+    const int row = hx == 1 ? t : (int)__umulhi((uint32_t)t, m_hx), h = t - row * hx;
+    const int k = ny == 1 ? row : (int)__umulhi((uint32_t)row, m_ny), j = row - k * ny;
+    const int par = (j + k) & 1;  // offset of the black cell in the pair ((i + j + k) even)
+    const int xb = 2 * h + par;
+    const int e1 = xb + 1 < nx ? xb + 1 : 0, w1 = xb > 0 ? xb - 1 : nx - 1;
+    const int e2 = e1 + 1 < nx ? e1 + 1 : 0, w2 = w1 > 0 ? w1 - 1 : nx - 1;
+    const int jn = min(j + 1, ny - 1), js = max(j - 1, 0), jn2 = min(j + 2, ny - 1), js2 = max(j - 2, 0);
+    const int kf = k + 1 < nz ? k + 1 : 0, kb = k > 0 ? k - 1 : nz - 1;
+    const int kf2 = kf + 1 < nz ? kf + 1 : 0, kb2 = kb > 0 ? kb - 1 : nz - 1;
+    auto rw = [&](int jj, int kk) { return nx * (jj + ny * kk); };
+    const int rc = rw(j, k), rn = rw(jn, k), rs = rw(js, k), rf = rw(j, kf), rb = rw(j, kb);
+    const int o_n2 = rw(jn2, k) + xb, o_s2 = rw(js2, k) + xb, o_f2 = rw(j, kf2) + xb, o_b2 = rw(j, kb2) + xb;
+    const int o_nf = rw(jn, kf) + xb, o_nb = rw(jn, kb) + xb, o_sf = rw(js, kf) + xb, o_sb = rw(js, kb) + xb;
 
-    // every load of the brick issued before the first LDS store (one wait)
-    constexpr int NPL = (PS + NT - 1) / NT, NQL = (QS + NT - 1) / NT;
-    T rb[NPL], rp[NPL], rq[NQL];
-#pragma unroll
-    for (int m = 0; m < NPL; ++m) {
-        const int t = min((int)threadIdx.x + m * NT, PS - 1);
-        const int xx = t % PX, r = t / PX, yy = r % PY, zz = r / PY;
-        const size_t g = plane * wrapi(z0 + zz - 2, nz) + (size_t)nx * clampi(y0 + yy - 2, ny) + wrapi(x0 + xx - 2, nx);
-        rb[m] = beta[g];
-        if (!FIRST) rp[m] = pin[g];
+    // beta: row of the cell, the four rows beside it, the diagonals and second neighbours
+    const T bw2 = beta[rc + w2], bw = beta[rc + w1], bc = beta[rc + xb], be = beta[rc + e1], be2 = beta[rc + e2];
+    const T bnw = beta[rn + w1], bn = beta[rn + xb], bne = beta[rn + e1];
+    const T bsw = beta[rs + w1], bs = beta[rs + xb], bse = beta[rs + e1];
+    const T bfw = beta[rf + w1], bf = beta[rf + xb], bfe = beta[rf + e1];
+    const T bbw = beta[rb + w1], bb = beta[rb + xb], bbe = beta[rb + e1];
+    const T bn2 = beta[o_n2], bs2 = beta[o_s2], bf2 = beta[o_f2], bb2 = beta[o_b2];
+    const T bnf = beta[o_nf], bnb = beta[o_nb], bsf = beta[o_sf], bsb = beta[o_sb];
+    double2 dr = {0.0, 0.0}, dq = {0.0, 0.0};
+    if (DOTS) {
+        dr = *reinterpret_cast<const double2*>(dots.r + rc + 2 * h);
+        if (!dots.init) dq = *reinterpret_cast<const double2*>(dots.qv + rc + 2 * h);
     }
-#pragma unroll
-    for (int m = 0; m < NQL; ++m) {
-        const int t = min((int)threadIdx.x + m * NT, QS - 1);
-        const int xx = t % QX, r = t / QX, yy = r % QY, zz = r / QY;
-        rq[m] = (T)q[plane * wrapi(z0 + zz - 1, nz) + (size_t)nx * clampi(y0 + yy - 1, ny) + wrapi(x0 + xx - 1, nx)];
-    }
-#pragma unroll
-    for (int m = 0; m < NPL; ++m) {
-        const int t = min((int)threadIdx.x + m * NT, PS - 1);
-        sB[t] = rb[m];
-        if (!FIRST) sP[t] = rp[m];
-    }
-#pragma unroll
-    for (int m = 0; m < NQL; ++m) sQ[min((int)threadIdx.x + m * NT, QS - 1)] = rq[m];
-    for (int t = threadIdx.x; t < QX + QY + QZ; t += NT) {
-        const T *fp, *fm;
-        int g;
-        if (t < QX) {
-            fp = L.a[0].ip;
-            fm = L.a[0].im;
-            g = wrapi(x0 + t - 1, nx);
-        } else if (t < QX + QY) {
-            fp = L.a[1].ip;
-            fm = L.a[1].im;
-            g = clampi(y0 + t - QX - 1, ny);
-        } else {
-            fp = L.a[2].ip;
-            fm = L.a[2].im;
-            g = wrapi(z0 + t - QX - QY - 1, nz);
-        }
-        sT[t] = fp[g];
-        sT[QX + QY + QZ + t] = fm[g];
-    }
-    __syncthreads();
-    constexpr int TM = QX + QY + QZ;  // offset of the im factors
+    const T qc = (T)q[rc + xb], qe = (T)q[rc + e1], qw = (T)q[rc + w1], qn = (T)q[rn + xb], qs = (T)q[rs + xb],
+            qf = (T)q[rf + xb], qb = (T)q[rb + xb];
+    auto ld = [&](int o) { return FIRST ? (T)0 : pin[o]; };
+    const T pc = ld(rc + xb), pw2 = ld(rc + w2), pe2 = ld(rc + e2);
+    const T pnw = ld(rn + w1), pne = ld(rn + e1), psw = ld(rs + w1), pse = ld(rs + e1);
+    const T pfw = ld(rf + w1), pfe = ld(rf + e1), pbw = ld(rb + w1), pbe = ld(rb + e1);
+    const T pn2 = ld(o_n2), ps2 = ld(o_s2), pf2 = ld(o_f2), pb2 = ld(o_b2);
+    const T pnf = ld(o_nf), pnb = ld(o_nb), psf = ld(o_sf), psb = ld(o_sb);
+    // face factors times 1/2 (exact) at the cell and the two neighbours of each axis
     const T half = (T)0.5;
+    const T xp = half * L.a[0].ip[xb], xm = half * L.a[0].im[xb];
+    const T xpe = half * L.a[0].ip[e1], xme = half * L.a[0].im[e1], xpw = half * L.a[0].ip[w1], xmw = half * L.a[0].im[w1];
+    const T yp = half * L.a[1].ip[j], ym = half * L.a[1].im[j];
+    const T ypn = half * L.a[1].ip[jn], ymn = half * L.a[1].im[jn], yps = half * L.a[1].ip[js], yms = half * L.a[1].im[js];
+    const T zp = half * L.a[2].ip[k], zm = half * L.a[2].im[k];
+    const T zpf = half * L.a[2].ip[kf], zmf = half * L.a[2].im[kf], zpb = half * L.a[2].ip[kb], zmb = half * L.a[2].im[kb];
 
-    // red cells (gx + gy + gz odd) of the brick and its ring; ghost rows
-    // beyond the walls are not cells (their values are never read)
-    constexpr int NRED = (QX / 2) * QY * QZ;
-    for (int t = threadIdx.x; t < NRED; t += NT) {
-        const int hh = t % (QX / 2), r = t / (QX / 2), yy = r % QY, zz = r / QY;
-        const int gy = y0 + yy - 1, gz = z0 + zz - 1;
-        if (gy < 0 || gy >= ny) continue;
-        const int xx = 2 * hh + ((x0 + gy + gz) & 1);  // ring-1 coordinates (nx, nz even)
-        const int ip = ((zz + 1) * PY + yy + 1) * PX + xx + 1;
-        const T bc = sB[ip];
-        const T aR = half * (sB[ip + 1] + bc) * sT[xx];
-        const T aL = half * (bc + sB[ip - 1]) * sT[TM + xx];
-        const T aT = half * (sB[ip + PX] + bc) * sT[QX + yy];
-        const T aB = half * (bc + sB[ip - PX]) * sT[TM + QX + yy];
-        const T aF = half * (sB[ip + PX * PY] + bc) * sT[QX + QY + zz];
-        const T aK = half * (bc + sB[ip - PX * PY]) * sT[TM + QX + QY + zz];
-        const T den = aR + aL + aT + aB + aF + aK;
-        const T qc = sQ[(zz * QY + yy) * QX + xx];
-        T num;
-        if (FIRST) {
-            num = -qc;
-        } else {
-            // rows beyond the walls hold the wall row: the ghost is the cell itself
-            num = -qc + (aR * sP[ip + 1] + aL * sP[ip - 1]) + (aT * sP[ip + PX] + aB * sP[ip - PX]) +
-                  (aF * sP[ip + PX * PY] + aK * sP[ip - PX * PY]);
+    const std::true_type red;
+    // one update: centre beta, the six neighbours' beta and p
+    auto update = [&](T qq, T c, T bE, T bW, T bN, T bS, T bF, T bB, T fxp, T fxm, T fyp, T fym, T fzp, T fzm, T pE, T pW,
+                      T pN, T pS, T pF, T pB, auto red) {
+        return smooth_cell<T, FIRST && decltype(red)::value>(
+            qq, c, {bE, bW, bN, bS, bF, bB}, fxp, fxm, fyp, fym, fzp, fzm, {pE, pW, pN, pS, pF, pB});
+    };
+    const T re = update(qe, be, be2, bc, bne, bse, bfe, bbe, xpe, xme, yp, ym, zp, zm, pe2, pc, pne, pse, pfe, pbe, red);
+    const T rwv = update(qw, bw, bc, bw2, bnw, bsw, bfw, bbw, xpw, xmw, yp, ym, zp, zm, pc, pw2, pnw, psw, pfw, pbw, red);
+    const T rnv = update(qn, bn, bne, bnw, bn2, bc, bnf, bnb, xp, xm, ypn, ymn, zp, zm, pne, pnw, pn2, pc, pnf, pnb, red);
+    const T rsv = update(qs, bs, bse, bsw, bc, bs2, bsf, bsb, xp, xm, yps, yms, zp, zm, pse, psw, pc, ps2, psf, psb, red);
+    const T rfv = update(qf, bf, bfe, bfw, bnf, bsf, bf2, bc, xp, xm, yp, ym, zpf, zmf, pfe, pfw, pnf, psf, pf2, pc, red);
+    const T rbv = update(qb, bb, bbe, bbw, bnb, bsb, bc, bb2, xp, xm, yp, ym, zpb, zmb, pbe, pbw, pnb, psb, pc, pb2, red);
+    // the black cell: a wall's ghost is its own value before the sweep
+    const T vb = update(qc, bc, be, bw, bn, bs, bf, bb, xp, xm, yp, ym, zp, zm, re, rwv, j + 1 < ny ? rnv : pc,
+                        j > 0 ? rsv : pc, rfv, rbv, std::false_type());
+    typename Vec2<T>::type v;
+    v.x = par ? rwv : vb;
+    v.y = par ? vb : re;
+    if (own) *reinterpret_cast<typename Vec2<T>::type*>(pout + rc + 2 * h) = v;
+    if (DOTS) {  // the order of k_pcg_dots, cell by cell
+        double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+        if (own) {
+            const double z0 = (double)v.x, z1 = (double)v.y;
+            acc[0] = dr.x * z0 + dr.y * z1;
+            acc[2] = z0 + z1;
+            acc[3] = dr.x + dr.y;
+            if (!dots.init) {
+                acc[1] = dq.x * z0 + dq.y * z1;
+                acc[4] = dq.x + dq.y;
+            }
         }
-        sR[(zz * QY + yy) * QX + xx] = smooth_div(num, den);
+        block_partial<5>(acc, dots.red);
     }
-    __syncthreads();
+}
 
-    // black cells of the brick, written with their red neighbour in x as pairs
-    constexpr int NBLK = (BX / 2) * BY * BZ;
-    for (int t = threadIdx.x; t < NBLK; t += NT) {
-        const int hh = t % (BX / 2), r = t / (BX / 2), yy = r % BY, zz = r / BY;
-        const int gy = y0 + yy, gz = z0 + zz;
-        const int pr = (x0 + gy + gz + 1) & 1;  // red offset in the pair
-        const int xb = 2 * hh + (pr ^ 1);       // brick coordinates of the black cell
-        const int ip = ((zz + 2) * PY + yy + 2) * PX + xb + 2;
-        const int iq = ((zz + 1) * QY + yy + 1) * QX + xb + 1;
-        const int tx = xb + 1, ty = QX + yy + 1, tz = QX + QY + zz + 1;
-        const T bc = sB[ip];
-        const T aR = half * (sB[ip + 1] + bc) * sT[tx];
-        const T aL = half * (bc + sB[ip - 1]) * sT[TM + tx];
-        const T aT = half * (sB[ip + PX] + bc) * sT[ty];
-        const T aB = half * (bc + sB[ip - PX]) * sT[TM + ty];
-        const T aF = half * (sB[ip + PX * PY] + bc) * sT[tz];
-        const T aK = half * (bc + sB[ip - PX * PY]) * sT[TM + tz];
-        const T den = aR + aL + aT + aB + aF + aK;
-        const T self = FIRST ? (T)0 : sP[ip];
-        const T pn = gy == ny - 1 ? self : sR[iq + QX];
-        const T ps = gy == 0 ? self : sR[iq - QX];
-        const T num = -sQ[iq] + (aR * sR[iq + 1] + aL * sR[iq - 1]) + (aT * pn + aB * ps) +
-                      (aF * sR[iq + QX * QY] + aK * sR[iq - QX * QY]);
-        const T vb = smooth_div(num, den);
-        const T vr = sR[iq + 1 - 2 * (pr ^ 1)];  // the red cell of the pair
-        typename Vec2<T>::type v;
-        v.x = pr ? vb : vr;
-        v.y = pr ? vr : vb;
-        *reinterpret_cast<typename Vec2<T>::type*>(pout + plane * gz + (size_t)nx * gy + x0 + 2 * hh) = v;
-    }
+// The same sweep as a march along z with whole rows in a wavefront: a lane holds four
+// cells along x (two red, two black), lr = nx / 4 lanes a row, rw = 64 / lr rows a
+// wavefront, NW wavefronts a workgroup.  At step m a lane updates its red cells of plane
+// m and then its black cells of plane m - 1, whose red neighbours are its own of planes
+// m - 2, m - 1, m (registers), those of the lanes beside it (shuffles: the row's ends
+// meet, so the periodic image is in the wavefront too) and those of the rows beside it
+// (LDS, two slots, one barrier per step).  Every array is read as 4-cell vectors straight
+// into registers, each plane's loads issued a step before their use; the rows beside a
+// lane's own come from L1.  The rows of a wavefront have one parity of j, so which of the
+// four cells are red is uniform and known in each unrolled step: nothing is selected per
+// lane.  The red cells of the rows before and after the tile are recomputed, each plane
+// by two wavefronts that own none.  x and z are uniform axes (validate_grid): one face
+// factor each.
+//
+// Against k_sweep: 150 instead of 210 vector instructions per 4 cells, a fifth of the LDS
+// traffic, no staging.  Per launch, plain / with the dots / from zero: 128x96x128 FP32
+// 14.8 / - / 14.7 -> 8.6 / - / 9.1; 128^3 FP64 28.8 / 36 / 20.7 -> 19 / 26 / 13.7.  A march
+// of the same steps without LDS (the neighbours' red cells recomputed) took twice as long,
+// one with a lane per pair of cells 1.7 times: their loads of single cells strided the
+// L1.  More wavefronts per CU (a bound on registers) spilled and lost; FP64, twice the
+// registers, runs best with two row wavefronts.
+template <class TS>
+struct Quad {
+    TS v[4];
+};
+template <>
+struct alignas(8) Quad<bf16s> {
+    bf16s v[4];
+};
+template <>
+struct alignas(16) Quad<float> {
+    float v[4];
+};
+template <>
+struct alignas(8) Quad<double> {  // (a caller's array need only be aligned to its elements)
+    double v[4];
+};
+
+template <class TS>
+__device__ __forceinline__ Quad<TS> load4(const TS* __restrict__ base, unsigned e)
+{
+    return *reinterpret_cast<const Quad<TS>*>(reinterpret_cast<const char*>(base) + e * (unsigned)sizeof(TS));
+}
+template <class T, class TS>
+__device__ __forceinline__ void widen(T (&d)[4], const Quad<TS>& x)
+{
+#pragma unroll
+    for (int i = 0; i < 4; ++i) d[i] = (T)x.v[i];
+}
+
+// a lane's cells, and the rows beside them with q of its own: as loaded (in flight), and
+// in the arithmetic's type
+template <class T, class TB>
+struct RawCentre {
+    Quad<TB> b;
+    Quad<T> p;
+};
+template <class T, class TQ, class TB>
+struct RawSides {
+    Quad<TB> bn, bs;
+    Quad<T> pn, ps;
+    Quad<TQ> q;
+};
+template <class T>
+struct RowCentre {
+    T b[4], p[4];
+};
+
+// wavefronts of a workgroup that own rows; two more compute the red cells of the rows
+// before and after the tile
+template <class T>
+constexpr int row_waves() { return sizeof(T) == 4 ? 6 : 2; }
+
+template <class T, class TQ, class TB, bool FIRST, bool DOTS>
+__global__ void __launch_bounds__(64 * (row_waves<T>() + 2))
+    k_row_sweep(LevelDev<T> L, const TB* __restrict__ beta, const TQ* __restrict__ q, const T* __restrict__ pin,
+                T* __restrict__ pout, int kc, int lr, int rw, int ntiles, const int* done, SweepDots dots)
+{
+    constexpr int NW = row_waves<T>();
+    __shared__ T sR[2][2 * 64 * (NW + 2)];  // red values, rows -1 .. NW rw of 2 lr
+    if (done && *done) return;
+    unsigned id = blockIdx.x;  // consecutive tiles of a chunk on one XCD
+    if ((gridDim.x & 7u) == 0) id = (id & 7u) * (gridDim.x >> 3) + (id >> 3);
+    const int nx = L.nx, ny = L.ny, nz = L.nz;
+    const int k0 = (int)(id / (unsigned)ntiles) * kc, k1 = min(nz, k0 + kc);
+    const int ty0 = (int)(id % (unsigned)ntiles) * NW * rw;
+    const int lane = (int)threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), cls = wave & 1;
+    // wavefronts NW, NW + 1: the row after the tile and the one before it
+    const bool ring = wave >= NW;
+    const int rows = ring ? 1 : rw;
+    const int li = min(lane / lr, rows - 1), xl = lane / lr < rows ? lane - li * lr : 0;
+    // row in the tile, of parity cls (ty0 and NW are even)
+    const int r = ring ? (cls ? -1 : NW * rw) : 2 * ((wave >> 1) * rw + li) + cls;
+    const bool put = lane / lr < rows && ty0 + r >= 0 && ty0 + r < ny;
+    const bool own = put && !ring;
+    const int j = min(max(ty0 + r, 0), ny - 1), jn = min(j + 1, ny - 1), js = max(j - 1, 0);
+    const bool wall_n = j == ny - 1, wall_s = j == 0;
+    const int left = li * lr + (xl > 0 ? xl - 1 : lr - 1), right = li * lr + (xl + 1 < lr ? xl + 1 : 0);
+    const unsigned oc = (unsigned)(nx * j + 4 * xl), on = (unsigned)(nx * jn + 4 * xl), os = (unsigned)(nx * js + 4 * xl);
+    const T half = (T)0.5;
+    const T fx = half * L.a[0].ip[0], fz = half * L.a[2].ip[0];
+    const T yp = half * L.a[1].ip[j], ym = half * L.a[1].im[j];
+    const size_t plane = (size_t)nx * ny;
+    auto wrap = [&](int k) { return k < 0 ? k + nz : (k >= nz ? k - nz : k); };
+    auto load_c = [&](RawCentre<T, TB>& v, int k) __attribute__((always_inline)) {
+        const size_t o = plane * (size_t)wrap(min(k, k1 + 1));  // (the last planes' prefetch: a plane already read)
+        v.b = load4(beta + o, oc);
+        if (!FIRST) v.p = load4(pin + o, oc);
+    };
+    auto load_s = [&](RawSides<T, TQ, TB>& v, int k) __attribute__((always_inline)) {
+        const size_t o = plane * (size_t)wrap(min(k, k1 + 1));
+        v.bn = load4(beta + o, on);
+        v.bs = load4(beta + o, os);
+        v.q = load4(q + o, oc);
+        if (!FIRST) {
+            v.pn = load4(pin + o, on);
+            v.ps = load4(pin + o, os);
+        }
+    };
+    auto take_c = [&](RowCentre<T>& d, const RawCentre<T, TB>& v) __attribute__((always_inline)) {
+        widen(d.b, v.b);
+        if (!FIRST) widen(d.p, v.p);
+    };
+    auto update = [&](T qq, T c, T bE, T bW, T bN, T bS, T bF, T bB, T fyp, T fym, T pE, T pW, T pN, T pS, T pF, T pB,
+                      auto red) __attribute__((always_inline)) {
+        return smooth_cell<T, FIRST && decltype(red)::value>(
+            qq, c, {bE, bW, bN, bS, bF, bB}, fx, fx, fyp, fym, fz, fz, {pE, pW, pN, pS, pF, pB});
+    };
+    // the red cells of four (P: the parity of row + plane; red are 0, 2 if odd, 1, 3 if
+    // even) from the rows about them; be, pe: the cell next to the four on the red side
+    auto red2 = [&](auto par, T (&out)[2], const T (&qq)[4], const T (&b)[4], const T (&bn)[4], const T (&bs)[4],
+                    const T (&bf)[4], const T (&bk)[4], const T (&p)[4], const T (&pn)[4], const T (&ps)[4],
+                    const T (&pf)[4], const T (&pk)[4], T be, T pe, T fyp, T fym) __attribute__((always_inline)) {
+        constexpr int P = decltype(par)::value;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            constexpr int odd = P ? 0 : 1;
+            const int e = 2 * i + odd;
+            const T bE = e < 3 ? b[e < 3 ? e + 1 : 3] : be, bW = e > 0 ? b[e > 0 ? e - 1 : 0] : be;
+            const T pE = e < 3 ? p[e < 3 ? e + 1 : 3] : pe, pW = e > 0 ? p[e > 0 ? e - 1 : 0] : pe;
+            out[i] = update(qq[e], b[e], bE, bW, bn[e], bs[e], bf[e], bk[e], fyp, fym, pE, pW, pn[e], ps[e], pf[e], pk[e],
+                            std::true_type());
+        }
+    };
+
+    double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};  // DOTS: the sums of k_pcg_dots, one partial per workgroup
+    RawCentre<T, TB> rc;       // plane m + 1 (at a step's start), then m + 2
+    RawSides<T, TQ, TB> rs;    // plane m, then m + 1
+    RowCentre<T> C[3];         // planes m - 1, m, m + 1
+    T R2[2] = {(T)0, (T)0}, R1[2] = {(T)0, (T)0};  // new red values of planes m - 2, m - 1
+    T kb[2] = {(T)0, (T)0};                        // beta of plane m - 2 behind the black cells of m - 1
+    T kn[2] = {(T)0, (T)0}, ks[2] = {(T)0, (T)0}, kq[2] = {(T)0, (T)0};  // of plane m - 1: beta n, s and q there
+    load_c(rc, k0 - 2);
+    take_c(C[1], rc);
+    load_c(rc, k0 - 1);
+    take_c(C[2], rc);
+    load_c(rc, k0);
+    load_s(rs, k0 - 1);
+    T* const mine = sR[0] + (r + 1) * 2 * lr + 2 * xl;
+    constexpr int kSlot = 2 * 64 * (NW + 2);
+    constexpr int kUnroll = sizeof(T) == 4 ? 4 : 2;  // steps per turn of the loop (registers)
+
+    auto step = [&](auto par, int m, int sl) __attribute__((always_inline)) {
+        constexpr int P = decltype(par)::value;        // parity of row + m
+        constexpr int o_red = P ? 0 : 1, o_blk = P ? 1 : 0;  // of plane m; of plane m - 1 the other way round
+        C[0] = C[1];
+        C[1] = C[2];
+        take_c(C[2], rc);
+        const RowCentre<T>&Cm = C[0], &C0 = C[1], &Cp = C[2];
+        T s_bn[4], s_bs[4], s_q[4], s_pn[4], s_ps[4];
+        widen(s_bn, rs.bn);
+        widen(s_bs, rs.bs);
+        widen(s_q, rs.q);
+        if (!FIRST) {
+            widen(s_pn, rs.pn);
+            widen(s_ps, rs.ps);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        load_c(rc, m + 2);
+        load_s(rs, m + 1);
+        const bool black = m > k0;
+        const size_t ob = plane * (size_t)wrap(m - 1) + oc;
+        double dr[4] = {0.0, 0.0, 0.0, 0.0}, dq[4] = {0.0, 0.0, 0.0, 0.0};
+        if (DOTS && black && !ring) {
+            widen(dr, load4(dots.r + ob, 0));
+            if (!dots.init) widen(dq, load4(dots.qv + ob, 0));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        T R0[2];
+        {
+            const T be = __shfl(C0.b[P ? 3 : 0], P ? left : right, 64);
+            const T pe = FIRST ? (T)0 : __shfl(C0.p[P ? 3 : 0], P ? left : right, 64);
+            red2(par, R0, s_q, C0.b, s_bn, s_bs, Cp.b, Cm.b, C0.p, s_pn, s_ps, Cp.p, Cm.p, be, pe, yp, ym);
+        }
+        __syncthreads();  // plane m - 1 is in LDS, and plane m - 2's readers are done
+        if (put) {
+            mine[sl * kSlot] = R0[0];
+            mine[sl * kSlot + 1] = R0[1];
+        }
+        if (black && !ring) {
+            // black cells of plane m - 1 at o_red + {0, 2} (the red positions of plane m)
+            const T* at = mine + (sl ^ 1) * kSlot;
+            const T be = __shfl(Cm.b[P ? 3 : 0], P ? left : right, 64);
+            const T re = __shfl(R1[P ? 1 : 0], P ? left : right, 64);
+            T vb[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int e = 2 * i + o_red;
+                const T bE = e < 3 ? Cm.b[e < 3 ? e + 1 : 3] : be, bW = e > 0 ? Cm.b[e > 0 ? e - 1 : 0] : be;
+                // its red neighbours along x: R1 holds the cells at o_blk + {0, 2}
+                const T rE = P ? R1[i] : (i == 0 ? R1[1] : re), rW = P ? (i == 0 ? re : R1[0]) : R1[i];
+                const T self = FIRST ? (T)0 : Cm.p[e];  // a wall's ghost: the cell before the sweep
+                const T rn = wall_n ? self : at[2 * lr + i], rs = wall_s ? self : at[i - 2 * lr];
+                vb[i] = update(kq[i], Cm.b[e], bE, bW, kn[i], ks[i], C0.b[e], kb[i], yp, ym, rE, rW, rn, rs, R0[i],
+                               R2[i], std::false_type());
+            }
+            if (own) {
+                Quad<T> v;
+                v.v[o_red] = vb[0], v.v[o_red + 2] = vb[1];
+                v.v[o_blk] = R1[0], v.v[o_blk + 2] = R1[1];
+                *reinterpret_cast<Quad<T>*>(pout + ob) = v;
+                if (DOTS) {  // the order of k_pcg_dots, cell by cell
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const double z = (double)v.v[e];
+                        acc[0] += dr[e] * z;
+                        acc[2] += z;
+                        acc[3] += dr[e];
+                        if (!dots.init) {
+                            acc[1] += dq[e] * z;
+                            acc[4] += dq[e];
+                        }
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int e = 2 * i + o_blk;  // plane m's black cells, the next step's
+            kb[i] = Cm.b[e], kn[i] = s_bn[e], ks[i] = s_bs[e], kq[i] = s_q[e];
+            R2[i] = R1[i], R1[i] = R0[i];
+        }
+    };
+    auto march = [&](auto p0) {  // p0: the parity of row + (k0 - 1)
+        constexpr int A = decltype(p0)::value;
+        const std::integral_constant<int, A> pa;
+        const std::integral_constant<int, 1 - A> pb;
+        for (int m = k0 - 1; m <= k1; m += kUnroll) {
+#pragma unroll
+            for (int u = 0; u < kUnroll; u += 2) {
+                if (u > 0 && m + u > k1) break;
+                step(pa, m + u, 0);
+                if (m + u + 1 > k1) break;
+                step(pb, m + u + 1, 1);
+            }
+        }
+    };
+    if ((cls + k0 - 1) & 1)
+        march(std::integral_constant<int, 1>{});
+    else
+        march(std::integral_constant<int, 0>{});
+    if (DOTS) block_partial<5>(acc, dots.red);
 }
 
 }  // namespace
 
 template <class T>
-static void brick_dims(int& bx, int& by, int& bz)
+bool point_supported(const LevelDev<T>& L)
 {
-    bx = 16;
-    by = 8;
-    bz = sizeof(T) == 4 ? 8 : 4;
-}
-
-template <class T>
-bool brick_supported(const LevelDev<T>& L)
-{
-    int bx, by, bz;
-    brick_dims<T>(bx, by, bz);
-    return L.nx % bx == 0 && L.ny % by == 0 && L.nz % bz == 0 && L.nz % 2 == 0;
+    // pairs along x, the colours of a periodic z, indices of the launch and of its
+    // divisions in 32 bits
+    const uint64_t pairs = (uint64_t)(L.nx / 2) * L.ny * L.nz;
+    return L.nx % 2 == 0 && L.nz % 2 == 0 && pairs * (uint64_t)std::max(L.nx / 2, L.ny) < ((uint64_t)1 << 32) &&
+           pairs < ((uint64_t)1 << 30);
 }
 
 template <class T, class TQ>
-int launch_brick_sweep(const LevelDev<T>& L, const T* beta, const TQ* q, const T* pin, T* pout, bool first,
-                       const int* done, void* stream)
+int launch_point_sweep(const LevelDev<T>& L, const T* beta, const TQ* q, const T* pin, T* pout, bool first,
+                       const int* done, void* stream, const SweepDots* dots, unsigned* nblocks_out)
 {
-    if (!brick_supported(L)) {
-        set_error("launch_brick_sweep: level %dx%dx%d not supported", L.nx, L.ny, L.nz);
+    if (!point_supported(L) || (dots && first)) {
+        set_error("launch_point_sweep: level %dx%dx%d not supported", L.nx, L.ny, L.nz);
         return TBFG_EINVAL;
     }
-    int bx, by, bz;
-    brick_dims<T>(bx, by, bz);
-    const dim3 grid((unsigned)((L.nx / bx) * (L.ny / by) * (L.nz / bz)));
-    constexpr int BZ = sizeof(T) == 4 ? 8 : 4;
-    if (first)
-        hipLaunchKernelGGL((k_brick_sweep<T, TQ, 16, 8, BZ, true>), grid, dim3(kBrickThreads), 0, (hipStream_t)stream,
-                           L, beta, q, pin, pout, done);
-    else
-        hipLaunchKernelGGL((k_brick_sweep<T, TQ, 16, 8, BZ, false>), grid, dim3(kBrickThreads), 0,
-                           (hipStream_t)stream, L, beta, q, pin, pout, done);
+    auto magic = [](int d) { return d <= 1 ? 0u : (uint32_t)((((uint64_t)1 << 32) + (uint64_t)d - 1) / (uint64_t)d); };
+    const int pairs = (L.nx / 2) * L.ny * L.nz;
+    const unsigned nblocks = ceil_div((size_t)pairs, 256);
+    if (dots && (size_t)nblocks * 5 > dots->capacity) {
+        set_error("launch_point_sweep: %u workgroups exceed the reduction scratch", nblocks);
+        return TBFG_EINVAL;
+    }
+    auto k = dots    ? k_point_sweep<T, TQ, false, true>
+             : first ? k_point_sweep<T, TQ, true, false>
+                     : k_point_sweep<T, TQ, false, false>;
+    hipLaunchKernelGGL(k, dim3(nblocks), dim3(256), 0, (hipStream_t)stream, L, beta, q, pin, pout, magic(L.nx / 2),
+                       magic(L.ny), pairs, done, dots ? *dots : SweepDots{});
     TBFG_HIP(hipGetLastError());
+    if (nblocks_out) *nblocks_out = nblocks;
     return TBFG_OK;
+}
+
+template <class T>
+bool row_supported(const LevelDev<T>& L)
+{
+    // rows of 4-cell lanes that fit a wavefront, the colours of a periodic z, the plane's
+    // element offsets in 32-bit bytes
+    return L.nx % 4 == 0 && L.nx >= 16 && L.nx <= 256 && L.nz % 2 == 0 && L.nz >= 4 &&
+           (uint64_t)L.nx * L.ny < ((uint64_t)1 << 28);
+}
+
+template <class T, class TQ, class TB, bool FIRST, bool DOTS>
+static int launch_row_form(const LevelDev<T>& L, const TB* beta, const TQ* q, const T* pin, T* pout, const int* done,
+                           const SweepDots& dots, unsigned* nblocks_out, void* stream, const KernelEvents* kev)
+{
+    // resident workgroups per CU and CU count, queried once (threads may race
+    // to fill it; they store the same value)
+    static std::atomic<int> occ{-1};
+    auto k = k_row_sweep<T, TQ, TB, FIRST, DOTS>;
+    int o = occ.load(std::memory_order_acquire);
+    if (o < 0) {
+        int dev = 0, ncu = 0, nb = 0;
+        TBFG_HIP(hipGetDevice(&dev));
+        TBFG_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+        TBFG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k, 64 * (row_waves<T>() + 2), 0));
+        o = (nb < 1 ? 1 : nb) * (ncu > 0 ? ncu : 256);
+        occ.store(o, std::memory_order_release);
+    }
+    // one resident round of workgroups (a second, partly filled one costs as much as a
+    // full one), chunks of at least 4 planes
+    const int lr = L.nx / 4, rw = 64 / lr;
+    const int ntiles = (int)ceil_div(L.ny, row_waves<T>() * rw);
+    const int chunks = std::max(1, std::min(L.nz / 4, o / ntiles));
+    int kc = (L.nz + chunks - 1) / chunks;
+    const unsigned nblocks = (unsigned)ntiles * ceil_div(L.nz, kc);
+    if (DOTS && (size_t)nblocks * 5 > dots.capacity) {
+        set_error("launch_row_sweep: %u workgroups exceed the reduction scratch", nblocks);
+        return TBFG_EINVAL;
+    }
+    const dim3 blk(64 * (row_waves<T>() + 2));
+    if (kev)
+        hipExtLaunchKernelGGL(k, dim3(nblocks), blk, 0, (hipStream_t)stream, kev->start, kev->stop, 0, L, beta, q, pin,
+                              pout, kc, lr, rw, ntiles, done, dots);
+    else
+        hipLaunchKernelGGL(k, dim3(nblocks), blk, 0, (hipStream_t)stream, L, beta, q, pin, pout, kc, lr, rw, ntiles, done,
+                           dots);
+    TBFG_HIP(hipGetLastError());
+    if (nblocks_out) *nblocks_out = nblocks;
+    return TBFG_OK;
+}
+
+template <class T, class TQ, class TB>
+int launch_row_sweep(const LevelDev<T>& L, const TB* beta, const TQ* q, const T* pin, T* pout, bool first,
+                     const int* done, void* stream, const SweepDots* dots, unsigned* nblocks_out,
+                     const KernelEvents* kev)
+{
+    if (!row_supported(L) || (dots && first)) {
+        set_error("launch_row_sweep: level %dx%dx%d not supported", L.nx, L.ny, L.nz);
+        return TBFG_EINVAL;
+    }
+    const SweepDots none{};
+    if (dots) return launch_row_form<T, TQ, TB, false, true>(L, beta, q, pin, pout, done, *dots, nblocks_out, stream, kev);
+    return first ? launch_row_form<T, TQ, TB, true, false>(L, beta, q, pin, pout, done, none, nblocks_out, stream, kev)
+                 : launch_row_form<T, TQ, TB, false, false>(L, beta, q, pin, pout, done, none, nblocks_out, stream, kev);
 }
 
 struct SweepCfg {
@@ -639,9 +930,11 @@ constexpr SweepCfg kShapesF[] = {{64, 8, 256}, {32, 16, 256}, {64, 16, 512}, {32
 constexpr SweepCfg kShapesFPlain[] = {{32, 16, 256}, {64, 8, 256}, {64, 16, 512}, {32, 8, 128}};
 constexpr SweepCfg kShapesD[] = {{64, 4, 128}, {64, 8, 256}, {32, 8, 128}};
 
+// tuned (optional): whether TBFG_SWEEP_SHAPE or the tuning table names the shape
 template <class T>
-static bool pick_shape(const LevelDev<T>& L, SweepCfg& out, bool plain = false)
+static bool pick_shape(const LevelDev<T>& L, SweepCfg& out, bool plain = false, bool* tuned_out = nullptr)
 {
+    if (tuned_out) *tuned_out = false;
     // nz even (the colour of a plane is its index's parity), nz >= 16 (a
     // chunk's plane steps wrap around z at most once); the level's arrays
     // addressable by 32-bit buffer offsets (< 2 GiB)
@@ -664,6 +957,7 @@ static bool pick_shape(const LevelDev<T>& L, SweepCfg& out, bool plain = false)
             if (pass == 0 && !(c.tx == want_tx && c.ty == want_ty && c.nt == want_nt)) continue;
             if (L.nx % c.tx == 0 && L.ny % c.ty == 0) {
                 out = c;
+                if (tuned_out) *tuned_out = pass == 0;
                 return true;
             }
         }
@@ -675,6 +969,13 @@ bool sweep_supported(const LevelDev<T>& L)
 {
     SweepCfg c;
     return pick_shape(L, c);
+}
+template <class T>
+bool sweep_named(const LevelDev<T>& L, bool plain)
+{
+    SweepCfg c;
+    bool tuned = false;
+    return pick_shape(L, c, plain, &tuned) && tuned;
 }
 
 // prefetch distance in plane steps: 4 in FP32 on long chunks; 2 in FP64, with
@@ -783,14 +1084,22 @@ int launch_sweep(const LevelDev<T>& L, const TB* beta, const TQ* q, const T* pin
     return TBFG_EINVAL;
 }
 
-template bool brick_supported<float>(const LevelDev<float>&);
-template bool brick_supported<double>(const LevelDev<double>&);
-template int launch_brick_sweep<float, float>(const LevelDev<float>&, const float*, const float*, const float*,
-                                              float*, bool, const int*, void*);
-template int launch_brick_sweep<double, double>(const LevelDev<double>&, const double*, const double*,
-                                                const double*, double*, bool, const int*, void*);
+template bool row_supported<float>(const LevelDev<float>&);
+template bool row_supported<double>(const LevelDev<double>&);
+template int launch_row_sweep<float, float, float>(const LevelDev<float>&, const float*, const float*, const float*, float*, bool,
+                                             const int*, void*, const SweepDots*, unsigned*, const KernelEvents*);
+template int launch_row_sweep<double, double, double>(const LevelDev<double>&, const double*, const double*, const double*, double*, bool,
+                                             const int*, void*, const SweepDots*, unsigned*, const KernelEvents*);
+template bool point_supported<float>(const LevelDev<float>&);
+template bool point_supported<double>(const LevelDev<double>&);
+template int launch_point_sweep<float, float>(const LevelDev<float>&, const float*, const float*, const float*,
+                                              float*, bool, const int*, void*, const SweepDots*, unsigned*);
+template int launch_point_sweep<double, double>(const LevelDev<double>&, const double*, const double*, const double*,
+                                                double*, bool, const int*, void*, const SweepDots*, unsigned*);
 template bool sweep_supported<float>(const LevelDev<float>&);
 template bool sweep_supported<double>(const LevelDev<double>&);
+template bool sweep_named<float>(const LevelDev<float>&, bool);
+template bool sweep_named<double>(const LevelDev<double>&, bool);
 template int launch_sweep<float, float, float>(const LevelDev<float>&, const float*, const float*, const float*,
                                                float*, bool, const int*, void*, const SweepDots*, unsigned*,
                                                const KernelEvents*);

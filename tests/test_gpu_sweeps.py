@@ -1,0 +1,98 @@
+"""The two sweep kernels without LDS staging against the two half-sweep launches: one
+preconditioner application at the remainders of their tiles and chunks -- rows from 16
+cells to a full wavefront, several rows to a wavefront, heights and depths that leave the
+last tile and chunk partly filled, axes of two cells.  The same arithmetic up to fused
+multiply-adds, so the bounds of the other sweep tests (1e-13 in FP64, 1e-6 in FP32)."""
+import numpy as np
+import pytest
+
+import tbfsolver_amd as T
+from tbfsolver_amd import fields as F
+from conftest import to_dev, to_host
+
+pytestmark = pytest.mark.gpu
+
+
+def case(torch, n, seed=9):
+    g = T.channel_grid(n, stretch_y=1, gamma=1.5)
+    r = np.random.default_rng(seed)
+    beta = to_dev(np.exp(r.uniform(-1.5, 1.5, n)), torch)
+    q = torch.zeros_like(beta)
+    F.computeSource(g, *(to_dev(a, torch) for a in F.make_velocity(g, seed)), q)
+    return g, beta, q
+
+
+def apply(torch, g, beta, q, **kw):
+    s = T.PCG(g, nLevels=2, nPreSweep=2, nPostSweep=3, coarse_max_iter=0, **kw)
+    z = torch.zeros_like(q)
+    s.precondition(beta, q, z)
+    out = to_host(z)
+    s.close()
+    return out
+
+
+def rel(a, b):
+    return np.linalg.norm(a - b) / np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("precision,bound", [("fp64", 1e-13), ("mixed", 1e-6)])
+@pytest.mark.parametrize("n", [(16, 6, 8), (20, 10, 4), (36, 14, 6), (44, 18, 4), (100, 4, 8), (16, 62, 4), (72, 40, 56),
+                               (252, 2, 4), (256, 12, 8), (128, 20, 8)])
+def test_row_sweep_matches_half_sweeps(torch_gpu, monkeypatch, n, precision, bound):
+    print("case row sweep", n, precision, flush=True)
+    c = case(torch_gpu, n)
+    monkeypatch.setenv("TBFG_SWEEP_MIN_CELLS", "0")
+    a = apply(torch_gpu, *c, precision=precision)
+    monkeypatch.setenv("TBFG_HALF_SWEEPS", "1")
+    b = apply(torch_gpu, *c, precision=precision)
+    assert np.all(np.isfinite(a)) and rel(a, b) < bound
+
+
+@pytest.mark.parametrize("precision,bound", [("fp64", 1e-13), ("mixed", 1e-6)])
+@pytest.mark.parametrize("n", [(2, 2, 2), (2, 6, 8), (6, 10, 4), (18, 14, 10), (34, 2, 6), (260, 4, 2), (72, 40, 56)])
+def test_point_sweep_matches_half_sweeps(torch_gpu, monkeypatch, n, precision, bound):
+    print("case point sweep", n, precision, flush=True)
+    c = case(torch_gpu, n)
+    monkeypatch.setenv("TBFG_SWEEP_MIN_CELLS", str(10 ** 12))
+    a = apply(torch_gpu, *c, precision=precision)
+    monkeypatch.setenv("TBFG_HALF_SWEEPS", "1")
+    b = apply(torch_gpu, *c, precision=precision)
+    assert np.all(np.isfinite(a)) and rel(a, b) < bound
+
+
+@pytest.mark.parametrize("precision,bound", [("mixed-bf16", 1e-6), ("mixed", 1e-6), ("fp64", 1e-13)])
+def test_row_sweep_matches_staged_tiles(torch_gpu, monkeypatch, precision, bound):
+    """The same level by rows and by a tile shape of the staged kernel, which the shape
+    switch (or an entry of the tuning table) selects, bf16 storage included."""
+    n = (64, 48, 64)
+    print("case row sweep vs staged tiles", precision, flush=True)
+    c = case(torch_gpu, n)
+    monkeypatch.setenv("TBFG_SWEEP_MIN_CELLS", "0")
+    a = apply(torch_gpu, *c, precision=precision)
+    monkeypatch.setenv("TBFG_SWEEP_SHAPE", "64x8x256")
+    b = apply(torch_gpu, *c, precision=precision)
+    assert rel(a, b) < bound
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("n,min_cells", [((72, 40, 56), 0), ((72, 40, 56), 10 ** 12), ((36, 12, 20), 0), ((18, 14, 10), 0)])
+def test_dots_in_row_and_point_sweeps(torch_gpu, monkeypatch, n, min_cells, precision):
+    """A solve with the dot products formed by the last sweep against the separate pass:
+    the same iterations and, to 1e-11 residual, the same pressure to 1e-9 (the sums'
+    order alone differs)."""
+    print("case dots in sweeps", n, min_cells, precision, flush=True)
+    g, beta, q = case(torch_gpu, n)
+    monkeypatch.setenv("TBFG_SWEEP_MIN_CELLS", str(min_cells))
+    out = []
+    for unfused in (False, True):
+        if unfused:
+            monkeypatch.setenv("TBFG_UNFUSED_DOTS", "1")
+        s = T.PCG(g, nLevels=2, tolPCG=1e-11, maxIterPCG=200, precision=precision, flexible=1, coarse_max_iter=0)
+        psi = torch_gpu.zeros_like(q)
+        s.solvePCG(psi, beta, q)
+        assert s.converged
+        p = to_host(psi)
+        out.append((s.iterations, p - p.mean()))
+        s.close()
+    assert abs(out[0][0] - out[1][0]) <= 1
+    assert rel(out[0][1], out[1][1]) < 1e-9
