@@ -74,11 +74,12 @@ template <class T, class TQ, class TB = T>
 int launch_sweep(const LevelDev<T>& L, const TB* beta, const TQ* q, const T* pin, T* pout, bool first,
                  const int* done, void* stream, const SweepDots* dots = nullptr, unsigned* nblocks_out = nullptr,
                  const KernelEvents* kev = nullptr);
-// the march with whole rows in a wavefront (nx a multiple of 4, 16..256)
+// the march with whole rows in a wavefront (nx a multiple of 4, 16..256); tiles (FP32,
+// where sweep_supported, without dots): bit for bit as launch_sweep
 template <class T>
 bool row_supported(const LevelDev<T>& L);
 template <class T, class TQ, class TB = T>
-int launch_row_sweep(const LevelDev<T>& L, const TB* beta, const TQ* q, const T* pin, T* pout, bool first,
+int launch_row_sweep(const LevelDev<T>& L, const TB* beta, const TQ* q, const T* pin, T* pout, bool first, bool tiles,
                      const int* done, void* stream, const SweepDots* dots = nullptr, unsigned* nblocks_out = nullptr,
                      const KernelEvents* kev = nullptr);
 // a thread per pair of cells (any even nx, nz)

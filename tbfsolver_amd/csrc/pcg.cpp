@@ -542,36 +542,32 @@ static int smooth(tbfg_pcg* h, int l, const T0* b, const T0* q, T*& p, T*& alt, 
     }
     for (int s = 0; s < nsweeps; ++s) {
         const bool f0 = first && s == 0;
-        if constexpr (narrow) {
-            const bool last = s == nsweeps - 1;
-            const bool plain = l == 0 && !f0 && !(last && last_dots);
-            ProfScope ps(h, plain ? 0 : -1, stream, true);
-            TBFG_TRY(launch_sweep<T, T0, T0>(L, b, q, p, alt, f0, done, stream, last ? last_dots : nullptr,
-                                             last ? nb_out : nullptr, ps.events()));
-            std::swap(p, alt);
-        } else if (h->fused[l] == 2) {
-            ProfScope ps(h, l == 0 ? 0 : -1, stream);
-            const bool last = s == nsweeps - 1;
-            TBFG_TRY(launch_point_sweep<T, T>(L, b, q, p, alt, f0, done, stream, last ? last_dots : nullptr,
-                                              last ? nb_out : nullptr));
-            std::swap(p, alt);
-        } else if (h->fused[l]) {
-            const bool last = s == nsweeps - 1;
+        const bool last = s == nsweeps - 1;
+        const SweepDots* dots = last ? last_dots : nullptr;
+        unsigned* nb = last ? nb_out : nullptr;
+        if (h->fused[l] == 1 || h->fused[l] == 3) {
             // the timed finest-level sweep: from a non-zero start, without the dot products
-            const bool plain = l == 0 && !f0 && !(last && last_dots);
+            const bool plain = l == 0 && !f0 && !dots;
             ProfScope ps(h, plain ? 0 : -1, stream, true);
-            // by rows, except where a tile shape is asked for, and under bf16 storage: the
-            // residual cut to 8 bits there turns a last bit of FP32 into a few 1e-9 of the
-            // solution (1 % of its error), so those levels keep k_sweep's order of sums
-            const bool tiles = h->fused[l] == 1 && (h->b16 || !row_supported<T>(L) || sweep_named<T>(L, !f0 && !(last && last_dots)));
-            auto go = tiles ? launch_sweep<T, T, T> : launch_row_sweep<T, T, T>;
-            TBFG_TRY(go(L, b, q, p, alt, f0, done, stream, last ? last_dots : nullptr, last ? nb_out : nullptr,
-                        ps.events()));
+            // by rows, except where a tile shape is asked for.  Under bf16 storage the last bit
+            // of a sweep or of a dot product becomes a few 1e-9 of the solution (1 % of its
+            // error), the residual being cut to 8 bits: there the rows round as the tiles
+            // do, and the sweep that forms the dot products stays with them
+            if (h->fused[l] == 1 && (!row_supported<T>(L) || sweep_named<T>(L, !f0 && !dots) || (h->b16 && dots)))
+                TBFG_TRY(launch_sweep<T, T0, T0>(L, b, q, p, alt, f0, done, stream, dots, nb, ps.events()));
+            else
+                TBFG_TRY(launch_row_sweep<T, T0, T0>(L, b, q, p, alt, f0, h->b16 && h->fused[l] == 1, done, stream, dots,
+                                                     nb, ps.events()));
             std::swap(p, alt);
-        } else {
+        } else if constexpr (!narrow) {
             ProfScope ps(h, l == 0 ? 0 : -1, stream);
-            TBFG_TRY(launch_rbgs<T, T>(L, b, q, p, RED, f0, done, stream));
-            TBFG_TRY(launch_rbgs<T, T>(L, b, q, p, BLACK, f0, done, stream));
+            if (h->fused[l] == 2) {
+                TBFG_TRY(launch_point_sweep<T, T>(L, b, q, p, alt, f0, done, stream, dots, nb));
+                std::swap(p, alt);
+            } else {
+                TBFG_TRY(launch_rbgs<T, T>(L, b, q, p, RED, f0, done, stream));
+                TBFG_TRY(launch_rbgs<T, T>(L, b, q, p, BLACK, f0, done, stream));
+            }
         }
     }
     return TBFG_OK;

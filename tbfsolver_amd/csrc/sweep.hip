@@ -3,8 +3,8 @@
 // values before the sweep and is only read, pout receives the values after it.
 // Three kernels, chosen per level (pcg_create, smooth):
 //   k_row_sweep    marches along z with whole rows of up to 256 cells in a wavefront
-//   k_sweep        marches along z with tiles staged in LDS: rows longer than that, bf16
-//                  storage, and the tile shapes a tuning table names
+//   k_sweep        marches along z with tiles staged in LDS: rows longer than that, the tile
+//                  shapes a tuning table names, the dot products under bf16 storage
 //   k_point_sweep  no march, a thread per pair of cells: small levels and odd row lengths
 // The values a workgroup needs from beyond its cells are recomputed from pin, so
 // no workgroup waits on another and the result equals the two half-sweep launches up to
@@ -569,7 +569,8 @@ __global__ void __launch_bounds__(256)
 //
 // Against k_sweep: 150 instead of 210 vector instructions per 4 cells, a fifth of the LDS
 // traffic, no staging.  Per launch, plain / with the dots / from zero: 128x96x128 FP32
-// 14.8 / - / 14.7 -> 8.6 / - / 9.1; 128^3 FP64 28.8 / 36 / 20.7 -> 19 / 26 / 13.7.  A march
+// 14.8 / - / 14.7 -> 8.6 / - / 9.1; 128^3 FP64 28.8 / 36 / 20.7 -> 19 / 26 / 13.7; with bf16
+// q and beta 256x192x256 46.2 / - / 44.6 -> 35 / - / 33 (30 / 20 at the copy rate).  A march
 // of the same steps without LDS (the neighbours' red cells recomputed) took twice as long,
 // one with a lane per pair of cells 1.7 times: their loads of single cells strided the
 // L1.  More wavefronts per CU (a bound on registers) spilled and lost; FP64, twice the
@@ -626,13 +627,16 @@ struct RowCentre {
 template <class T>
 constexpr int row_waves() { return sizeof(T) == 4 ? 6 : 2; }
 
-template <class T, class TQ, class TB, bool FIRST, bool DOTS>
+// TILES: rounded as k_sweep rounds with tiles of tx x ty cells (powers of two, tx >= 4):
+// black cells take red neighbours across a tile's edge in their other rounding.
+template <class T, class TQ, class TB, bool FIRST, bool DOTS, bool TILES>
 __global__ void __launch_bounds__(64 * (row_waves<T>() + 2))
     k_row_sweep(LevelDev<T> L, const TB* __restrict__ beta, const TQ* __restrict__ q, const T* __restrict__ pin,
-                T* __restrict__ pout, int kc, int lr, int rw, int ntiles, const int* done, SweepDots dots)
+                T* __restrict__ pout, int kc, int lr, int rw, int ntiles, int tx, int ty, const int* done, SweepDots dots)
 {
     constexpr int NW = row_waves<T>();
-    __shared__ T sR[2][2 * 64 * (NW + 2)];  // red values, rows -1 .. NW rw of 2 lr
+    constexpr int kSlot = 2 * 64 * (NW + 2);
+    __shared__ T sR[(TILES ? 4 : 2) * kSlot];  // red values, rows -1 .. NW rw of 2 lr; as seen across a tile's edge
     if (done && *done) return;
     unsigned id = blockIdx.x;  // consecutive tiles of a chunk on one XCD
     if ((gridDim.x & 7u) == 0) id = (id & 7u) * (gridDim.x >> 3) + (id >> 3);
@@ -653,6 +657,9 @@ __global__ void __launch_bounds__(64 * (row_waves<T>() + 2))
     const bool wall_n = j == ny - 1, wall_s = j == 0;
     const int left = li * lr + (xl > 0 ? xl - 1 : lr - 1), right = li * lr + (xl + 1 < lr ? xl + 1 : 0);
     const unsigned oc = (unsigned)(nx * j + 4 * xl), on = (unsigned)(nx * jn + 4 * xl), os = (unsigned)(nx * js + 4 * xl);
+    // TILES: the row's neighbours and the lane's ends across a tile's edge
+    const bool edge_n = TILES && ((j + 1) & (ty - 1)) == 0, edge_s = TILES && (j & (ty - 1)) == 0;
+    const bool edge_e = TILES && ((4 * xl + 4) & (tx - 1)) == 0, edge_w = TILES && ((4 * xl) & (tx - 1)) == 0;
     const T half = (T)0.5;
     const T fx = half * L.a[0].ip[0], fz = half * L.a[2].ip[0];
     const T yp = half * L.a[1].ip[j], ym = half * L.a[1].im[j];
@@ -684,7 +691,7 @@ __global__ void __launch_bounds__(64 * (row_waves<T>() + 2))
     };
     // the red cells of four (P: the parity of row + plane; red are 0, 2 if odd, 1, 3 if
     // even) from the rows about them; be, pe: the cell next to the four on the red side
-    auto red2 = [&](auto par, T (&out)[2], const T (&qq)[4], const T (&b)[4], const T (&bn)[4], const T (&bs)[4],
+    auto red2 = [&](auto par, T (&out)[2], T (&alt)[2], const T (&qq)[4], const T (&b)[4], const T (&bn)[4], const T (&bs)[4],
                     const T (&bf)[4], const T (&bk)[4], const T (&p)[4], const T (&pn)[4], const T (&ps)[4],
                     const T (&pf)[4], const T (&pk)[4], T be, T pe, T fyp, T fym) __attribute__((always_inline)) {
         constexpr int P = decltype(par)::value;
@@ -694,8 +701,12 @@ __global__ void __launch_bounds__(64 * (row_waves<T>() + 2))
             const int e = 2 * i + odd;
             const T bE = e < 3 ? b[e < 3 ? e + 1 : 3] : be, bW = e > 0 ? b[e > 0 ? e - 1 : 0] : be;
             const T pE = e < 3 ? p[e < 3 ? e + 1 : 3] : pe, pW = e > 0 ? p[e > 0 ? e - 1 : 0] : pe;
-            out[i] = update(qq[e], b[e], bE, bW, bn[e], bs[e], bf[e], bk[e], fyp, fym, pE, pW, pn[e], ps[e], pf[e], pk[e],
-                            std::true_type());
+            if constexpr (TILES)
+                out[i] = smooth_red(qq[e], b[e], {bE, bW, bn[e], bs[e], bf[e], bk[e]}, fx, fx, fyp, fym, fz, fz,
+                                    {pE, pW, pn[e], ps[e], pf[e], pk[e]}, alt[i]);
+            else
+                out[i] = update(qq[e], b[e], bE, bW, bn[e], bs[e], bf[e], bk[e], fyp, fym, pE, pW, pn[e], ps[e], pf[e],
+                                pk[e], std::true_type());
         }
     };
 
@@ -704,6 +715,7 @@ __global__ void __launch_bounds__(64 * (row_waves<T>() + 2))
     RawSides<T, TQ, TB> rs;    // plane m, then m + 1
     RowCentre<T> C[3];         // planes m - 1, m, m + 1
     T R2[2] = {(T)0, (T)0}, R1[2] = {(T)0, (T)0};  // new red values of planes m - 2, m - 1
+    T X1 = (T)0;                                   // of plane m - 1, what the lane beside takes
     T kb[2] = {(T)0, (T)0};                        // beta of plane m - 2 behind the black cells of m - 1
     T kn[2] = {(T)0, (T)0}, ks[2] = {(T)0, (T)0}, kq[2] = {(T)0, (T)0};  // of plane m - 1: beta n, s and q there
     load_c(rc, k0 - 2);
@@ -712,8 +724,8 @@ __global__ void __launch_bounds__(64 * (row_waves<T>() + 2))
     take_c(C[2], rc);
     load_c(rc, k0);
     load_s(rs, k0 - 1);
-    T* const mine = sR[0] + (r + 1) * 2 * lr + 2 * xl;
-    constexpr int kSlot = 2 * 64 * (NW + 2);
+    T* const mine = sR + (r + 1) * 2 * lr + 2 * xl;
+    const int o_n = 2 * lr + (edge_n ? 2 * kSlot : 0), o_s = -2 * lr + (edge_s ? 2 * kSlot : 0);
     constexpr int kUnroll = sizeof(T) == 4 ? 4 : 2;  // steps per turn of the loop (registers)
 
     auto step = [&](auto par, int m, int sl) __attribute__((always_inline)) {
@@ -742,22 +754,26 @@ __global__ void __launch_bounds__(64 * (row_waves<T>() + 2))
             if (!dots.init) widen(dq, load4(dots.qv + ob, 0));
         }
         __builtin_amdgcn_sched_barrier(0);
-        T R0[2];
+        T R0[2], A0[2];
         {
             const T be = __shfl(C0.b[P ? 3 : 0], P ? left : right, 64);
             const T pe = FIRST ? (T)0 : __shfl(C0.p[P ? 3 : 0], P ? left : right, 64);
-            red2(par, R0, s_q, C0.b, s_bn, s_bs, Cp.b, Cm.b, C0.p, s_pn, s_ps, Cp.p, Cm.p, be, pe, yp, ym);
+            red2(par, R0, A0, s_q, C0.b, s_bn, s_bs, Cp.b, Cm.b, C0.p, s_pn, s_ps, Cp.p, Cm.p, be, pe, yp, ym);
         }
         __syncthreads();  // plane m - 1 is in LDS, and plane m - 2's readers are done
         if (put) {
             mine[sl * kSlot] = R0[0];
             mine[sl * kSlot + 1] = R0[1];
+            if (edge_n || edge_s) {
+                mine[(2 + sl) * kSlot] = A0[0];
+                mine[(2 + sl) * kSlot + 1] = A0[1];
+            }
         }
         if (black && !ring) {
             // black cells of plane m - 1 at o_red + {0, 2} (the red positions of plane m)
             const T* at = mine + (sl ^ 1) * kSlot;
             const T be = __shfl(Cm.b[P ? 3 : 0], P ? left : right, 64);
-            const T re = __shfl(R1[P ? 1 : 0], P ? left : right, 64);
+            const T re = __shfl(X1, P ? left : right, 64);
             T vb[2];
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
@@ -766,7 +782,7 @@ __global__ void __launch_bounds__(64 * (row_waves<T>() + 2))
                 // its red neighbours along x: R1 holds the cells at o_blk + {0, 2}
                 const T rE = P ? R1[i] : (i == 0 ? R1[1] : re), rW = P ? (i == 0 ? re : R1[0]) : R1[i];
                 const T self = FIRST ? (T)0 : Cm.p[e];  // a wall's ghost: the cell before the sweep
-                const T rn = wall_n ? self : at[2 * lr + i], rs = wall_s ? self : at[i - 2 * lr];
+                const T rn = wall_n ? self : at[o_n + i], rs = wall_s ? self : at[o_s + i];
                 vb[i] = update(kq[i], Cm.b[e], bE, bW, kn[i], ks[i], C0.b[e], kb[i], yp, ym, rE, rW, rn, rs, R0[i],
                                R2[i], std::false_type());
             }
@@ -796,6 +812,8 @@ __global__ void __launch_bounds__(64 * (row_waves<T>() + 2))
             kb[i] = Cm.b[e], kn[i] = s_bn[e], ks[i] = s_bs[e], kq[i] = s_q[e];
             R2[i] = R1[i], R1[i] = R0[i];
         }
+        X1 = R0[P ? 0 : 1];  // (the next step takes the other side)
+        if (P ? edge_w : edge_e) X1 = A0[P ? 0 : 1];
     };
     auto march = [&](auto p0) {  // p0: the parity of row + (k0 - 1)
         constexpr int A = decltype(p0)::value;
@@ -864,14 +882,19 @@ bool row_supported(const LevelDev<T>& L)
            (uint64_t)L.nx * L.ny < ((uint64_t)1 << 28);
 }
 
-template <class T, class TQ, class TB, bool FIRST, bool DOTS>
+struct SweepCfg {
+    int tx, ty, nt;
+};
+
+template <class T, class TQ, class TB, bool FIRST, bool DOTS, bool TILES>
 static int launch_row_form(const LevelDev<T>& L, const TB* beta, const TQ* q, const T* pin, T* pout, const int* done,
-                           const SweepDots& dots, unsigned* nblocks_out, void* stream, const KernelEvents* kev)
+                           const SweepDots& dots, unsigned* nblocks_out, void* stream, const KernelEvents* kev,
+                           const SweepCfg& c)
 {
     // resident workgroups per CU and CU count, queried once (threads may race
     // to fill it; they store the same value)
     static std::atomic<int> occ{-1};
-    auto k = k_row_sweep<T, TQ, TB, FIRST, DOTS>;
+    auto k = k_row_sweep<T, TQ, TB, FIRST, DOTS, TILES>;
     int o = occ.load(std::memory_order_acquire);
     if (o < 0) {
         int dev = 0, ncu = 0, nb = 0;
@@ -895,33 +918,14 @@ static int launch_row_form(const LevelDev<T>& L, const TB* beta, const TQ* q, co
     const dim3 blk(64 * (row_waves<T>() + 2));
     if (kev)
         hipExtLaunchKernelGGL(k, dim3(nblocks), blk, 0, (hipStream_t)stream, kev->start, kev->stop, 0, L, beta, q, pin,
-                              pout, kc, lr, rw, ntiles, done, dots);
+                              pout, kc, lr, rw, ntiles, c.tx, c.ty, done, dots);
     else
-        hipLaunchKernelGGL(k, dim3(nblocks), blk, 0, (hipStream_t)stream, L, beta, q, pin, pout, kc, lr, rw, ntiles, done,
-                           dots);
+        hipLaunchKernelGGL(k, dim3(nblocks), blk, 0, (hipStream_t)stream, L, beta, q, pin, pout, kc, lr, rw, ntiles, c.tx,
+                           c.ty, done, dots);
     TBFG_HIP(hipGetLastError());
     if (nblocks_out) *nblocks_out = nblocks;
     return TBFG_OK;
 }
-
-template <class T, class TQ, class TB>
-int launch_row_sweep(const LevelDev<T>& L, const TB* beta, const TQ* q, const T* pin, T* pout, bool first,
-                     const int* done, void* stream, const SweepDots* dots, unsigned* nblocks_out,
-                     const KernelEvents* kev)
-{
-    if (!row_supported(L) || (dots && first)) {
-        set_error("launch_row_sweep: level %dx%dx%d not supported", L.nx, L.ny, L.nz);
-        return TBFG_EINVAL;
-    }
-    const SweepDots none{};
-    if (dots) return launch_row_form<T, TQ, TB, false, true>(L, beta, q, pin, pout, done, *dots, nblocks_out, stream, kev);
-    return first ? launch_row_form<T, TQ, TB, true, false>(L, beta, q, pin, pout, done, none, nblocks_out, stream, kev)
-                 : launch_row_form<T, TQ, TB, false, false>(L, beta, q, pin, pout, done, none, nblocks_out, stream, kev);
-}
-
-struct SweepCfg {
-    int tx, ty, nt;
-};
 
 // tile shapes with an instantiated kernel, in order of preference: in FP32
 // the plain sweep runs fastest on 32x16 tiles (a smaller ring per cell), the
@@ -976,6 +980,29 @@ bool sweep_named(const LevelDev<T>& L, bool plain)
     SweepCfg c;
     bool tuned = false;
     return pick_shape(L, c, plain, &tuned) && tuned;
+}
+
+template <class T, class TQ, class TB>
+int launch_row_sweep(const LevelDev<T>& L, const TB* beta, const TQ* q, const T* pin, T* pout, bool first, bool tiles,
+                     const int* done, void* stream, const SweepDots* dots, unsigned* nblocks_out,
+                     const KernelEvents* kev)
+{
+    SweepCfg c{0, 0, 0};
+    if (!row_supported(L) || (dots && first) || (tiles && (dots || !pick_shape(L, c, !first)))) {
+        set_error("launch_row_sweep: level %dx%dx%d not supported", L.nx, L.ny, L.nz);
+        return TBFG_EINVAL;
+    }
+    const SweepDots none{};
+    auto go = [&](auto f, auto d, auto t) {
+        return launch_row_form<T, TQ, TB, decltype(f)::value, decltype(d)::value, decltype(t)::value>(
+            L, beta, q, pin, pout, done, dots ? *dots : none, nblocks_out, stream, kev, c);
+    };
+    const std::true_type yes;
+    const std::false_type no;
+    if (first) return go(yes, no, no);  // (from zero: no z term, one rounding)
+    if constexpr (sizeof(T) == 4)
+        if (tiles) return go(no, no, yes);
+    return dots ? go(no, yes, no) : go(no, no, no);
 }
 
 // prefetch distance in plane steps: 4 in FP32 on long chunks; 2 in FP64, with
@@ -1086,9 +1113,12 @@ int launch_sweep(const LevelDev<T>& L, const TB* beta, const TQ* q, const T* pin
 
 template bool row_supported<float>(const LevelDev<float>&);
 template bool row_supported<double>(const LevelDev<double>&);
-template int launch_row_sweep<float, float, float>(const LevelDev<float>&, const float*, const float*, const float*, float*, bool,
+template int launch_row_sweep<float, float, float>(const LevelDev<float>&, const float*, const float*, const float*, float*, bool, bool,
                                              const int*, void*, const SweepDots*, unsigned*, const KernelEvents*);
-template int launch_row_sweep<double, double, double>(const LevelDev<double>&, const double*, const double*, const double*, double*, bool,
+template int launch_row_sweep<float, bf16s, bf16s>(const LevelDev<float>&, const bf16s*, const bf16s*, const float*, float*,
+                                                   bool, bool, const int*, void*, const SweepDots*, unsigned*,
+                                                   const KernelEvents*);
+template int launch_row_sweep<double, double, double>(const LevelDev<double>&, const double*, const double*, const double*, double*, bool, bool,
                                              const int*, void*, const SweepDots*, unsigned*, const KernelEvents*);
 template bool point_supported<float>(const LevelDev<float>&);
 template bool point_supported<double>(const LevelDev<double>&);

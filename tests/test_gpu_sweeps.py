@@ -74,6 +74,19 @@ def test_row_sweep_matches_staged_tiles(torch_gpu, monkeypatch, precision, bound
     assert rel(a, b) < bound
 
 
+@pytest.mark.parametrize("n", [(64, 48, 64), (32, 16, 16), (256, 32, 32), (96, 48, 96)])
+def test_row_sweep_rounds_as_tiles(torch_gpu, monkeypatch, n):
+    """Under bf16 storage the rows give the staged kernel's bits: its preferred shape
+    named (32x16 tiles for the plain sweep), against the rows that run unasked."""
+    print("case rows round as tiles", n, flush=True)
+    c = case(torch_gpu, n)
+    monkeypatch.setenv("TBFG_SWEEP_MIN_CELLS", "0")
+    a = apply(torch_gpu, *c, precision="mixed-bf16")
+    monkeypatch.setenv("TBFG_SWEEP_SHAPE", "32x16x256")
+    b = apply(torch_gpu, *c, precision="mixed-bf16")
+    assert np.array_equal(a, b)
+
+
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 @pytest.mark.parametrize("n,min_cells", [((72, 40, 56), 0), ((72, 40, 56), 10 ** 12), ((36, 12, 20), 0), ((18, 14, 10), 0)])
 def test_dots_in_row_and_point_sweeps(torch_gpu, monkeypatch, n, min_cells, precision):
