@@ -1004,26 +1004,33 @@ struct TailView<T, true> {
     lds_ptr<T> q;
     lds_ptr<const T> beta;
     uint32_t dm_nx, dm_ny, dm_hx, dm_hy;
+    // (the plan is in LDS: its values are made scalar, or they would fill vector registers)
+    static __device__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+    template <class E>
+    static __device__ lds_ptr<E> uni(E* v)
+    {
+        return (lds_ptr<E>)__builtin_amdgcn_readfirstlane((int)(uint32_t)(size_t)(lds_ptr<E>)v);
+    }
     __device__ explicit TailView(const TailLevel<T>& lv)
     {
-        dm_nx = lv.dm_nx;
-        dm_ny = lv.dm_ny;
-        dm_hx = lv.dm_hx;
-        dm_hy = lv.dm_hy;
-        geo.nx = lv.geo.nx;
-        geo.ny = lv.geo.ny;
-        geo.nz = lv.geo.nz;
+        dm_nx = uni(lv.dm_nx);
+        dm_ny = uni(lv.dm_ny);
+        dm_hx = uni(lv.dm_hx);
+        dm_hy = uni(lv.dm_hy);
+        geo.nx = uni(lv.geo.nx);
+        geo.ny = uni(lv.geo.ny);
+        geo.nz = uni(lv.geo.nz);
         for (int a = 0; a < 3; ++a) {
-            geo.a[a].ip = (lds_ptr<const T>)lv.geo.a[a].ip;
-            geo.a[a].im = (lds_ptr<const T>)lv.geo.a[a].im;
-            geo.a[a].rlo = (lds_ptr<const T>)lv.geo.a[a].rlo;
-            geo.a[a].rhi = (lds_ptr<const T>)lv.geo.a[a].rhi;
-            geo.a[a].plo = (lds_ptr<const T>)lv.geo.a[a].plo;
-            geo.a[a].phi = (lds_ptr<const T>)lv.geo.a[a].phi;
+            geo.a[a].ip = uni(lv.geo.a[a].ip);
+            geo.a[a].im = uni(lv.geo.a[a].im);
+            geo.a[a].rlo = uni(lv.geo.a[a].rlo);
+            geo.a[a].rhi = uni(lv.geo.a[a].rhi);
+            geo.a[a].plo = uni(lv.geo.a[a].plo);
+            geo.a[a].phi = uni(lv.geo.a[a].phi);
         }
-        p = (lds_ptr<T>)lv.p;
-        q = (lds_ptr<T>)lv.q;
-        beta = (lds_ptr<const T>)lv.beta;
+        p = uni(lv.p);
+        q = uni(lv.q);
+        beta = uni(lv.beta);
     }
 };
 
@@ -1100,15 +1107,271 @@ __device__ void tail_prolong(const TailLevel<T>& lvl, const TailLevel<T>& lcl)
     __syncthreads();
 }
 
-// x = G q on the bottom level: S threads per row (S a power of two, at most
-// 64, as many as the workgroup allows) each sum every S-th product of the row,
-// then a butterfly over the S lanes; a row's loads are coalesced and in flight
-// together instead of one dependent load per column.
+// ---- levels of the LDS-resident tail smoothed from registers.  A thread owns U pairs of
+// x neighbours (one red and one black cell each) and computes their coefficients,
+// reciprocal diagonals and neighbour addresses once per visit: a half sweep is then five
+// LDS reads, ten multiply-adds and a write per cell, where recomputing them cost 20 reads,
+// the index arithmetic and a division -- and one compute unit's instruction rate bounds
+// the launch.  The residual comes from the same registers.  The arithmetic, order
+// included, is smooth_cell's, resid_restrict_plane's and prolong_cell's.  One application,
+// cells of the first level: 16x12x16 in FP32 32 -> 23 us, 18x10x14 67 -> 26 (36 -> 13 of it
+// the bottom of 315 cells), 1024 21 -> 17; 16^3 in FP64 40 -> 36.  What is left is code that
+// runs once from a cold instruction cache (the first of four equal half sweeps takes three
+// times the others') and the latency of the loads at the start.
+template <class T, int U>
+struct TailPairs {
+    struct Cell {
+        T a[6], rden;  // towards E W N S F B
+        T v;           // p of the cell
+    };
+    Cell cell[U][2];  // red, black
+    // two 16-bit indices to a register: the pair's first cell and its place along x; those
+    // of the pairs beside it; the x neighbours outside it; its place along y and z
+    unsigned ci[U], ns[U], fb[U], xo[U], jk[U];
+    bool odd[U], wn[U], ws[U], has[U];  // whether red is the pair's second cell; walls
+    static __device__ __forceinline__ unsigned two(int lo, int hi) { return (unsigned)lo | ((unsigned)hi << 16); }
+    static __device__ __forceinline__ int lo(unsigned x) { return (int)(x & 0xffffu); }
+    static __device__ __forceinline__ int hi(unsigned x) { return (int)(x >> 16); }
+    __device__ __forceinline__ int at(int u, int col) const { return lo(ci[u]) + ((int)odd[u] ^ col); }
+    __device__ __forceinline__ T quotient(const Cell& x, T num) const
+    {
+#pragma clang fp contract(off)
+        if constexpr (sizeof(T) == 4) return num * x.rden;
+        // the last step of a division with a correctly rounded reciprocal
+        const T den = x.a[0] + x.a[1] + x.a[2] + x.a[3] + x.a[4] + x.a[5], y = num * x.rden;
+        return __builtin_elementwise_fma(__builtin_elementwise_fma(-den, y, num), x.rden, y);
+    }
+
+    // where the pair and its neighbours are, and its coefficients
+    __device__ __forceinline__ void load(const TailView<T, true>& lv)
+    {
+#pragma clang fp contract(off)
+        const auto& L = lv.geo;
+        const int nx = L.nx, ny = L.ny, nz = L.nz, ncx = nx >> 1;
+        const int np = ncx * ny * nz;
+        int id = (int)threadIdx.x;
+        asm volatile("" : "+v"(id));  // the addresses are not to be hoisted out of a loop of visits (registers)
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int t0 = id + u * 1024, t = min(t0, np - 1);
+            has[u] = t0 < np;
+            const int r = mdiv(t, ncx, lv.dm_hx), h = t - r * ncx, kk = mdiv(r, ny, lv.dm_ny), jj = r - kk * ny;
+            const int i0 = 2 * h;
+            auto row = [&](int y, int z) { return nx * (y + ny * z) + i0; };
+            wn[u] = jj == ny - 1;
+            ws[u] = jj == 0;
+            const int c = row(jj, kk), n = row(min(jj + 1, ny - 1), kk), s = row(max(jj - 1, 0), kk);
+            const int f = row(jj, wrap_up(kk, nz)), b = row(jj, wrap_dn(kk, nz));
+            odd[u] = ((RED + jj + kk + 1) & 1) != 0;
+            const int xm = c - i0 + wrap_dn(i0, nx), xp = c - i0 + wrap_up(i0 + 1, nx);
+            ci[u] = two(c, h), ns[u] = two(n, s), fb[u] = two(f, b), jk[u] = two(jj, kk);
+            xo[u] = odd[u] ? two(xp, xm) : two(xm, xp);
+            const T half = (T)0.5;
+            const T fy = half * L.a[1].ip[jj], gy = half * L.a[1].im[jj];
+            const T fz = half * L.a[2].ip[kk], gz = half * L.a[2].im[kk];
+#pragma unroll
+            for (int col = 0; col < 2; ++col) {
+                const int o = (int)odd[u] ^ col;
+                Cell& x = cell[u][col];
+                const T bc = lv.beta[c + o], bp = lv.beta[c + (o ^ 1)], bo = lv.beta[o ? xp : xm];
+                const T bE = o ? bo : bp, bW = o ? bp : bo;
+                const T fx = half * L.a[0].ip[i0 + o], gx = half * L.a[0].im[i0 + o];
+                const T sE = bE + bc, sW = bc + bW, sN = lv.beta[n + o] + bc, sS = bc + lv.beta[s + o];
+                const T sF = lv.beta[f + o] + bc, sB = bc + lv.beta[b + o];
+                x.a[0] = sE * fx, x.a[1] = sW * gx, x.a[2] = sN * fy, x.a[3] = sS * gy, x.a[4] = sF * fz, x.a[5] = sB * gz;
+                if constexpr (sizeof(T) == 4) {  // (smooth_sums' sum of the coefficients)
+                    T den = __builtin_elementwise_fma(sE, fx, x.a[1]);
+                    den = __builtin_elementwise_fma(sN, fy, den);
+                    den = __builtin_elementwise_fma(sS, gy, den);
+                    den = __builtin_elementwise_fma(sF, fz, den);
+                    x.rden = __builtin_amdgcn_rcpf(__builtin_elementwise_fma(sB, gz, den));
+                } else {
+                    x.rden = (T)1 / (x.a[0] + x.a[1] + x.a[2] + x.a[3] + x.a[4] + x.a[5]);
+                }
+                asm volatile("" : "+v"(x.rden));  // (not put off to the first sweep, with all it is made from)
+            }
+        }
+    }
+    // p beside a cell (own: of the cell itself, a wall's ghost)
+    __device__ __forceinline__ Around<T> around(lds_ptr<const T> p, int u, int col) const
+    {
+        const int o = (int)odd[u] ^ col;
+        const T own = cell[u][col].v, par = cell[u][col ^ 1].v, out = p[col ? hi(xo[u]) : lo(xo[u])];
+        const T pn = p[lo(ns[u]) + o], ps = p[hi(ns[u]) + o];
+        return {o ? out : par, o ? par : out, wn[u] ? own : pn, ws[u] ? own : ps, p[lo(fb[u]) + o], p[hi(fb[u]) + o]};
+    }
+    __device__ __forceinline__ void half_sweep(const TailView<T, true>& lv, int col, bool zero)
+    {
+#pragma clang fp contract(off)
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            Cell& x = cell[u][col];
+            const int c = at(u, col);
+            T num = -lv.q[c];
+            if (!zero) {
+                const Around<T> p = around(lv.p, u, col);
+                num = __builtin_elementwise_fma(x.a[0], p.E, x.a[1] * p.W) + num;
+                num = num + __builtin_elementwise_fma(x.a[2], p.N, x.a[3] * p.S);
+                num = num + __builtin_elementwise_fma(x.a[4], p.F, x.a[5] * p.B);
+            }
+            x.v = quotient(x, num);
+            if (has[u]) lv.p[c] = x.v;
+        }
+        __syncthreads();
+    }
+    // the residual into rs and from there the coarse level's right-hand side: a plane's
+    // four children in order, then both planes
+    __device__ __forceinline__ void restrict_residual(const TailView<T, true>& lv, lds_ptr<T> rs, lds_ptr<T> qc) const
+    {
+#pragma clang fp contract(off)
+        const auto& L = lv.geo;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+#pragma unroll
+            for (int col = 0; col < 2; ++col) {
+                const Cell& x = cell[u][col];
+                const int c = at(u, col);
+                const Around<T> p = around(lv.p, u, col);
+                T ap = __builtin_elementwise_fma(x.a[0], p.E - x.v, -(x.a[1] * (x.v - p.W)));
+                ap = __builtin_elementwise_fma(x.a[2], p.N - x.v, ap);
+                ap = __builtin_elementwise_fma(-x.a[3], x.v - p.S, ap);
+                ap = __builtin_elementwise_fma(x.a[4], p.F - x.v, ap);
+                ap = __builtin_elementwise_fma(-x.a[5], x.v - p.B, ap);
+                const T res = lv.q[c] - ap;
+                if (has[u]) rs[c] = res;
+            }
+        }
+        __syncthreads();
+        const int nx = L.nx, ny = L.ny, ncx = nx >> 1, ncy = ny >> 1, cells = ncx * ncy * (L.nz >> 1);
+        for (int t = threadIdx.x; t < cells; t += 1024) {
+            const int r = mdiv(t, ncx, lv.dm_hx), X = t - r * ncx, Z = mdiv(r, ncy, lv.dm_hy), Y = r - Z * ncy;
+            const T xl = L.a[0].rlo[X], xh = L.a[0].rhi[X], yl = L.a[1].rlo[Y], yh = L.a[1].rhi[Y];
+            const lds_ptr<const T> at = rs + 2 * (X + nx * (Y + ny * Z));
+            T part[2];
+#pragma unroll
+            for (int dk = 0; dk < 2; ++dk) {
+                const T wz = dk ? L.a[2].rhi[Z] : L.a[2].rlo[Z];
+                const int o = dk * nx * ny;
+                T acc = __builtin_elementwise_fma((xl * yl) * wz, at[o], (T)0);
+                acc = __builtin_elementwise_fma((xh * yl) * wz, at[o + 1], acc);
+                acc = __builtin_elementwise_fma((xl * yh) * wz, at[o + nx], acc);
+                part[dk] = __builtin_elementwise_fma((xh * yh) * wz, at[o + nx + 1], acc);
+            }
+            qc[t] = part[0] + part[1];
+        }
+        __syncthreads();
+    }
+    // p += P pc
+    __device__ __forceinline__ void prolong(const TailView<T, true>& lv, const TailView<T, true>& lc)
+    {
+#pragma clang fp contract(off)
+        const auto& L = lv.geo;
+        const int ncx = lc.geo.nx, ncy = lc.geo.ny, ncz = lc.geo.nz;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int h = hi(ci[u]), i0 = 2 * h, jj = lo(jk[u]), kk = hi(jk[u]);
+            const int hm = wrap_dn(h, ncx), hp = wrap_up(h, ncx);
+            const int jl = max(((jj + 1) >> 1) - 1, 0), jh = min((jj + 1) >> 1, ncy - 1);
+            const int ka = (kk + 1) >> 1, kl = ka > 0 ? ka - 1 : ncz - 1, kh = ka < ncz ? ka : 0;
+            const T wyl = L.a[1].plo[jj], wyh = L.a[1].phi[jj], wzl = L.a[2].plo[kk], wzh = L.a[2].phi[kk];
+            const T xl0 = L.a[0].plo[i0], xh0 = L.a[0].phi[i0], xl1 = L.a[0].plo[i0 + 1], xh1 = L.a[0].phi[i0 + 1];
+            T v[2][2][2];  // plane, row, cell of the pair
+#pragma unroll
+            for (int a = 0; a < 2; ++a)
+#pragma unroll
+                for (int d = 0; d < 2; ++d) {
+                    const int r = ncx * ((d ? jh : jl) + ncy * (a ? kh : kl));
+                    const T pm = lc.p[r + hm], p0 = lc.p[r + h], pp = lc.p[r + hp];
+                    v[a][d][0] = __builtin_elementwise_fma(xl0, pm, xh0 * p0);
+                    v[a][d][1] = __builtin_elementwise_fma(xl1, p0, xh1 * pp);
+                }
+            T add[2];
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const T lo = __builtin_elementwise_fma(wyl, v[0][0][e], wyh * v[0][1][e]);
+                const T hi = __builtin_elementwise_fma(wyl, v[1][0][e], wyh * v[1][1][e]);
+                add[e] = __builtin_elementwise_fma(wzl, lo, wzh * hi);
+            }
+#pragma unroll
+            for (int col = 0; col < 2; ++col) {
+                const int o = (int)odd[u] ^ col;
+                const T x = lv.p[lo(ci[u]) + o] + (o ? add[1] : add[0]);
+                cell[u][col].v = x;
+                if (has[u]) lv.p[lo(ci[u]) + o] = x;
+            }
+        }
+        __syncthreads();
+    }
+};
+
+// one level's part of a V-cycle after load(): from zero and the residual restricted on the
+// way down, the correction added first on the way up
+template <class T, int U>
+__device__ __forceinline__ void tail_visit(TailPairs<T, U>& t, const TailView<T, true>& lv, const TailView<T, true>& lc,
+                                           lds_ptr<T> rs, bool up, int sweeps, bool reverse)
+{
+    if (up) {
+        t.prolong(lv, lc);
+    } else {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            t.cell[u][0].v = t.cell[u][1].v = (T)0;
+            if (sweeps == 0 && t.has[u]) lv.p[t.at(u, 0)] = lv.p[t.at(u, 1)] = (T)0;
+        }
+        if (sweeps == 0) __syncthreads();
+    }
+#pragma unroll 1
+    for (int h = 0; h < 2 * sweeps; ++h) {
+        if (((h & 1) != 0) != (up && reverse))
+            t.half_sweep(lv, 1, false);
+        else
+            t.half_sweep(lv, 0, !up && h == 0);
+    }
+    if (!up) t.restrict_residual(lv, rs, lc.q);
+}
+
+// x = G q on a bottom level of more than 64 cells: a wavefront takes four rows at once,
+// its lanes along them, 16 loads in flight; the four sums share the butterfly's steps
+// (each lane goes on with half of the rows).  The phase is one compute unit reading nb^2
+// doubles.  With two lanes per row (as many as the workgroup gives 315 rows) a load
+// instruction read from 32 rows, 36 us for 0.8 MB; this takes 13.
+template <class T, class LQ, class LP>
+__device__ __forceinline__ void tail_dense_rows(const double* __restrict__ G, LQ q, LP p, int nb)
+{
+    const int lane = (int)threadIdx.x & 63, w = (int)threadIdx.x >> 6, nw = (int)blockDim.x >> 6;
+    const bool b5 = (lane & 32) != 0, b4 = (lane & 16) != 0;
+    for (int r0 = w * 4; r0 < nb; r0 += nw * 4) {
+        double acc[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+        for (int c0 = 0; c0 < nb; c0 += 64) {
+            const int c = min(c0 + lane, nb - 1);
+            const double v = c0 + lane < nb ? (double)q[c] : 0.0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                acc[i] += ((glb_ptr<const double>)(G + (size_t)min(r0 + i, nb - 1) * nb))[c] * v;
+        }
+        const double k0 = (b5 ? acc[2] : acc[0]) + __shfl_xor(b5 ? acc[0] : acc[2], 32, 64);
+        const double k1 = (b5 ? acc[3] : acc[1]) + __shfl_xor(b5 ? acc[1] : acc[3], 32, 64);
+        double x = (b4 ? k1 : k0) + __shfl_xor(b4 ? k0 : k1, 16, 64);
+        for (int off = 8; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+        const int r = r0 + (b5 ? 2 : 0) + (b4 ? 1 : 0);
+        if ((lane & 15) == 0 && r < nb) p[r] = (T)x;
+    }
+}
+
+// x = G q on the bottom level, at most 64 cells: S threads per row (S a power of two, as
+// many as the workgroup allows) each sum every S-th product of the row, then a butterfly
+// over the S lanes; a row's loads are coalesced and in flight together.
 template <class T, bool LDS = false>
 __device__ void tail_dense(const TailPlan<T>& P, const TailLevel<T>& lvl)
 {
     const TailView<T, LDS> lv(lvl);
     const int nb = lv.geo.nx * lv.geo.ny * lv.geo.nz;
+    if (nb > 64) {
+        tail_dense_rows<T>(P.G, lv.q, lv.p, nb);
+        __syncthreads();
+        return;
+    }
     int S = 1;
     while (S < 64 && nb * (S * 2) <= (int)blockDim.x) S *= 2;
     const int rows = (int)blockDim.x / S;
@@ -1575,6 +1838,40 @@ __device__ void tail_vcycle(const TailPlan<T>& P, int top, int bot, bool reset_t
     }
 }
 
+// The V-cycle of the LDS-resident tail with its levels smoothed from registers: U pairs
+// per thread on the first level, one on those below it (an eighth of its cells or fewer).
+// Each part's code stands once, in loops over the levels: the launch runs most of it a
+// few times on one compute unit, and fetching it counts.  In FP32 the first level's
+// coefficients stay in registers from the way down to the way up.
+template <class T, int U>
+__device__ void tail_vcycle_pairs(const TailPlan<T>& P, int bot, lds_ptr<T> rs)
+{
+    constexpr bool KEEP = sizeof(T) == 4;
+    const bool rev = P.rev_post != 0;
+    const TailView<T, true> l0(P.lv[0]), l1(P.lv[bot > 0 ? 1 : 0]);
+    TailPairs<T, U> t;
+#pragma unroll 1
+    for (int dir = 0; dir < 2; ++dir) {
+        if (bot > 0) {
+            if (!KEEP || dir == 0) t.load(l0);
+            tail_visit(t, l0, l1, rs, dir != 0, dir ? P.n_post : P.n_pre, rev);
+        }
+        if (dir) break;
+        const int mid = bot - 1;  // levels 1 .. bot - 1
+#pragma unroll 1
+        for (int v = 0; v < 2 * mid || v == 0; ++v) {
+            if (v == max(mid, 0)) tail_dense<T, true>(P, P.lv[bot]);
+            if (mid <= 0) break;
+            const bool up = v >= mid;
+            const int l = up ? 2 * mid - v : v + 1;
+            const TailView<T, true> lv(P.lv[l]), lc(P.lv[l + 1]);
+            TailPairs<T, 1> s;
+            s.load(lv);
+            tail_visit(s, lv, lc, rs, up, up ? P.n_post : P.n_pre, rev);
+        }
+    }
+}
+
 template <class T>
 __global__ void __launch_bounds__(1024) k_tail(const TailPlan<T>* __restrict__ plan, const int* done)
 {
@@ -1588,12 +1885,37 @@ __global__ void __launch_bounds__(1024) k_tail(const TailPlan<T>* __restrict__ p
 // costs LDS latency instead of an L2 round trip.  beta, the tables and q of the
 // first level come in at the start, p of the first level goes back to HBM at
 // the end (the next level up prolongs from it).
-template <class T>
+constexpr int kTouch = 4096;  // doubles per prefetching workgroup
+// loads issued for their lines' sake: keep() waits for them
+struct Touch {
+    double v[kTouch / 1024];
+    __device__ __forceinline__ Touch(const double* G, int first, int n)
+    {
+#pragma unroll
+        for (int u = 0; u < kTouch / 1024; ++u)
+            v[u] = ((glb_ptr<const double>)G)[min(first + u * 1024 + (int)threadIdx.x, n - 1)];
+    }
+    __device__ __forceinline__ void keep() const
+    {
+#pragma unroll
+        for (int u = 0; u < kTouch / 1024; ++u) asm volatile("" ::"v"(v[u]));
+    }
+};
+
+// U: pairs of cells per thread on the first level (0: too many, the phases loop over cells).
+template <class T, int U>
 __global__ void __launch_bounds__(1024) k_tail_lds(const TailPlan<T>* __restrict__ plan, const int* done)
 {
     extern __shared__ __align__(16) unsigned char tail_smem[];
     __shared__ TailPlan<T> Ps;
     if (done && *done) return;
+    if (blockIdx.x > 0) {
+        // the bottom operator into this chiplet's L2 while the first workgroup smooths: one
+        // compute unit reads it from there three times as fast (every eighth workgroup
+        // lands on the first one's chiplet; the others have nothing to do)
+        if ((blockIdx.x & 7u) == 0) Touch(plan->G, (blockIdx.x / 8 - 1) * kTouch, plan->nb * plan->nb).keep();
+        return;
+    }
     {
         static_assert(sizeof(TailPlan<T>) % 4 == 0, "plan copied as 32-bit words");
         const unsigned* src = reinterpret_cast<const unsigned*>(plan);
@@ -1622,19 +1944,27 @@ __global__ void __launch_bounds__(1024) k_tail_lds(const TailPlan<T>* __restrict
         lv.beta = base + lv.lds_beta;
     }
     {
-        // every thread issues the loads of up to kStage elements of the list
-        // before it stores any, so the HBM/L2 latency is paid once per round
-        // instead of once per array
-        constexpr int kStage = sizeof(T) == 4 ? 12 : 6;
+        // every thread issues its loads before it stores any, so the latency is paid once:
+        // beta and q of the first level directly (up to kBig elements of each in flight,
+        // all of them up to kTailPairCells), the rest from the list
+        constexpr int kBig = 4, kStage = 4;
         const lds_ptr<T> sm = (lds_ptr<T>)base;
-        const int total = Ps.seg_first[Ps.nseg];
-        for (int e0 = 0; e0 < total; e0 += kStage * (int)blockDim.x) {
-            T v[kStage];
+        const int n0 = Ps.seg_first[1] - Ps.seg_first[0], first = Ps.seg_first[1], total = Ps.seg_first[Ps.nseg - 1];
+        const glb_ptr<const T> b0 = (glb_ptr<const T>)Ps.seg_src[0], q0 = (glb_ptr<const T>)Ps.seg_src[Ps.nseg - 1];
+        const lds_ptr<T> sb = sm + Ps.seg_dst[0], sq = sm + Ps.seg_dst[Ps.nseg - 1];
+        const Touch g(Ps.G, 0, Ps.nb * Ps.nb);  // (of a bottom of at most 64 cells, all)
+        for (int e0 = 0, f0 = first; e0 < n0 || f0 < total; e0 += kBig * 1024, f0 += kStage * 1024) {
+            T vb[kBig], vq[kBig], v[kStage];
             int dst[kStage];
-            int sg = 0;
+#pragma unroll
+            for (int u = 0; u < kBig; ++u) {
+                const int e = e0 + u * 1024 + (int)threadIdx.x;
+                if (e < n0) vb[u] = b0[e], vq[u] = q0[e];
+            }
+            int sg = 1;
 #pragma unroll
             for (int u = 0; u < kStage; ++u) {
-                const int e = e0 + u * (int)blockDim.x + (int)threadIdx.x;
+                const int e = f0 + u * 1024 + (int)threadIdx.x;
                 dst[u] = -1;
                 if (e < total) {
                     while (e >= Ps.seg_first[sg + 1]) ++sg;  // e grows with u
@@ -1644,12 +1974,21 @@ __global__ void __launch_bounds__(1024) k_tail_lds(const TailPlan<T>* __restrict
                 }
             }
 #pragma unroll
+            for (int u = 0; u < kBig; ++u) {
+                const int e = e0 + u * 1024 + (int)threadIdx.x;
+                if (e < n0) sb[e] = vb[u], sq[e] = vq[u];
+            }
+#pragma unroll
             for (int u = 0; u < kStage; ++u)
                 if (dst[u] >= 0) sm[dst[u]] = v[u];
         }
+        g.keep();
     }
     __syncthreads();
-    tail_vcycle<T, false, true>(Ps, 0, Ps.user_last, true);
+    if constexpr (U > 0)
+        tail_vcycle_pairs<T, U>(Ps, Ps.user_last, (lds_ptr<T>)base + Ps.lds_res);
+    else
+        tail_vcycle<T, false, true>(Ps, 0, Ps.user_last, true);
     const int n0 = Ps.lv[0].geo.nx * Ps.lv[0].geo.ny * Ps.lv[0].geo.nz;
     const glb_ptr<T> gp = (glb_ptr<T>)plan->lv[0].p;
     const lds_ptr<T> p0 = (lds_ptr<T>)Ps.lv[0].p;
@@ -1963,10 +2302,12 @@ int launch_convert(size_t n, const TS* src, TD* dst, void* stream)
 }
 
 template <class T>
-int launch_tail(const TailPlan<T>* plan_dev, const int* done, size_t lds_bytes, void* stream)
+int launch_tail(const TailPlan<T>* plan_dev, size_t cells, int nb, const int* done, size_t lds_bytes, void* stream)
 {
     if (lds_bytes > 0) {
-        hipLaunchKernelGGL(k_tail_lds<T>, dim3(1), dim3(1024), lds_bytes, S(stream), plan_dev, done);
+        auto k = cells <= 2048 ? k_tail_lds<T, 1> : (cells <= (size_t)kTailPairCells ? k_tail_lds<T, 2> : k_tail_lds<T, 0>);
+        const int helpers = nb > 64 ? 8 * ((nb * nb + kTouch - 1) / kTouch) : 0;
+        hipLaunchKernelGGL(k, dim3(1 + helpers), dim3(1024), lds_bytes, S(stream), plan_dev, done);
         TBFG_HIP(hipGetLastError());
         return TBFG_OK;
     }
@@ -2012,8 +2353,8 @@ template int launch_pcg_update<float>(size_t, double*, double*, float*, const do
                                       const Reducer&, void*);
 template int launch_pcg_update<bf16s>(size_t, double*, double*, bf16s*, const double*, const double*, PcgState*,
                                       const Reducer&, void*);
-template int launch_tail<double>(const TailPlan<double>*, const int*, size_t, void*);
-template int launch_tail<float>(const TailPlan<float>*, const int*, size_t, void*);
+template int launch_tail<double>(const TailPlan<double>*, size_t, int, const int*, size_t, void*);
+template int launch_tail<float>(const TailPlan<float>*, size_t, int, const int*, size_t, void*);
 
 template <class T>
 size_t tail_lds_capacity()
@@ -2023,11 +2364,12 @@ size_t tail_lds_capacity()
     if (hipDeviceGetAttribute(&maxb, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess) return 0;
     const size_t avail = maxb > (int)(sizeof(TailPlan<T>) + 2048) ? (size_t)maxb - sizeof(TailPlan<T>) - 2048 : 0;
     if (avail == 0) return 0;
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tail_lds<T>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)avail) != hipSuccess) {
-        (void)hipGetLastError();
-        return 0;
-    }
+    for (auto k : {k_tail_lds<T, 0>, k_tail_lds<T, 1>, k_tail_lds<T, 2>})
+        if (hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)avail) !=
+            hipSuccess) {
+            (void)hipGetLastError();
+            return 0;
+        }
     return avail;
 }
 template size_t tail_lds_capacity<float>();

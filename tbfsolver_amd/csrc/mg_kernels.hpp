@@ -112,6 +112,9 @@ struct TailLevel {
     uint32_t dm_nx, dm_ny, dm_hx, dm_hy;
 };
 
+// largest first level that the LDS-resident tail smooths from registers (two pairs of
+// cells per thread: more do not fit them)
+constexpr int kTailPairCells = 4096;
 constexpr int kTailSegs = 2 * kMaxTail + 1;
 
 template <class T>
@@ -126,6 +129,8 @@ struct TailPlan {
     T *cx, *cr, *cd, *cad;  // inner PCG vectors (coarsest user level)
     const T* cvol;     // cell volumes of that level
     const double* G;   // bottom dense operator, row-major: x = G q
+    int nb;            // its rows
+    int lds_res;       // residual scratch of the LDS-resident tail (elements from the base)
     PcgState* st;      // receives the coarse-solve diagnostics (may be null)
     TailLevel<T> lv[kMaxTail];
     // the arrays the LDS-resident tail stages from HBM (beta and the tables of

@@ -122,8 +122,9 @@ template <class T>
 int launch_prolong_add(const LevelDev<T>& L, const T* pc, T* p, const int* done, void* stream);
 template <class TS, class TD>
 int launch_convert(size_t n, const TS* src, TD* dst, void* stream);
+// (cells: of the first tail level; nb: of the bottom)
 template <class T>
-int launch_tail(const TailPlan<T>* plan_dev, const int* done, size_t lds_bytes, void* stream);
+int launch_tail(const TailPlan<T>* plan_dev, size_t cells, int nb, const int* done, size_t lds_bytes, void* stream);
 // dynamic LDS the LDS-resident tail kernel may use on the current device (0: none)
 template <class T>
 size_t tail_lds_capacity();

@@ -184,6 +184,7 @@ static int build_plan(tbfg_pcg* h)
     P.cad = h->cad.as<T>();
     P.cvol = h->cvol.as<T>();
     P.G = h->G.as<double>();
+    P.nb = (int)h->hl[h->ntot - 1].cells();
     P.st = h->st.as<PcgState>();
     // LDS layout of the LDS-resident tail: per level p, q, beta, then its
     // table block (LevelTables::build), padded to 4 entries
@@ -230,6 +231,9 @@ static int build_plan(tbfg_pcg* h)
     }
     add_seg(P.lv[0].q, P.lv[0].lds_q, h->hl[h->t0].cells());
     P.seg_first[P.nseg] = first;
+    // the residual of a level on its way to the next
+    P.lds_res = (int)(lds / sizeof(T));
+    if (h->hl[h->t0].cells() <= (size_t)kTailPairCells) lds += h->hl[h->t0].cells() * sizeof(T);
     // the LDS-resident tail when its levels fit (the inner coarsest-level CG
     // keeps its vectors in HBM and uses the other form)
     h->tail_lds = 0;
@@ -594,7 +598,7 @@ static int inner_vcycle(tbfg_pcg* h, const int* done, void* stream)
         }
         TBFG_TRY(launch_resid_restrict<T, T>(L, b, q, p, h->q[l + 1].as<T>(), done, stream));
     }
-    TBFG_TRY(launch_tail<T>(h->plan.as<TailPlan<T>>(), done, h->tail_lds, stream));
+    TBFG_TRY(launch_tail<T>(h->plan.as<TailPlan<T>>(), h->hl[h->t0].cells(), (int)h->hl[h->ntot - 1].cells(), done, h->tail_lds, stream));
     for (int l = t0 - 1; l >= h->kin; --l) {
         const LevelDev<T>& L = geo<T>(h, l);
         const T* b = h->beta[l].as<T>();
@@ -721,7 +725,7 @@ static int vcycle(tbfg_pcg* h, const T0* r0, T** z, const T0* beta0, const int* 
                                         h->G.as<double>(), h->q[t0].as<double>(), h->p[t0].as<double>(),
                                         h->st.as<PcgState>(), done, stream));
         } else {
-            TBFG_TRY(launch_tail<T>(h->plan.as<TailPlan<T>>(), done, h->tail_lds, stream));
+            TBFG_TRY(launch_tail<T>(h->plan.as<TailPlan<T>>(), h->hl[h->t0].cells(), (int)h->hl[h->ntot - 1].cells(), done, h->tail_lds, stream));
         }
         for (int l = t0 - 1; l >= 0; --l) {
             const T* pc = (l + 1 < t0) ? cur[l + 1] : h->p[l + 1].as<T>();
