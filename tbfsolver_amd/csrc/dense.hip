@@ -336,13 +336,12 @@ __global__ void __launch_bounds__(256)
 // its residual over that of the right-hand side projected onto the range of A
 // (q - (sum V q) / (n V)), counted as one inner iteration; a zero right-hand side
 // counts no call.  One workgroup, at most two cells per thread.
-__global__ void __launch_bounds__(1024)
-    k_dense_check(LevelDev<double> L, const double* __restrict__ beta, const double* __restrict__ vol,
-                  const double* __restrict__ q, const double* __restrict__ x, PcgState* st, const int* done)
+__device__ __forceinline__ void dense_check(const DenseCheck& a, PcgState* st)
 {
     __shared__ double lds[32 * 2];
     __shared__ double s_shift;
-    if (done && *done) return;
+    const LevelDev<double>& L = a.L;
+    const double *beta = a.beta, *vol = a.vol, *q = a.q, *x = a.x;
     const int n = L.nx * L.ny * L.nz;
     double v[2], qc[2], ax[2], sum[1] = {0.0};
 #pragma unroll
@@ -380,6 +379,24 @@ __global__ void __launch_bounds__(1024)
         if (rel > st->coarse_res_max) st->coarse_res_max = rel;
     }
 }
+__global__ void __launch_bounds__(1024) k_dense_check(DenseCheck a, PcgState* st, const int* done)
+{
+    if (done && *done) return;
+    dense_check(a, st);
+}
+
+// k_fin_dots with the check beside it, in a second workgroup: nothing reads the diagnostics
+// before the solve ends, and as a launch of its own the check cost 7.3 us of the 186 that an
+// iteration takes at 96x64x96.
+__global__ void __launch_bounds__(1024)
+    k_fin_dots_check(unsigned nblocks, size_t ncell, int init, PcgState* st, Reducer red, int32_t* host_done,
+                     DenseCheck a)
+{
+    if (blockIdx.x == 0)
+        fin_dots(nblocks, ncell, init, st, red, host_done);
+    else if (!st->done)
+        dense_check(a, st);
+}
 
 int padded(int n) { return (n + kTile - 1) / kTile * kTile; }
 
@@ -415,17 +432,25 @@ int launch_dense_setup(const LevelDev<double>& L, const T* beta, const double* v
     TBFG_HIP(hipGetLastError());
     return TBFG_OK;
 }
-int launch_dense_solve(const LevelDev<double>& L, const double* beta, const double* vol, const double* G,
-                       const double* q, double* x, PcgState* st, const int* done, void* stream)
+int launch_dense_solve(const DenseCheck& a, const double* G, double* x, bool check, PcgState* st, const int* done,
+                       void* stream)
 {
     hipStream_t s = (hipStream_t)stream;
-    const int n = L.nx * L.ny * L.nz;
+    const int n = a.L.nx * a.L.ny * a.L.nz;
     if (n > kDenseDirectCells) {
         set_error("launch_dense_solve: %d cells (at most %d)", n, kDenseDirectCells);
         return TBFG_EINVAL;
     }
-    hipLaunchKernelGGL(k_dense_apply, dim3(ceil_div(n, 4)), dim3(256), 0, s, n, G, q, x, done);
-    hipLaunchKernelGGL(k_dense_check, dim3(1), dim3(1024), 0, s, L, beta, vol, q, x, st, done);
+    hipLaunchKernelGGL(k_dense_apply, dim3(ceil_div(n, 4)), dim3(256), 0, s, n, G, a.q, x, done);
+    if (check) hipLaunchKernelGGL(k_dense_check, dim3(1), dim3(1024), 0, s, a, st, done);
+    TBFG_HIP(hipGetLastError());
+    return TBFG_OK;
+}
+int launch_fin_dots_check(unsigned nblocks, size_t ncell, int init, PcgState* st, const Reducer& red,
+                          int32_t* host_done, const DenseCheck& a, void* stream)
+{
+    hipLaunchKernelGGL(k_fin_dots_check, dim3(2), dim3(1024), 0, (hipStream_t)stream, nblocks, ncell, init, st, red,
+                       host_done, a);
     TBFG_HIP(hipGetLastError());
     return TBFG_OK;
 }

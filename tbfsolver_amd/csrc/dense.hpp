@@ -16,8 +16,18 @@ template <class T>
 int launch_dense_setup(const LevelDev<double>& L, const T* beta, const double* vol, double* work, double* G,
                        void* stream);
 
-// x = G q by grid-wide kernels, and the solve's diagnostics into st
-int launch_dense_solve(const LevelDev<double>& L, const double* beta, const double* vol, const double* G,
-                       const double* q, double* x, PcgState* st, const int* done, void* stream);
+// one exact solve of a level, for its diagnostics
+struct DenseCheck {
+    LevelDev<double> L;
+    const double *beta, *vol, *q, *x;
+};
+
+// x = G q by grid-wide kernels; check: its diagnostics into st too
+int launch_dense_solve(const DenseCheck& a, const double* G, double* x, bool check, PcgState* st, const int* done,
+                       void* stream);
+
+// launch_fin_dots, and beside it the diagnostics of the solve that launch_dense_solve left out
+int launch_fin_dots_check(unsigned nblocks, size_t ncell, int init, PcgState* st, const Reducer& red,
+                          int32_t* host_done, const DenseCheck& a, void* stream);
 
 }  // namespace tbfg

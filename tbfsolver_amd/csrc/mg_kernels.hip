@@ -378,17 +378,20 @@ __global__ void k_psi_last(size_t ncell, double* __restrict__ psi, const double*
 
 __global__ void k_fin_alpha(unsigned nblocks, PcgState* st, Reducer red)
 {
-    if (st->done) return;
+    // (the state and the partials are loaded together, here and in the kernels below: each
+    // wait of a one-block kernel is some 0.7 us of nothing else)
+    const int done = st->done;
+    const double delta = st->delta;
     double tot[1];
     final_sum<1>(red, nblocks, tot);
-    if (threadIdx.x == 0) {
+    if (threadIdx.x == 0 && !done) {
         const double den = tot[0];
-        if (!(den != 0.0) || !isfinite(den) || !isfinite(st->delta)) {
+        if (!(den != 0.0) || !isfinite(den) || !isfinite(delta)) {
             st->done = 1;
             st->status = TBFG_ENUMERIC;
             st->alpha = 0.0;
         } else {
-            st->alpha = st->delta / den;
+            st->alpha = delta / den;
         }
     }
 }
@@ -598,21 +601,22 @@ __global__ void k_pcg_update(size_t ncell, double* __restrict__ psi, double* __r
 
 __global__ void k_fin_update(unsigned nblocks, PcgState* st, Reducer red)
 {
-    if (st->done) return;
+    const int done = st->done, iter = st->iter + 1, max_iter = st->max_iter;
+    const double qq = st->qq, tol = st->tol;
     double tot[1];
     final_sum<1>(red, nblocks, tot);
-    if (threadIdx.x == 0) {
+    if (threadIdx.x == 0 && !done) {
         st->rr = tot[0];
-        st->iter += 1;
-        const double res = sqrt(tot[0]) / sqrt(st->qq + 2.2250738585072014e-308);
+        st->iter = iter;
+        const double res = sqrt(tot[0]) / sqrt(qq + 2.2250738585072014e-308);
         st->res = res;
         if (!isfinite(res)) {
             st->done = 1;
             st->status = TBFG_ENUMERIC;
-        } else if (res <= st->tol) {
+        } else if (res <= tol) {
             st->done = 1;
             st->status = TBFG_OK;
-        } else if (st->iter >= st->max_iter) {
+        } else if (iter >= max_iter) {
             st->done = 1;
             st->status = TBFG_ENOTCONVERGED;
         }
@@ -644,29 +648,9 @@ __global__ void k_pcg_dots(size_t ncell, const double* __restrict__ r, const TZ*
     block_partial<5>(v, red);
 }
 
-__global__ void k_fin_dots(unsigned nblocks, size_t ncell, int init, PcgState* st, Reducer red)
+__global__ void k_fin_dots(unsigned nblocks, size_t ncell, int init, PcgState* st, Reducer red, int32_t* host_done)
 {
-    if (st->done) return;
-    double tot[5];
-    final_sum<5>(red, nblocks, tot);
-    if (threadIdx.x == 0) {
-        const double m = tot[2] / (double)ncell;
-        const double rz = tot[0] - m * tot[3];
-        st->zmean = m;
-        if (init) {
-            st->delta = rz;
-            st->gamma = 0.0;
-        } else {
-            const double qz = tot[1] - m * tot[4];
-            const double g = st->flexible ? (-st->alpha * qz / st->delta) : (rz / st->delta);
-            st->gamma = g;
-            st->delta = rz;
-            if (!isfinite(g) || !isfinite(rz)) {
-                st->done = 1;
-                st->status = TBFG_ENUMERIC;
-            }
-        }
-    }
+    fin_dots(nblocks, ncell, init, st, red, host_done);
 }
 
 // d = (z - m) + gamma d (pcg.f90:266-290 with d0 <- d, pcg.f90:127,133-134)
@@ -2217,18 +2201,19 @@ int launch_pcg_update(size_t n, double* psi, double* r, TR* r32, const double* d
 
 template <class TZ>
 int launch_pcg_dots(size_t n, const double* r, const TZ* z, const double* qv, int init, PcgState* st,
-                    const Reducer& red, void* stream)
+                    const Reducer& red, int32_t* host_done, void* stream)
 {
     const unsigned nb = red_blocks1(n);
     hipLaunchKernelGGL(k_pcg_dots<TZ>, dim3(nb), dim3(256), 0, S(stream), n, r, z, qv, init, st, red);
-    hipLaunchKernelGGL(k_fin_dots, dim3(1), dim3(256), 0, S(stream), nb, n, init, st, red);
+    hipLaunchKernelGGL(k_fin_dots, dim3(1), dim3(256), 0, S(stream), nb, n, init, st, red, host_done);
     TBFG_HIP(hipGetLastError());
     return TBFG_OK;
 }
 
-int launch_fin_dots(unsigned nblocks, size_t ncell, int init, PcgState* st, const Reducer& red, void* stream)
+int launch_fin_dots(unsigned nblocks, size_t ncell, int init, PcgState* st, const Reducer& red, int32_t* host_done,
+                    void* stream)
 {
-    hipLaunchKernelGGL(k_fin_dots, dim3(1), dim3(1024), 0, S(stream), nblocks, ncell, init, st, red);
+    hipLaunchKernelGGL(k_fin_dots, dim3(1), dim3(1024), 0, S(stream), nblocks, ncell, init, st, red, host_done);
     TBFG_HIP(hipGetLastError());
     return TBFG_OK;
 }
@@ -2318,9 +2303,9 @@ int launch_tail(const TailPlan<T>* plan_dev, size_t cells, int nb, const int* do
 
 // explicit instantiations
 template int launch_pcg_dots<double>(size_t, const double*, const double*, const double*, int, PcgState*,
-                                     const Reducer&, void*);
+                                     const Reducer&, int32_t*, void*);
 template int launch_pcg_dots<float>(size_t, const double*, const float*, const double*, int, PcgState*,
-                                    const Reducer&, void*);
+                                    const Reducer&, int32_t*, void*);
 template int launch_pcg_dir<double>(size_t, const double*, double*, int, const PcgState*, void*);
 template int launch_pcg_dir<float>(size_t, const float*, double*, int, const PcgState*, void*);
 template int launch_rbgs<double, double>(const LevelDev<double>&, const double*, const double*, double*, int, bool,

@@ -40,7 +40,7 @@ int launch_pcg_update(size_t n, double* psi, double* r, TR* r32, const double* d
                       PcgState* st, const Reducer& red, void* stream);
 template <class TZ>
 int launch_pcg_dots(size_t n, const double* r, const TZ* z, const double* qv, int init, PcgState* st,
-                    const Reducer& red, void* stream);
+                    const Reducer& red, int32_t* host_done, void* stream);
 template <class TZ>
 int launch_pcg_dir(size_t n, const TZ* z, double* d, int init, const PcgState* st, void* stream);
 
@@ -112,7 +112,8 @@ struct InnerArgs {
 template <class T>
 int launch_inner(InnerOp op, const LevelDev<T>& L, const InnerArgs<T>& a, InnerState* is, PcgState* st,
                  const Reducer& red, void* stream);
-int launch_fin_dots(unsigned nblocks, size_t ncell, int init, PcgState* st, const Reducer& red, void* stream);
+int launch_fin_dots(unsigned nblocks, size_t ncell, int init, PcgState* st, const Reducer& red, int32_t* host_done,
+                    void* stream);
 template <class T, class TQ, class TB = T>
 int launch_resid_restrict(const LevelDev<T>& L, const TB* beta, const TQ* q, const T* p, T* qc, const int* done,
                           void* stream);

@@ -478,7 +478,8 @@ int pcg_create(const tbfg_grid_desc* g, const tbfg_pcg_params* prm_in, tbfg_pcg*
         TBFG_TRY(build_plan<double>(h.get()));
     TBFG_HIP(hipHostMalloc((void**)&h->hst, sizeof(PcgState), hipHostMallocDefault));
     std::memset(h->hst, 0, sizeof(PcgState));
-    TBFG_HIP(hipHostMalloc((void**)&h->hring, 2 * sizeof(PcgState), hipHostMallocDefault));
+    // coherent: written by kernels, read after an event
+    TBFG_HIP(hipHostMalloc((void**)&h->hring, 2 * sizeof(PcgState), hipHostMallocMapped | hipHostMallocCoherent));
     TBFG_HIP(hipHostMalloc((void**)&h->hmg, sizeof(int32_t), hipHostMallocDefault));
     for (auto& e : h->hev) TBFG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     // footprint: every device buffer of the handle
@@ -670,10 +671,11 @@ static int inner_solve(tbfg_pcg* h, void* stream)
 // r0 is the finest right-hand side in the multigrid precision; on return *z
 // points at the level-0 buffer that holds the result.  dots_init >= 0: the
 // finest level's last sweep also forms the PCG dot products of z (k_pcg_dots
-// with that init flag, finalized here); *dots_done tells whether it could.
+// with that init flag, finalized here, the stop flag left in *host_done too); *dots_done
+// tells whether it could.
 template <class T, class T0 = T>
 static int vcycle(tbfg_pcg* h, const T0* r0, T** z, const T0* beta0, const int* done, void* stream,
-                  int dots_init = -1, bool* dots_done = nullptr)
+                  int dots_init = -1, bool* dots_done = nullptr, int32_t* host_done = nullptr)
 {
     if (dots_done) *dots_done = false;
     // solveMG's loop (mg_tol > 0): after every cycle the finest residual is
@@ -701,6 +703,10 @@ static int vcycle(tbfg_pcg* h, const T0* r0, T** z, const T0* beta0, const int* 
         cur[l] = h->p[l].as<T>();
         alt[l] = h->palt[l].as<T>();
     }
+    auto bottom = [&] {
+        return DenseCheck{h->tabd[t0]->view, h->beta[t0].as<double>(), h->vol.as<double>(), h->q[t0].as<double>(),
+                          h->p[t0].as<double>()};
+    };
     for (int cyc = 0; cyc < ncycles; ++cyc) {
         for (int l = 0; l < t0; ++l) {
             const bool first = (l > 0) || (cyc == 0);
@@ -721,9 +727,9 @@ static int vcycle(tbfg_pcg* h, const T0* r0, T** z, const T0* beta0, const int* 
         if (h->kin >= 0) {
             TBFG_TRY(inner_solve<T>(h, stream));
         } else if (std::is_same<T, double>::value && h->direct) {
-            TBFG_TRY(launch_dense_solve(h->tabd[t0]->view, h->beta[t0].as<double>(), h->vol.as<double>(),
-                                        h->G.as<double>(), h->q[t0].as<double>(), h->p[t0].as<double>(),
-                                        h->st.as<PcgState>(), done, stream));
+            // (the diagnostics of the last cycle's solve go beside the finalize of the dot products)
+            TBFG_TRY(launch_dense_solve(bottom(), h->G.as<double>(), h->p[t0].as<double>(),
+                                        !(want_dots && cyc == ncycles - 1), h->st.as<PcgState>(), done, stream));
         } else {
             TBFG_TRY(launch_tail<T>(h->plan.as<TailPlan<T>>(), h->hl[h->t0].cells(), (int)h->hl[h->ntot - 1].cells(), done, h->tail_lds, stream));
         }
@@ -739,7 +745,11 @@ static int vcycle(tbfg_pcg* h, const T0* r0, T** z, const T0* beta0, const int* 
                 TBFG_TRY(smooth<T>(h, l, h->beta[l].as<T>(), h->q[l].as<T>(), cur[l], alt[l], h->prm.n_post, false,
                                    done, stream));
             if (fuse) {
-                TBFG_TRY(launch_fin_dots(nb, h->n0, dots_init, h->st.as<PcgState>(), sd.red, stream));
+                if (std::is_same<T, double>::value && h->direct)
+                    TBFG_TRY(launch_fin_dots_check(nb, h->n0, dots_init, h->st.as<PcgState>(), sd.red, host_done,
+                                                   bottom(), stream));
+                else
+                    TBFG_TRY(launch_fin_dots(nb, h->n0, dots_init, h->st.as<PcgState>(), sd.red, host_done, stream));
                 if (dots_done) *dots_done = true;
             }
         }
@@ -832,19 +842,20 @@ static int solve_t(tbfg_pcg* h, double* psi, const double* beta, const double* q
         r0 = r;
     // z = M r and the dot products of z (pcg.f90:118-139, 294-327)
     bool dots_done = false;
-    auto precondition = [&](int init) -> int {
+    auto precondition = [&](int init, int32_t* host_done) -> int {
         if constexpr (FFT) {
             z = h->zfft.as<double>();
             TBFG_TRY(fps_solve_dev(h->fps, r, z, stream));
-            TBFG_TRY(launch_pcg_dots<double>(n, r, z, qv, init, st, red, stream));
+            TBFG_TRY(launch_pcg_dots<double>(n, r, z, qv, init, st, red, host_done, stream));
         } else {
-            TBFG_TRY(vcycle<T, T0>(h, r0, &z, beta0, done, stream, h->fuse_dots ? init : -1, &dots_done));
-            if (!dots_done) TBFG_TRY(launch_pcg_dots<T>(n, r, z, qv, init, st, red, stream));
+            TBFG_TRY(vcycle<T, T0>(h, r0, &z, beta0, done, stream, h->fuse_dots ? init : -1, &dots_done,
+                                   host_done));
+            if (!dots_done) TBFG_TRY(launch_pcg_dots<T>(n, r, z, qv, init, st, red, host_done, stream));
         }
         return TBFG_OK;
     };
     TBFG_TRY(launch_residual_init(L0, h->opp, beta, q, psi, r, r32, st, red, stream));
-    TBFG_TRY(precondition(1));
+    TBFG_TRY(precondition(1, queue > 0 ? nullptr : &h->hring[0].done));
     // one iteration (pcg.f90:142-290): d = (z - m) + gamma d, qv = A d, alpha,
     // psi += alpha d, r -= alpha qv, the stop test, z = M r, the dot products.
     // Fused form: iteration j writes its direction to dbuf[j & 1] from
@@ -852,7 +863,7 @@ static int solve_t(tbfg_pcg* h, double* psi, const double* beta, const double* q
     // iteration's alpha d to psi; the last one is added after the loop.
     double* dbuf[2] = {d, h->fuse_op ? h->d2.as<double>() : d};
     int j = 0;
-    auto iteration = [&](int init) -> int {
+    auto iteration = [&](int init, int32_t* host_done) -> int {
         ++j;
         if (h->fuse_op) {
             double* dj = dbuf[j & 1];
@@ -872,17 +883,17 @@ static int solve_t(tbfg_pcg* h, double* psi, const double* beta, const double* q
             ProfScope ps(h, 3, stream);
             TBFG_TRY(launch_pcg_update(n, psi, r, r32, d, qv, st, red, stream));
         }
-        TBFG_TRY(precondition(0));
+        TBFG_TRY(precondition(0, host_done));
         return TBFG_OK;
     };
-    // copy of the device state after the work enqueued so far, and its event
+    // The stop flag after each iteration goes to a pinned slot from the kernel that ends it
+    // (a copy in the stream cost 4 us an iteration), followed by the slot's event.
     auto snapshot = [&](int slot) -> int {
-        TBFG_HIP(hipMemcpyAsync(&h->hring[slot], st, sizeof(PcgState), hipMemcpyDeviceToHost, s));
         TBFG_HIP(hipEventRecord(h->hev[slot], s));
         return TBFG_OK;
     };
     if (queue > 0) {
-        for (int32_t it = 1; it <= queue; ++it) TBFG_TRY(iteration(it == 1 ? 1 : 0));
+        for (int32_t it = 1; it <= queue; ++it) TBFG_TRY(iteration(it == 1 ? 1 : 0, nullptr));
         if (h->fuse_op) TBFG_TRY(launch_psi_last(n, psi, dbuf[0], dbuf[1], st, stream));
         h->queued_fft = FFT;
         return TBFG_OK;
@@ -891,12 +902,12 @@ static int solve_t(tbfg_pcg* h, double* psi, const double* beta, const double* q
     // already queued, so the device does not idle through the stop test; the
     // kernels of an iteration queued after convergence return at once.
     TBFG_TRY(snapshot(0));
-    TBFG_TRY(iteration(1));
+    TBFG_TRY(iteration(1, &h->hring[1].done));
     TBFG_TRY(snapshot(1));
     for (int slot = 0;; slot ^= 1) {
         TBFG_HIP(hipEventSynchronize(h->hev[slot]));
         if (h->hring[slot].done) break;
-        TBFG_TRY(iteration(0));
+        TBFG_TRY(iteration(0, &h->hring[slot].done));
         TBFG_TRY(snapshot(slot));
     }
     if (h->fuse_op) TBFG_TRY(launch_psi_last(n, psi, dbuf[0], dbuf[1], st, stream));
@@ -972,7 +983,7 @@ static int precond_t(tbfg_pcg* h, const double* beta, const double* r, double* z
     T* zt = nullptr;
     TBFG_TRY(vcycle<T, T0>(h, r0, &zt, beta0, nullptr, stream));
     // z with its arithmetic mean removed, as the reference's sweeps leave it
-    TBFG_TRY(launch_pcg_dots<T>(h->n0, r, zt, nullptr, 1, st, red, stream));
+    TBFG_TRY(launch_pcg_dots<T>(h->n0, r, zt, nullptr, 1, st, red, nullptr, stream));
     TBFG_TRY(launch_pcg_dir<T>(h->n0, zt, z, 1, st, stream));
     if (h->prm.mg_tol > 0.0) {  // the cycles taken, for tbfg_pcg_mg_stats (the loop synchronised already)
         TBFG_HIP(hipMemcpyAsync(h->hst, st, sizeof(PcgState), hipMemcpyDeviceToHost, s));

@@ -47,7 +47,7 @@ struct tbfg_pcg {
     tbfg_fps* fps = nullptr;            // FFT preconditioner (TBFG_PRECOND_FFT)
     tbfg::DevBuf zfft;                  // its output z (FP64)
     tbfg::PcgState* hst = nullptr;      // pinned mirror of the device state (final, after a solve)
-    tbfg::PcgState* hring = nullptr;    // pinned copies of the state after consecutive iterations
+    tbfg::PcgState* hring = nullptr;    // pinned slots of consecutive iterations' stop flags
     hipEvent_t hev[2] = {nullptr, nullptr};
     tbfg::HostRingUser ring_user;       // keeps the process's pinned staging
     int64_t footprint = 0;

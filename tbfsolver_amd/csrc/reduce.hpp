@@ -4,6 +4,7 @@
 
 namespace tbfg {
 
+// Sums over the workgroup (at most 16 wavefronts), valid in thread 0.
 template <int NV>
 __device__ __forceinline__ void block_sum(double (&v)[NV], double* lds /* >= 32*NV */)
 {
@@ -17,12 +18,23 @@ __device__ __forceinline__ void block_sum(double (&v)[NV], double* lds /* >= 32*
     if ((lane & 63) == 0)
         for (int q = 0; q < NV; ++q) lds[wave * NV + q] = v[q];
     __syncthreads();
-    if (lane == 0) {
-        for (int q = 0; q < NV; ++q) {
-            double s = 0.0;
-            for (int w = 0; w < nwaves; ++w) s += lds[w * NV + q];
-            v[q] = s;
+    if (lane < 64) {
+        // sum q in lane q, its LDS reads issued together, in the order of the wavefronts
+        // (one lane reading 80 values one by one took half of a finalize's 5 us)
+        const int q = lane < NV ? lane : NV - 1;
+        double s = 0.0;
+        if (nwaves <= 4) {
+#pragma unroll
+            for (int w = 0; w < 4; ++w) s += w < nwaves ? lds[w * NV + q] : 0.0;
+        } else {
+#pragma unroll
+            for (int w = 0; w < 16; ++w) s += w < nwaves ? lds[w * NV + q] : 0.0;
         }
+        if (NV == 1)
+            v[0] = s;
+        else
+#pragma unroll
+            for (int u = 0; u < NV; ++u) v[u] = __shfl(s, u, 64);
     }
 }
 
@@ -49,11 +61,58 @@ __device__ __forceinline__ void final_sum(const Reducer& red, unsigned nblocks, 
     double acc[NV];
 #pragma unroll
     for (int q = 0; q < NV; ++q) acc[q] = 0.0;
-    for (unsigned b = threadIdx.x; b < nblocks; b += blockDim.x)
-        for (int q = 0; q < NV; ++q) acc[q] += red.partials[(size_t)b * NV + q];
+    // several partials of a thread in flight: a loop of single loads waits for each
+    constexpr int U = NV == 1 ? 8 : 2;
+    for (unsigned b0 = threadIdx.x; b0 < nblocks; b0 += U * blockDim.x) {
+        double x[U][NV];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const unsigned b = b0 + u * blockDim.x;
+#pragma unroll
+            for (int q = 0; q < NV; ++q) x[u][q] = red.partials[(size_t)(b < nblocks ? b : b0) * NV + q];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int q = 0; q < NV; ++q) acc[q] += b0 + u * blockDim.x < nblocks ? x[u][q] : 0.0;
+    }
     block_sum<NV>(acc, lds);
     if (threadIdx.x == 0)
         for (int q = 0; q < NV; ++q) tot[q] = acc[q];
+}
+
+// The scalars of the next direction from the sums of the dot products (pcg.f90:294-327), by
+// one workgroup.  host_done (pinned host memory, may be NULL) receives the stop flag: the
+// host's stop test of the iteration that ends here, without a copy in the stream.
+__device__ __forceinline__ void fin_dots(unsigned nblocks, size_t ncell, int init, PcgState* st, const Reducer& red,
+                                         int32_t* host_done)
+{
+    int done = st->done;
+    const int flexible = st->flexible;
+    const double alpha = st->alpha, delta = st->delta;
+    double tot[5];
+    final_sum<5>(red, nblocks, tot);
+    if (threadIdx.x == 0) {
+        if (!done) {
+            const double m = tot[2] / (double)ncell;
+            const double rz = tot[0] - m * tot[3];
+            st->zmean = m;
+            if (init) {
+                st->delta = rz;
+                st->gamma = 0.0;
+            } else {
+                const double qz = tot[1] - m * tot[4];
+                const double g = flexible ? (-alpha * qz / delta) : (rz / delta);
+                st->gamma = g;
+                st->delta = rz;
+                if (!isfinite(g) || !isfinite(rz)) {
+                    st->done = done = 1;
+                    st->status = TBFG_ENUMERIC;
+                }
+            }
+        }
+        if (host_done) __hip_atomic_store(host_done, done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
 }  // namespace tbfg

@@ -79,3 +79,22 @@ def test_direct_coarsest_solve_matches_inner_cg(torch_gpu, monkeypatch, n, nlev,
     print("  iterations", it, it_cg, cs, cs_cg, flush=True)
     assert cs_cg["iters_max"] > 1 and abs(it - it_cg) <= 1
     assert rel(psi, psi_cg) < 1e-10
+
+
+@pytest.mark.parametrize("kw", [dict(), dict(mg_cycles=2), dict(unfused=True)], ids=["fused", "two cycles", "unfused"])
+def test_direct_coarsest_diagnostics_counted_once_per_solve(torch_gpu, monkeypatch, kw):
+    """The diagnostics of the dense coarsest solves, formed beside the dot products or by a launch of their
+    own: one call and one iteration per V-cycle, each to round-off."""
+    kw = dict(kw)
+    if kw.pop("unfused", False):
+        monkeypatch.setenv("TBFG_UNFUSED_DOTS", "1")
+    print("case direct diagnostics", kw, flush=True)
+    g, go, q, beta = setup((48, 32, 48), 1)
+    s = T.PCG(g, nLevels=3, tolPCG=1e-10, maxIterPCG=200, flexible=1, **kw)
+    psi = torch_gpu.zeros(48, 32, 48, dtype=torch_gpu.float64, device="cuda")
+    s.solvePCG(psi, to_dev(beta, torch_gpu), to_dev(q, torch_gpu))
+    cs, it = s.coarse_stats(), s.iterations
+    s.close()
+    # (an application follows every update but the last, plus the first)
+    assert cs["calls"] == it * kw.get("mg_cycles", 1), (cs, it)
+    assert cs["iters"] == cs["calls"] and cs["iters_max"] == 1 and cs["res_max"] <= 1e-10
