@@ -476,12 +476,11 @@ __global__ void __launch_bounds__(kFftThreads)
 // Stockham passes in LDS.  With n = N2 n1 + n2 and k = k1 + N1 k2,
 //   X[k1 + N1 k2] = sum_n2 W_N2^(n2 k2) [ W_N^(n2 k1) sum_n1 x[N2 n1 + n2] W_N1^(n1 k1) ].
 // Step A: thread n2 of a line holds x[N2 n1 + n2], n1 = 0..N1-1, in registers
-// (loaded from HBM, or from the pre-processed line in LDS), runs the inner
+// (loaded from HBM), runs the inner
 // N1-point DFT, multiplies by W_N^(n2 k1) and writes Y[k1][n2] to LDS.
 // Step B: thread k1 reads Y[k1][0..N2-1] and runs the outer N2-point DFT,
-// which leaves X[k1 + N1 k2] in its registers, stored straight to HBM (z
-// passes) or through one more LDS line (x passes, whose r2c/c2r packing pairs
-// X[m] with X[N-m]).  One LDS exchange per line replaces the staging, the
+// which leaves X[k1 + N1 k2] in its registers, stored straight to HBM (the x
+// passes' r2c/c2r packing, which pairs X[m] with X[N-m], by lane swaps: TlPair).  One LDS exchange per line replaces the staging, the
 // Stockham passes and the output round trip of fft_lines.  8 lines per
 // workgroup of 8 max(N1, N2) threads (the threads of the smaller factor idle
 // through the other step); Y rows of N2 + 1 elements and lines of
@@ -495,12 +494,54 @@ constexpr int kTlLines = 8;
 template <int N1, int N2>
 struct TlShape {
     static constexpr int N = N1 * N2;
-    static constexpr int NT = kTlLines * (N1 > N2 ? N1 : N2);  // threads
+    // threads: a factor's indices in pairs (TlPair)
+    static constexpr int NT = kTlLines * (N1 > N2 ? N1 + (N1 & 1) : N2 + (N2 & 1));
     static constexpr int ROW = N2 + 1;
     static constexpr int LINE = N1 * ROW + 1;
-    static constexpr int LDS = kTlLines * LINE + N;            // Y (or the x passes' lines) + twiddles
-    static_assert(LINE >= N + 1, "the x passes' lines of N + 1 fit in a Y line");
+    static constexpr int LDS = kTlLines * LINE + N;  // Y + twiddles
 };
+
+// The index of a factor N and the line that a thread works on in the x passes' step beside the
+// spectrum.  Rows m and N - m of two real lines packed into one complex line are formed from
+// Z[m] and Z[N - m], which indices k and N - k hold: they sit 8 lanes apart in a row of 16
+// (swap8), the lines across the lanes of each half, and 0 and N/2, which are their own images
+// (self), share the first row.  So the packing takes no exchange through LDS: it was one line
+// buffer, two more barriers and another round of LDS reads and writes in each x pass.
+// 256x192x256 in FP64: inverse 41.5 -> 33.3 us, forward 40.5 -> 39.8 (its input comes from HBM
+// at the rate of a copy); 144x99x108: 9.2 -> 8.0 and 10.2 -> 8.4.
+template <int N>
+struct TlPair {
+    int l, k;
+    bool act, real, self;  // has a line; an index of its own (odd N: one idle half row)
+    __device__ __forceinline__ explicit TlPair(int tid)
+    {
+        const int g = tid >> 4, s = (tid >> 3) & 1;
+        l = tid & 7;
+        self = g == 0;
+        act = tid < kTlLines * (N + (N & 1));
+        real = act && (N % 2 == 0 || tid < 8 || tid > 15);
+        k = self ? s * (N / 2) : (s ? N - g : g);
+        if (!act) k = 0;
+    }
+};
+
+// the value of the lane 8 lanes away in a row of 16 (DPP row rotate)
+__device__ __forceinline__ float swap8(float v)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128, 0xf, 0xf, true));
+}
+__device__ __forceinline__ double swap8(double v)
+{
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)b, 0x128, 0xf, 0xf, true);
+    const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), 0x128, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+template <class T>
+__device__ __forceinline__ C2<T> swap8(C2<T> v)
+{
+    return C2<T>{swap8(v.x), swap8(v.y)};
+}
 
 // cos and sin of 2 pi e / 144 for e = 0..36 (a quarter turn; the W_R of every
 // supported factor R divides 144)
@@ -720,17 +761,20 @@ __global__ void __launch_bounds__((TlShape<N1, N2>::NT))
     }
 }
 
-// K1, two-level: s(:, j, k0..k0+15) -> A[kx][j][k], kx = 0..N/2 (line l packs
-// the real lines k0+2l and k0+2l+1 into one complex line, as k_xfwd)
+// K1, two-level: s(:, j, k0..k0+15) -> A[kx][j][k], kx = 0..N/2.  Line l packs the real
+// lines k0+l and k0+l+8 (half the lines of a last workgroup) into one complex line: a
+// store of either then covers 8 neighbouring elements, where pairs of neighbours made
+// every store skip every second one (44.6 us at 256x192x256)
 template <class T, class TIN, int N1, int N2, bool PART>
 __global__ void __launch_bounds__((TlShape<N1, N2>::NT))
     k_xfwd_tl(int ny, int nz, const C2<T>* __restrict__ tw, const TIN* __restrict__ s, C2<T>* __restrict__ A)
 {
     using S = TlShape<N1, N2>;
-    constexpr int N = S::N, KT = 2 * kTlLines, LS = N + 1, nh = N / 2 + 1;
+    constexpr int N = S::N, KT = 2 * kTlLines;
     __shared__ C2<T> Y[S::LDS];
     C2<T>* twl = Y + kTlLines * S::LINE;
     const int j = blockIdx.y, k0 = blockIdx.x * KT;
+    const int hf = PART ? min(kTlLines, (nz - k0) / 2) : kTlLines;  // lines of this workgroup
     const int tid = threadIdx.x;
     __builtin_assume(tid < S::NT);  // the launch's block size
     TlTwiddles<T, N1, N2> tws;
@@ -739,11 +783,10 @@ __global__ void __launch_bounds__((TlShape<N1, N2>::NT))
         const int l = tid / N2, n2 = tid - l * N2;  // lanes along the line
         const bool act = tid < kTlLines * N2;
         const size_t plane = (size_t)N * ny;
-        const int kl = k0 + 2 * (act ? l : 0);
-        const TIN* s0 = s + n2 + (size_t)N * (j + (size_t)ny * (PART ? min(kl, nz - 2) : kl));
+        const TIN* s0 = s + n2 + (size_t)N * j + plane * (k0 + min(act ? l : 0, hf - 1));
         C2<T> v[N1];
 #pragma unroll
-        for (int n1 = 0; n1 < N1; ++n1) v[n1] = C2<T>{(T)s0[N2 * n1], (T)s0[N2 * n1 + plane]};
+        for (int n1 = 0; n1 < N1; ++n1) v[n1] = C2<T>{(T)s0[N2 * n1], (T)s0[N2 * n1 + plane * hf]};
         tws.put(twl);
         __syncthreads();
         if (act) {
@@ -752,35 +795,28 @@ __global__ void __launch_bounds__((TlShape<N1, N2>::NT))
         }
     }
     __syncthreads();
-    {
-        const int l = tid / N1, k1 = tid - l * N1;
-        const bool act = tid < kTlLines * N1;
-        C2<T> v[N2];
-        if (act) {
-            const C2<T>* y = Y + l * S::LINE + k1 * S::ROW;
+    const TlPair<N1> pr(tid);
+    if (!pr.act) return;
+    const int l = pr.l, k1 = pr.k;
+    const C2<T>* y = Y + l * S::LINE + k1 * S::ROW;
+    C2<T> v[N2];
 #pragma unroll
-            for (int n2 = 0; n2 < N2; ++n2) v[n2] = y[n2];
-            DftReg<T, -1, N2>::run(v);
-        }
-        __syncthreads();  // every Y row read before the lines overwrite them
-        if (act) {
-            C2<T>* x = Y + l * LS + k1;
+    for (int n2 = 0; n2 < N2; ++n2) v[n2] = y[n2];
+    DftReg<T, -1, N2>::run(v);
+    // rows m and N - m of the two real lines: Z[m] is v[k2], Z[N - m] the partner's v[N2 - 1 - k2]
+    C2<T>* dst = A + ((size_t)k1 * ny + j) * nz + k0 + l;
+    const bool store = pr.real && (!PART || l < hf);
 #pragma unroll
-            for (int k2 = 0; k2 < N2; ++k2) x[N1 * k2] = v[k2];
+    for (int k2 = 0; k2 <= N2 / 2; ++k2) {
+        const C2<T> Z = v[k2], own = v[N2 - 1 - k2], oth = swap8(own), zero = v[(N2 - k2) % N2];
+        const C2<T> Zn = pr.self ? (k1 == 0 ? zero : own) : oth;
+        const C2<T> e{(T)0.5 * (Z.x + Zn.x), (T)0.5 * (Z.y - Zn.y)};  // (Z + conj Zn)/2
+        const C2<T> o{(T)0.5 * (Z.y + Zn.y), (T)0.5 * (Zn.x - Z.x)};  // (Z - conj Zn)/(2i)
+        if (store && (k2 < N2 / 2 || 2 * (k1 + N1 * k2) <= N)) {
+            C2<T>* d = dst + (size_t)(N1 * k2) * ny * nz;
+            d[0] = e;
+            d[hf] = o;
         }
-    }
-    __syncthreads();
-    for (int t = tid; t < nh * KT; t += S::NT) {
-        const int m = t / KT, kk = t - m * KT;
-        const int l = kk >> 1;
-        const C2<T> Z = Y[l * LS + m];
-        const C2<T> Zn = Y[l * LS + (m == 0 ? 0 : N - m)];
-        C2<T> val;
-        if ((kk & 1) == 0)
-            val = C2<T>{(T)0.5 * (Z.x + Zn.x), (T)0.5 * (Z.y - Zn.y)};  // (Z + conj Zn)/2
-        else
-            val = C2<T>{(T)0.5 * (Z.y + Zn.y), (T)0.5 * (Zn.x - Z.x)};  // (Z - conj Zn)/(2i)
-        if (!PART || k0 + kk < nz) A[((size_t)m * ny + j) * nz + k0 + kk] = val;
     }
 }
 
@@ -792,70 +828,66 @@ __global__ void __launch_bounds__((TlShape<N1, N2>::NT))
               int mode, const double* __restrict__ shift)
 {
     using S = TlShape<N1, N2>;
-    constexpr int N = S::N, L = kTlLines, KT = 2 * L, LS = N + 1, nh = N / 2 + 1;
-    constexpr int kB = stage_batch<T>() / 2;  // two complex loads per element
+    constexpr int N = S::N, KT = 2 * kTlLines;
     __shared__ C2<T> Y[S::LDS];
     C2<T>* twl = Y + kTlLines * S::LINE;
     const int j = blockIdx.y, k0 = blockIdx.x * KT;
+    const int hf = PART ? min(kTlLines, (nz - k0) / 2) : kTlLines;  // lines of this workgroup
     const int tid = threadIdx.x;
     __builtin_assume(tid < S::NT);  // the launch's block size
     TlTwiddles<T, N1, N2> tws;
     tws.fetch(tw);
-    tws.put(twl);  // here: the compiler would otherwise issue the fetch after the staging loop
-    // Z_l[m] = X1[m] + i X2[m] with Hermitian extension, into the lines (as k_xinv)
-    for (int t0 = tid; t0 < nh * L; t0 += kB * S::NT) {
-        T x1r[kB], x1i[kB], x2r[kB], x2i[kB];
-#pragma unroll
-        for (int u = 0; u < kB; ++u) {
-            const int t = min(t0 + u * S::NT, nh * L - 1);
-            const int m = t / L, l = t - m * L;
-            const size_t o = ((size_t)m * ny + j) * nz + (PART ? min(k0 + 2 * l, nz - 2) : k0 + 2 * l);
-            const C2<T> a = A[o], b = A[o + 1];
-            x1r[u] = a.x;
-            x1i[u] = a.y;
-            x2r[u] = b.x;
-            x2i[u] = b.y;
-        }
-#pragma unroll
-        for (int u = 0; u < kB; ++u) {
-            const int t = t0 + u * S::NT;
-            if (t < nh * L) {
-                const int m = t / L, l = t - m * L;
-                const C2<T> x1{x1r[u], x1i[u]}, x2{x2r[u], x2i[u]};
-                if (m == 0 || 2 * m == N) {
-                    Y[l * LS + m] = C2<T>{x1.x, x2.x};
-                } else {
-                    Y[l * LS + m] = C2<T>{x1.x - x2.y, x1.y + x2.x};
-                    Y[l * LS + N - m] = C2<T>{x1.x + x2.y, x2.x - x1.y};
-                }
-            }
-        }
-    }
-    __syncthreads();
+    // Z_l[m] = X1[m] + i X2[m] for m = N2 n1 + n2, n1 = 0..N1-1: the rows up to N/2 loaded
+    // here, the others their Hermitian images, which the partner loaded (as row N - m)
     {
-        const int l = tid / N2, n2 = tid - l * N2;
-        const bool act = tid < kTlLines * N2;
-        C2<T> v[N1];
-        if (act) {
+        const TlPair<N2> pr(tid);
+        const int l = pr.l, n2 = pr.k;
+        const C2<T>* src = A + ((size_t)n2 * ny + j) * nz + k0 + min(l, hf - 1);
+        const bool mid = 2 * (N2 * (N1 / 2) + n2) <= N;  // row n1 = N1/2 is one of the lower half
+        C2<T> x1[N1 / 2 + 1], x2[N1 / 2 + 1];
 #pragma unroll
-            for (int n1 = 0; n1 < N1; ++n1) v[n1] = Y[l * LS + N2 * n1 + n2];
-            DftReg<T, +1, N1>::run(v);
+        for (int n1 = 0; n1 <= N1 / 2; ++n1) {
+            // (otherwise the row before it again: in the cache, and not used)
+            const int r = n1 < N1 / 2 || mid ? N2 * n1 : N2 * (n1 - 1);
+            const C2<T>* a = src + (size_t)r * ny * nz;
+            x1[n1] = a[0], x2[n1] = a[hf];
         }
-        __syncthreads();  // every line read before Y overwrites them
-        if (act) tl_store_y<T, +1, N1, N2>(Y, twl, l, n2, v);
+        tws.put(twl);
+        __syncthreads();
+        if (pr.act) {
+            C2<T> v[N1], im[N1 / 2 + 1];
+#pragma unroll
+            for (int n1 = 0; n1 <= N1 / 2; ++n1) {
+                const C2<T> a = x1[n1], b = x2[n1];
+                const bool ends = n1 == 0 ? n2 == 0 : (n1 == N1 / 2 && 2 * (N2 * n1 + n2) == N);
+                v[n1] = ends ? C2<T>{a.x, b.x} : C2<T>{a.x - b.y, a.y + b.x};
+                im[n1] = C2<T>{a.x + b.y, b.x - a.y};
+            }
+#pragma unroll
+            for (int n1 = N1 / 2; n1 < N1; ++n1) {
+                const C2<T> own = im[N1 - 1 - n1], oth = swap8(own), zero = im[N1 - n1 <= N1 / 2 ? N1 - n1 : 0];
+                const C2<T> up = pr.self ? (n2 == 0 ? zero : own) : oth;
+                if (n1 > N1 / 2)
+                    v[n1] = up;
+                else if (!mid)
+                    v[n1] = up;
+            }
+            DftReg<T, +1, N1>::run(v);
+            if (pr.real) tl_store_y<T, +1, N1, N2>(Y, twl, l, n2, v);
+        }
     }
     __syncthreads();
     if (tid >= kTlLines * N1) return;
     const int l = tid / N1, k1 = tid - l * N1;  // lanes along the line
-    if (PART && k0 + 2 * l >= nz) return;
+    if (PART && l >= hf) return;
     const C2<T>* y = Y + l * S::LINE + k1 * S::ROW;
     C2<T> v[N2];
 #pragma unroll
     for (int n2 = 0; n2 < N2; ++n2) v[n2] = y[n2];
     DftReg<T, +1, N2>::run(v);
     const double scale = 1.0 / ((double)N * (double)nz);
-    const size_t plane = (size_t)N * ny;
-    double* p0 = p + k1 + (size_t)N * (j + (size_t)ny * (k0 + 2 * l));
+    const size_t plane = (size_t)N * ny * hf;  // to the line's second real line
+    double* p0 = p + k1 + (size_t)N * (j + (size_t)ny * (k0 + l));
     if (mode == 0) {
 #pragma unroll
         for (int k2 = 0; k2 < N2; ++k2) {
