@@ -747,6 +747,7 @@ __device__ __forceinline__ T resid_restrict_cell(const LV& L, PB __restrict__ be
 // the fine planes either side), the eight in-plane neighbours of the 2x2 block
 // once per fine plane -- about 7 loads per fine cell instead of 20.
 constexpr int kRrPlanes = 2;
+constexpr size_t kRrSmallCells = (size_t)1 << 21;
 
 template <class T>
 __device__ __forceinline__ T cell_residual(T qc, T bc, T be, T bw, T bn, T bs, T bf, T bb, T pc, T pe, T pw, T pn,
@@ -838,6 +839,104 @@ __global__ void k_resid_restrict(LevelDev<T> L, const TB* __restrict__ beta, con
     }
 }
 
+template <class T>
+struct Pair;
+template <>
+struct Pair<float> {
+    using type = float2;
+};
+template <>
+struct Pair<double> {
+    using type = double2;
+};
+
+// two neighbouring values of a row (a caller's beta may be aligned to its elements only)
+template <class T, class TS>
+__device__ __forceinline__ typename Pair<T>::type load_pair(const TS* __restrict__ a)
+{
+    if constexpr (std::is_same<TS, bf16s>::value) {
+        const uint32_t w = *reinterpret_cast<const uint32_t*>(a);
+        return typename Pair<T>::type{__builtin_bit_cast(float, w << 16), __builtin_bit_cast(float, w & 0xffff0000u)};
+    } else {
+        using V = T __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+        const V v = *reinterpret_cast<const V*>(a);
+        return typename Pair<T>::type{v.x, v.y};
+    }
+}
+
+// The same, a thread per coarse cell with its 16 rows of p and beta and 8 of q loaded at once:
+// a small level's time is the rounds of loads that wait for one another (four of them
+// above), not its bytes.  Per launch, FP64: 2 M cells 10.9 -> 10.3 us, 393 K 7.0 -> 5.7, 49 K
+// 6.7 -> 4.4, 6 K 6.8 -> 3.7; FP32: 1.6 M 8.6 -> 7.5, 161 K 6.7 -> 4.3.  Above 2 M cells, where
+// the planes it reads twice count (12.6 M cells in bf16: 26.9 and 29.2 us), the segments stay.
+template <class T, class TQ, class TB>
+__global__ void __launch_bounds__(256)
+    k_resid_restrict_small(LevelDev<T> L, const TB* __restrict__ beta, const TQ* __restrict__ q,
+                           const T* __restrict__ p, T* __restrict__ qc, const int* done)
+{
+    if (done && *done) return;
+    const int nx = L.nx, ny = L.ny, nz = L.nz;
+    const int ncx = nx >> 1, ncy = ny >> 1;
+    const Blk3 bk = xcd_block3((ncx + blockDim.x - 1) / blockDim.x, (ncy + blockDim.y - 1) / blockDim.y);
+    const int I = bk.x * blockDim.x + threadIdx.x;
+    const int J = bk.y * blockDim.y + threadIdx.y;
+    const int K = bk.z;
+    if (I >= ncx || J >= ncy) return;
+    using P2 = typename Pair<T>::type;
+    const int i0 = 2 * I, j0 = 2 * J, k0 = 2 * K;
+    const int iw = i0 > 0 ? i0 - 1 : nx - 1, ie = i0 + 2 < nx ? i0 + 2 : 0;
+    const int js[4] = {j0 > 0 ? j0 - 1 : j0, j0, j0 + 1, j0 + 2 < ny ? j0 + 2 : j0 + 1};  // wall ghost = the cell itself
+    const int ks[4] = {k0 > 0 ? k0 - 1 : nz - 1, k0, k0 + 1, k0 + 2 < nz ? k0 + 2 : 0};
+    // x pairs of the 12 rows that touch the block (no corner rows), and for the four rows of
+    // the block the cells to the west and east
+    P2 P[4][4], B[4][4], Q[2][2];
+    T pw[2][2], pe[2][2], bw[2][2], be[2][2];
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            if ((b == 0 || b == 3) && (c == 0 || c == 3)) continue;
+            const size_t row = (size_t)nx * (js[b] + (size_t)ny * ks[c]);
+            P[c][b] = load_pair<T, T>(p + row + i0);
+            B[c][b] = load_pair<T, TB>(beta + row + i0);
+            if (b == 0 || b == 3 || c == 0 || c == 3) continue;
+            pw[c - 1][b - 1] = p[row + iw], pe[c - 1][b - 1] = p[row + ie];
+            bw[c - 1][b - 1] = beta[row + iw], be[c - 1][b - 1] = beta[row + ie];
+            Q[c - 1][b - 1] = load_pair<T, TQ>(q + row + i0);
+        }
+    const T ipx0 = L.a[0].ip[i0], imx0 = L.a[0].im[i0], ipx1 = L.a[0].ip[i0 + 1], imx1 = L.a[0].im[i0 + 1];
+    const T wx0 = L.a[0].rlo[I], wx1 = L.a[0].rhi[I];
+    T ipy[2], imy[2], ipz[2], imz[2], wy[2], wz[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        ipy[u] = L.a[1].ip[j0 + u], imy[u] = L.a[1].im[j0 + u];
+        ipz[u] = L.a[2].ip[k0 + u], imz[u] = L.a[2].im[k0 + u];
+    }
+    wy[0] = L.a[1].rlo[J], wy[1] = L.a[1].rhi[J], wz[0] = L.a[2].rlo[K], wz[1] = L.a[2].rhi[K];
+    __builtin_amdgcn_sched_barrier(0);  // every load above before the arithmetic
+    T acc = 0;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        T r[2][2];
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const P2 Pc = P[c + 1][b + 1], Bc = B[c + 1][b + 1], Pn = P[c + 1][b + 2], Bn = B[c + 1][b + 2],
+                     Ps = P[c + 1][b], Bs = B[c + 1][b], Pf = P[c + 2][b + 1], Bf = B[c + 2][b + 1], Pb = P[c][b + 1],
+                     Bb = B[c][b + 1];
+            r[b][0] = cell_residual<T>(Q[c][b].x, Bc.x, Bc.y, bw[c][b], Bn.x, Bs.x, Bf.x, Bb.x, Pc.x, Pc.y, pw[c][b],
+                                       Pn.x, Ps.x, Pf.x, Pb.x, ipx0, imx0, ipy[b], imy[b], ipz[c], imz[c]);
+            r[b][1] = cell_residual<T>(Q[c][b].y, Bc.y, be[c][b], Bc.x, Bn.y, Bs.y, Bf.y, Bb.y, Pc.y, pe[c][b], Pc.x,
+                                       Pn.y, Ps.y, Pf.y, Pb.y, ipx1, imx1, ipy[b], imy[b], ipz[c], imz[c]);
+        }
+        // children in the reference's order: dj outer, di inner
+        acc += (wx0 * wy[0] * wz[c]) * r[0][0];
+        acc += (wx1 * wy[0] * wz[c]) * r[0][1];
+        acc += (wx0 * wy[1] * wz[c]) * r[1][0];
+        acc += (wx1 * wy[1] * wz[c]) * r[1][1];
+    }
+    qc[I + (size_t)ncx * (J + (size_t)ncy * K)] = acc;
+}
+
 // plain restriction of a field (beta, restrictField at multiGrid.f90:210)
 template <class TF, class T>
 __global__ void k_restrict(LevelDev<T> L, const TF* __restrict__ fine, T* __restrict__ coarse)
@@ -885,19 +984,9 @@ __device__ __forceinline__ void prolong_cell(const LV& L, int ncx, int ncy, int 
     p[c] = p[c] + v;
 }
 
-template <class T>
-struct Pair;
-template <>
-struct Pair<float> {
-    using type = float2;
-};
-template <>
-struct Pair<double> {
-    using type = double2;
-};
-
 // One thread per coarse cell: its 2x2x2 fine children all interpolate from the
-// 3x3x3 coarse neighbourhood, loaded once (the weights and the order of the
+// 3x3x3 coarse neighbourhood, loaded once together with p and the weights (FP64, 6 K cells:
+// 4.4 -> 3.5 us, 2 M 9.3 -> 8.8; the weights and the order of the
 // arithmetic are prolong_cell's), and each pair of x-children is one vector
 // access.
 template <class T>
@@ -922,27 +1011,38 @@ __global__ void k_prolong_add(LevelDev<T> L, const T* __restrict__ pc, T* __rest
         for (int b = 0; b < 3; ++b)
 #pragma unroll
             for (int e = 0; e < 3; ++e) c[a][b][e] = pc[xs[e] + (size_t)ncx * (ys[b] + (size_t)ncy * zs[a])];
+    using P2 = typename Pair<T>::type;
+    P2 f[2][2];
+    P2* const p2 = reinterpret_cast<P2*>(p + 2 * I + (size_t)nx * (2 * J + (size_t)ny * (2 * K)));
+    const size_t sy = (size_t)ncx, sz = (size_t)ncx * ny;  // in pairs
+#pragma unroll
+    for (int dk = 0; dk < 2; ++dk)
+#pragma unroll
+        for (int dj = 0; dj < 2; ++dj) f[dk][dj] = p2[sz * dk + sy * dj];
     const T wxl0 = L.a[0].plo[2 * I], wxh0 = L.a[0].phi[2 * I];
     const T wxl1 = L.a[0].plo[2 * I + 1], wxh1 = L.a[0].phi[2 * I + 1];
+    T wy[2][2], wz[2][2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        wy[u][0] = L.a[1].plo[2 * J + u], wy[u][1] = L.a[1].phi[2 * J + u];
+        wz[u][0] = L.a[2].plo[2 * K + u], wz[u][1] = L.a[2].phi[2 * K + u];
+    }
+    __builtin_amdgcn_sched_barrier(0);  // one round of loads
 #pragma unroll
     for (int dk = 0; dk < 2; ++dk) {
-        const int k = 2 * K + dk;
-        const T wzl = L.a[2].plo[k], wzh = L.a[2].phi[k];
+        const T wzl = wz[dk][0], wzh = wz[dk][1];
 #pragma unroll
         for (int dj = 0; dj < 2; ++dj) {
-            const int j = 2 * J + dj;
-            const T wyl = L.a[1].plo[j], wyh = L.a[1].phi[j];
+            const T wyl = wy[dj][0], wyh = wy[dj][1];
             // children (2I, j, k) and (2I+1, j, k): coarse x cells (I-1, I) and (I, I+1)
             const T (&zl)[3][3] = c[dk], (&zh)[3][3] = c[dk + 1];
             const T v0 = wzl * (wyl * (wxl0 * zl[dj][0] + wxh0 * zl[dj][1]) + wyh * (wxl0 * zl[dj + 1][0] + wxh0 * zl[dj + 1][1])) +
                          wzh * (wyl * (wxl0 * zh[dj][0] + wxh0 * zh[dj][1]) + wyh * (wxl0 * zh[dj + 1][0] + wxh0 * zh[dj + 1][1]));
             const T v1 = wzl * (wyl * (wxl1 * zl[dj][1] + wxh1 * zl[dj][2]) + wyh * (wxl1 * zl[dj + 1][1] + wxh1 * zl[dj + 1][2])) +
                          wzh * (wyl * (wxl1 * zh[dj][1] + wxh1 * zh[dj][2]) + wyh * (wxl1 * zh[dj + 1][1] + wxh1 * zh[dj + 1][2]));
-            typename Pair<T>::type* q = reinterpret_cast<typename Pair<T>::type*>(p + 2 * I + (size_t)nx * (j + (size_t)ny * k));
-            typename Pair<T>::type f = *q;
-            f.x = f.x + v0;
-            f.y = f.y + v1;
-            *q = f;
+            f[dk][dj].x = f[dk][dj].x + v0;
+            f[dk][dj].y = f[dk][dj].y + v1;
+            p2[sz * dk + sy * dj] = f[dk][dj];
         }
     }
 }
@@ -2252,6 +2352,14 @@ int launch_resid_restrict(const LevelDev<T>& L, const TB* beta, const TQ* q, con
                           void* stream)
 {
     dim3 blk = block2d(L.nx >> 1);
+    if constexpr (std::is_same<TB, TQ>::value) {
+        if ((size_t)L.nx * L.ny * L.nz <= kRrSmallCells) {
+            const dim3 g1(ceil_div(L.nx >> 1, blk.x) * ceil_div(L.ny >> 1, blk.y) * (L.nz >> 1));
+            hipLaunchKernelGGL((k_resid_restrict_small<T, TQ, TB>), g1, blk, 0, S(stream), L, beta, q, p, qc, done);
+            TBFG_HIP(hipGetLastError());
+            return TBFG_OK;
+        }
+    }
     const dim3 grd(ceil_div(L.nx >> 1, blk.x) * ceil_div(L.ny >> 1, blk.y) * ceil_div(L.nz >> 1, kRrPlanes));
     hipLaunchKernelGGL((k_resid_restrict<T, TQ, TB>), grd, blk, 0, S(stream), L, beta, q, p, qc, done);
     TBFG_HIP(hipGetLastError());

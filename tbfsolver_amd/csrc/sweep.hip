@@ -517,6 +517,10 @@ __global__ void __launch_bounds__(256)
     const T zp = half * L.a[2].ip[k], zm = half * L.a[2].im[k];
     const T zpf = half * L.a[2].ip[kf], zmf = half * L.a[2].im[kf], zpb = half * L.a[2].ip[kb], zmb = half * L.a[2].im[kb];
 
+    // every load above before the arithmetic: the compiler otherwise saves registers by
+    // loading in rounds that each wait (FP64, 49 K cells: 5.4 -> 4.9 us)
+    __builtin_amdgcn_sched_barrier(0);
+
     const std::true_type red;
     // one update: centre beta, the six neighbours' beta and p
     auto update = [&](T qq, T c, T bE, T bW, T bN, T bS, T bF, T bB, T fxp, T fxm, T fyp, T fym, T fzp, T fzm, T pE, T pW,

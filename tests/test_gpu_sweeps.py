@@ -109,3 +109,41 @@ def test_dots_in_row_and_point_sweeps(torch_gpu, monkeypatch, n, min_cells, prec
         s.close()
     assert abs(out[0][0] - out[1][0]) <= 1
     assert rel(out[0][1], out[1][1]) < 1e-9
+
+
+@pytest.mark.parametrize("n", [(2, 4, 2), (4, 2, 6), (12, 10, 2), (66, 6, 4), (132, 4, 8), (256, 4, 8)])
+def test_beta_aligned_to_its_elements(torch_gpu, n):
+    """A caller's beta and q at an address that is no multiple of 16: the paired loads of the restriction
+    read the same values, so the application is the same to the bit."""
+    print("case element alignment", n, flush=True)
+    g, beta, q = case(torch_gpu, n)
+
+    def shifted(t):
+        b = torch_gpu.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view(t.shape)
+        b.copy_(t)
+        return b
+
+    a = apply(torch_gpu, g, beta, q, precision="fp64")
+    b = apply(torch_gpu, g, shifted(beta), shifted(q), precision="fp64")
+    assert np.all(np.isfinite(a)) and np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("n", [(2, 4, 2), (4, 2, 6), (12, 10, 2), (66, 6, 4), (132, 4, 8), (256, 4, 8), (32, 32, 32)])
+def test_cycle_with_one_sweep_matches_oracle_at_remainders(torch_gpu, n):
+    """One V-cycle (two levels, one sweep each way, so that the residual and the correction carry it) on axes
+    of two cells and rows that leave the last workgroup partly filled, against the oracle to 1e-12."""
+    from oracle import pyoracle as O
+
+    print("case restriction, prolongation", n, flush=True)
+    g, beta, q = case(torch_gpu, n)
+    s = T.PCG(g, nLevels=2, nPreSweep=1, nPostSweep=1, coarse_max_iter=0)
+    z = torch_gpu.zeros_like(q)
+    s.precondition(beta, q, z)
+    s.close()
+    go = O.desc(n, stretch=(0, 1, 0), gamma=1.5)
+    prm = O.params(n_levels=2, n_pre=1, n_post=1, coarse_mode=1, coarse_cycles=1)
+    ref = O.mg_apply(go, prm, to_host(beta), to_host(q))
+    out = to_host(z)
+    e = rel(out - out.mean(), ref - ref.mean())
+    print("  rel error", e, flush=True)
+    assert e < 1e-12
