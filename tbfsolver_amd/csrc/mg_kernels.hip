@@ -363,6 +363,126 @@ __global__ void __launch_bounds__(NT) k_op_march(LevelDev<double> L, const doubl
     block_partial<1>(acc, red);
 }
 
+template <class T>
+struct Pair;
+template <>
+struct Pair<float> {
+    using type = float2;
+};
+template <>
+struct Pair<double> {
+    using type = double2;
+};
+
+// two neighbouring values of a row (a caller's beta may be aligned to its elements only)
+template <class T, class TS>
+__device__ __forceinline__ typename Pair<T>::type load_pair(const TS* __restrict__ a)
+{
+    if constexpr (std::is_same<TS, bf16s>::value) {
+        const uint32_t w = *reinterpret_cast<const uint32_t*>(a);
+        return typename Pair<T>::type{__builtin_bit_cast(float, w << 16), __builtin_bit_cast(float, w & 0xffff0000u)};
+    } else {
+        using V = T __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+        const V v = *reinterpret_cast<const V*>(a);
+        return typename Pair<T>::type{v.x, v.y};
+    }
+}
+
+// The same pass on grids below 1 M cells, a thread per x pair of cells without any exchange:
+// the direction at the pair and its ten neighbours is formed from z and d_old there (the
+// rows beside a pair's own come from L1 and L2), every load issued at once.  A march of a few
+// planes is mostly its start and its barriers, and grids that no tile divides took a
+// separate direction kernel and columns of 16 planes.  Per launch: 393 K cells FP64
+// 13.8 -> 9.6 us, FP32 z 11.6 -> 7.3, 131 K 8.8 -> 4.4, 161 K (72x40x56) 13.1 -> 5.4.  Any even nx.
+template <class TZ, bool DIR>
+__global__ void __launch_bounds__(256)
+    k_op_point(LevelDev<double> L, const double* __restrict__ beta, const double* __restrict__ din,
+               double* __restrict__ qv, const PcgState* st, Reducer red, uint32_t m_hx, uint32_t m_ny, int npairs,
+               OpDir<TZ> od)
+{
+    if (st->done) return;
+    unsigned id = blockIdx.x;  // consecutive blocks on one XCD
+    if ((gridDim.x & 7u) == 0) id = (id & 7u) * (gridDim.x >> 3) + (id >> 3);
+    const int tp = (int)(id * 256u + threadIdx.x);
+    const bool own = tp < npairs;  // (the last block's idle threads follow the last pair)
+    const int t = own ? tp : npairs - 1;
+    const int nx = L.nx, ny = L.ny, nz = L.nz, hx = nx >> 1;
+    const int row = hx == 1 ? t : (int)__umulhi((uint32_t)t, m_hx), h = t - row * hx;
+    const int k = ny == 1 ? row : (int)__umulhi((uint32_t)row, m_ny), j = row - k * ny;
+    const int i = 2 * h, ie = i + 2 < nx ? i + 2 : 0, iw = i > 0 ? i - 1 : nx - 1;
+    auto rw = [&](int jj, int kk) { return nx * (jj + ny * kk); };
+    // the pair; the pairs to N, S (a wall's ghost: the cell itself), F, B
+    const int rc = rw(j, k), c = rc + i;
+    const int o[5] = {c, rw(min(j + 1, ny - 1), k) + i, rw(max(j - 1, 0), k) + i, rw(j, k + 1 < nz ? k + 1 : 0) + i,
+                      rw(j, k > 0 ? k - 1 : nz - 1) + i};
+    const bool init = DIR && od.init != 0;
+    const double* dsrc = DIR ? od.dold : din;
+    double2 b[5], d[5], psi = {0.0, 0.0};
+    typename Pair<TZ>::type z[5];
+    TZ ze = 0, zw = 0;
+#pragma unroll
+    for (int u = 0; u < 5; ++u) {
+        b[u] = load_pair<double, double>(beta + o[u]);
+        if (DIR) z[u] = load_pair<TZ, TZ>(od.z + o[u]);
+        d[u] = double2{0.0, 0.0};
+    }
+    const double be = beta[rc + ie], bw = beta[rc + iw];
+    if (DIR) ze = od.z[rc + ie], zw = od.z[rc + iw];
+    double de = 0.0, dw = 0.0;
+    if (!init) {
+#pragma unroll
+        for (int u = 0; u < 5; ++u) d[u] = load_pair<double, double>(dsrc + o[u]);
+        de = dsrc[rc + ie], dw = dsrc[rc + iw];
+        if (DIR) psi = load_pair<double, double>(od.psi + c);
+    }
+    const double zmean = DIR ? st->zmean : 0.0, gamma = DIR ? st->gamma : 0.0, alpha = DIR ? st->alpha : 0.0;
+    const double ipx0 = L.a[0].ip[i], imx0 = L.a[0].im[i], ipx1 = L.a[0].ip[i + 1], imx1 = L.a[0].im[i + 1];
+    const double ipy = L.a[1].ip[j], imy = L.a[1].im[j], ipz = L.a[2].ip[k], imz = L.a[2].im[k];
+    __builtin_amdgcn_sched_barrier(0);  // one round of loads
+    const double2 dold = d[0];
+    auto dir = [&](double zz, double dd) {  // k_pcg_dir's arithmetic
+        const double zc = zz - zmean;
+        return init ? zc : zc + gamma * dd;
+    };
+    if (DIR) {
+#pragma unroll
+        for (int u = 0; u < 5; ++u) d[u] = double2{dir((double)z[u].x, d[u].x), dir((double)z[u].y, d[u].y)};
+        de = dir((double)ze, de), dw = dir((double)zw, dw);
+    }
+    // face coefficients (rbgs.f90:220-226) and (A d)_c (pcg.f90:171-176), as apply_cell; the
+    // fused multiply-adds written out, so that both forms of the kernel round alike
+    auto apply = [&](double bc, double bE, double bW, double bN, double bS, double bF, double bB, double dc, double dE,
+                     double dW, double dN, double dS, double dF, double dB, double ipx, double imx) {
+#pragma clang fp contract(off)
+        const double aR = 0.5 * (bE + bc) * ipx;
+        const double aL = 0.5 * (bc + bW) * imx;
+        const double aT = 0.5 * (bN + bc) * ipy;
+        const double aB = 0.5 * (bc + bS) * imy;
+        const double aF = 0.5 * (bF + bc) * ipz;
+        const double aK = 0.5 * (bc + bB) * imz;
+        double v = fma(aR, dE - dc, -(aL * (dc - dW)));
+        v = fma(aT, dN - dc, v);
+        v = fma(-aB, dc - dS, v);
+        v = fma(aF, dF - dc, v);
+        return fma(-aK, dc - dB, v);
+    };
+    const double v0 = apply(b[0].x, b[0].y, bw, b[1].x, b[2].x, b[3].x, b[4].x, d[0].x, d[0].y, dw, d[1].x, d[2].x,
+                            d[3].x, d[4].x, ipx0, imx0);
+    const double v1 = apply(b[0].y, be, b[0].x, b[1].y, b[2].y, b[3].y, b[4].y, d[0].y, de, d[0].x, d[1].y, d[2].y,
+                            d[3].y, d[4].y, ipx1, imx1);
+    double acc[1] = {0.0};
+    if (own) {
+        acc[0] = fma(d[0].x, v0, d[0].y * v1);
+        *reinterpret_cast<double2*>(qv + c) = double2{v0, v1};
+        if (DIR) *reinterpret_cast<double2*>(od.dnew + c) = d[0];
+        if (DIR && !init) {  // k_pcg_update's arithmetic; psi is the caller's, aligned to its elements
+            od.psi[c] = psi.x + alpha * dold.x;
+            od.psi[c + 1] = psi.y + alpha * dold.y;
+        }
+    }
+    block_partial<1>(acc, red);
+}
+
 // psi += alpha d of the last iteration that ran (its direction is in buffer
 // iter & 1 of the pair); nothing after a non-finite value or before any iteration
 __global__ void k_psi_last(size_t ncell, double* __restrict__ psi, const double* __restrict__ d0,
@@ -836,31 +956,6 @@ __global__ void k_resid_restrict(LevelDev<T> L, const TB* __restrict__ beta, con
             acc += (wx1 * wy1 * wz) * r11;
         }
         qc[I + (size_t)ncx * (J + (size_t)ncy * K)] = acc;
-    }
-}
-
-template <class T>
-struct Pair;
-template <>
-struct Pair<float> {
-    using type = float2;
-};
-template <>
-struct Pair<double> {
-    using type = double2;
-};
-
-// two neighbouring values of a row (a caller's beta may be aligned to its elements only)
-template <class T, class TS>
-__device__ __forceinline__ typename Pair<T>::type load_pair(const TS* __restrict__ a)
-{
-    if constexpr (std::is_same<TS, bf16s>::value) {
-        const uint32_t w = *reinterpret_cast<const uint32_t*>(a);
-        return typename Pair<T>::type{__builtin_bit_cast(float, w << 16), __builtin_bit_cast(float, w & 0xffff0000u)};
-    } else {
-        using V = T __attribute__((ext_vector_type(2), aligned(sizeof(T))));
-        const V v = *reinterpret_cast<const V*>(a);
-        return typename Pair<T>::type{v.x, v.y};
     }
 }
 
@@ -2122,6 +2217,13 @@ static unsigned red_blocks1(size_t n)
 // operator blocks: whole rows (up to 256 cells, so the x neighbours of a row
 // come from the same block), two rows, kOpPlanes planes per thread
 constexpr int kOpPlanes = 16;
+constexpr uint64_t kOpPointCells = (uint64_t)1 << 20;
+
+// multiplier of a 32-bit division by d (__umulhi), exact below 2^32 / d
+static uint32_t magic32(int d)
+{
+    return d <= 1 ? 0u : (uint32_t)((((uint64_t)1 << 32) + (uint64_t)d - 1) / (uint64_t)d);
+}
 
 static dim3 op_block(const LevelDev<double>& L)
 {
@@ -2139,6 +2241,12 @@ OpPlan op_plan(const LevelDev<double>& L)
 {
     OpPlan m;
     const char* env = std::getenv("TBFG_OP_TILE");
+    // pairs below 1 M cells whatever the tiles (the index divisions in 32 bits, as point_supported)
+    const uint64_t cells = (uint64_t)L.nx * L.ny * L.nz;
+    if (!env && L.nx % 2 == 0 && cells < kOpPointCells && cells / 2 * (uint64_t)std::max(L.nx / 2, L.ny) < ((uint64_t)1 << 32)) {
+        m.point = true;
+        m.pblocks = ceil_div((size_t)(cells / 2), 256);
+    }
     // 256-thread tiles first: with long marches they measured fastest (256x192x256:
     // 64x256 tiles 136 us, 32x256 138 us, 128x512 152 us, all with 64-plane chunks)
     std::vector<std::pair<int, int>> cand = {{64, 256}, {32, 256}, {128, 512}, {64, 512}};
@@ -2182,7 +2290,7 @@ size_t reduction_slots(const LevelDev<double>& L, const OpPlan& plan)
     const dim3 go = op_grid(L, op_block(L));
     const size_t chunked = (size_t)g3.x * g3.y * g3.z * 5;  // dots: 5 sums per block
     const size_t flat = (size_t)kRedBlocks * 5;
-    const size_t op = std::max((size_t)go.x * go.y * go.z, (size_t)plan.nblocks);
+    const size_t op = std::max((size_t)go.x * go.y * go.z, std::max((size_t)plan.nblocks, (size_t)plan.pblocks));
     // the sweep with the dot products on any tile shape: at most one workgroup
     // per 32x8 tile and 6-plane chunk
     const size_t sweep = (size_t)(L.nx / 32 + 1) * (L.ny / 8 + 1) * (L.nz / 6 + 1) * 5;
@@ -2192,6 +2300,13 @@ size_t reduction_slots(const LevelDev<double>& L, const OpPlan& plan)
 int launch_op_dot(const LevelDev<double>& L, const OpPlan& m, const double* beta, const double* d, double* qv,
                   PcgState* st, const Reducer& red, void* stream)
 {
+    if (m.point) {
+        hipLaunchKernelGGL((k_op_point<double, false>), dim3(m.pblocks), dim3(256), 0, S(stream), L, beta, d, qv, st, red,
+                           magic32(L.nx / 2), magic32(L.ny), (L.nx / 2) * L.ny * L.nz, OpDir<double>{});
+        hipLaunchKernelGGL(k_fin_alpha, dim3(1), dim3(1024), 0, S(stream), m.pblocks, st, red);
+        TBFG_HIP(hipGetLastError());
+        return TBFG_OK;
+    }
     if (m.tx) {
 #define TBFG_OPM(TX_, NT_)                                                                                          \
     if (m.tx == TX_ && m.nt == NT_)                                                                                 \
@@ -2221,6 +2336,19 @@ int launch_op_dir(const LevelDev<double>& L, const OpPlan& m, const double* beta
                   const KernelEvents* kev)
 {
     const OpDir<TZ> od{z, dold, dnew, psi, init};
+    if (m.point) {
+        const int pairs = (L.nx / 2) * L.ny * L.nz;
+        if (kev)
+            hipExtLaunchKernelGGL((k_op_point<TZ, true>), dim3(m.pblocks), dim3(256), 0, S(stream), kev->start,
+                                  kev->stop, 0, L, beta, nullptr, qv, st, red, magic32(L.nx / 2), magic32(L.ny), pairs,
+                                  od);
+        else
+            hipLaunchKernelGGL((k_op_point<TZ, true>), dim3(m.pblocks), dim3(256), 0, S(stream), L, beta, nullptr, qv, st,
+                               red, magic32(L.nx / 2), magic32(L.ny), pairs, od);
+        hipLaunchKernelGGL(k_fin_alpha, dim3(1), dim3(1024), 0, S(stream), m.pblocks, st, red);
+        TBFG_HIP(hipGetLastError());
+        return TBFG_OK;
+    }
     // (kev: events recorded by the dispatch of the pass itself, for timing it alone)
 #define TBFG_OPD(TX_, NT_)                                                                                         \
     if (m.tx == TX_ && m.nt == NT_) {                                                                              \

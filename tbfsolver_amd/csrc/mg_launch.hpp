@@ -11,6 +11,8 @@ namespace tbfg {
 struct OpPlan {
     int tx = 0, nt = 0, tiles_x = 0, ntiles = 0, kc = 0;
     unsigned nblocks = 0;
+    bool point = false;     // launch_op_dir by a thread per x pair (pblocks of 256) instead
+    unsigned pblocks = 0;
 };
 OpPlan op_plan(const LevelDev<double>& L);
 // doubles of reduction scratch the CG kernels of a level need (with its operator launch)
@@ -20,7 +22,7 @@ int launch_apply_op(const LevelDev<double>& L, const double* beta, const double*
 int launch_op_dot(const LevelDev<double>& L, const OpPlan& plan, const double* beta, const double* d, double* qv,
                   PcgState* st, const Reducer& red, void* stream);
 // the direction d = (z - m) + gamma d_old into dnew, qv = A d, d.qv and psi +=
-// alpha_prev d_old in one pass (plane-marching tiles: plan.tx != 0)
+// alpha_prev d_old in one pass (plan.point, or plane-marching tiles: plan.tx != 0)
 struct KernelEvents;
 template <class TZ>
 int launch_op_dir(const LevelDev<double>& L, const OpPlan& plan, const double* beta, const TZ* z, const double* dold,

@@ -428,7 +428,7 @@ int pcg_create(const tbfg_grid_desc* g, const tbfg_pcg_params* prm_in, tbfg_pcg*
     TBFG_TRY(h->qv.alloc(h->n0 * 8));
     TBFG_TRY(h->st.alloc(sizeof(PcgState)));
     h->opp = op_plan(h->tabd[0]->view);
-    h->fuse_op = h->opp.tx != 0 && !std::getenv("TBFG_UNFUSED_OP");
+    h->fuse_op = (h->opp.tx != 0 || h->opp.point) && !std::getenv("TBFG_UNFUSED_OP");
     if (h->fuse_op) TBFG_TRY(h->d2.alloc(h->n0 * 8));
     TBFG_TRY(h->partials.alloc(reduction_slots(h->tabd[0]->view, h->opp) * sizeof(double)));
     TBFG_TRY(h->counter.alloc(256));

@@ -147,3 +147,31 @@ def test_cycle_with_one_sweep_matches_oracle_at_remainders(torch_gpu, n):
     e = rel(out - out.mean(), ref - ref.mean())
     print("  rel error", e, flush=True)
     assert e < 1e-12
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("n", [(2, 4, 2), (4, 2, 6), (12, 10, 2), (66, 6, 4), (72, 40, 56), (256, 4, 8)])
+def test_pair_operator_matches_columns(torch_gpu, monkeypatch, n, precision):
+    """The direction, operator and pressure update by a thread per pair against the separate kernels with
+    the column operator (TBFG_OP_TILE=columns): the solves take the same iterations and agree to 1e-9, the
+    target of their residual being 1e-11; the caller's arrays aligned to their elements only."""
+    print("case pair operator", n, precision, flush=True)
+    g, beta, q = case(torch_gpu, n)
+
+    def shifted(t):
+        b = torch_gpu.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view(t.shape)
+        b.copy_(t)
+        return b
+
+    def solve(beta, psi):
+        s = T.PCG(g, nLevels=2, tolPCG=1e-11, maxIterPCG=200, flexible=1, coarse_max_iter=0, precision=precision)
+        s.solvePCG(psi, beta, q)
+        it = s.iterations
+        s.close()
+        return it, to_host(psi)
+
+    ia, a = solve(shifted(beta), shifted(torch_gpu.zeros_like(q)))
+    monkeypatch.setenv("TBFG_OP_TILE", "columns")
+    ib, b = solve(beta, torch_gpu.zeros_like(q))
+    print("  iterations", ia, ib, "rel", rel(a, b), flush=True)
+    assert abs(ia - ib) <= 1 and rel(a, b) < 1e-9
