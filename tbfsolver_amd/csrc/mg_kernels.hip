@@ -392,10 +392,13 @@ __device__ __forceinline__ typename Pair<T>::type load_pair(const TS* __restrict
 // the direction at the pair and its ten neighbours is formed from z and d_old there (the
 // rows beside a pair's own come from L1 and L2), every load issued at once.  A march of a few
 // planes is mostly its start and its barriers, and grids that no tile divides took a
-// separate direction kernel and columns of 16 planes.  Per launch: 393 K cells FP64
-// 13.8 -> 9.6 us, FP32 z 11.6 -> 7.3, 131 K 8.8 -> 4.4, 161 K (72x40x56) 13.1 -> 5.4.  Any even nx.
+// separate direction kernel and columns of 16 planes.  Per launch: 590 K cells FP64
+// 13.8 -> 9.6 us, FP32 z 393 K 11.6 -> 7.3, 131 K 8.8 -> 4.4, 161 K (72x40x56) 13.1 -> 5.4.
+// Any even nx.
+// 512 threads: the residual update reads a partial per workgroup, at most 1024.
+constexpr int kOpPointThreads = 512;
 template <class TZ, bool DIR>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(kOpPointThreads)
     k_op_point(LevelDev<double> L, const double* __restrict__ beta, const double* __restrict__ din,
                double* __restrict__ qv, const PcgState* st, Reducer red, uint32_t m_hx, uint32_t m_ny, int npairs,
                OpDir<TZ> od)
@@ -403,7 +406,7 @@ __global__ void __launch_bounds__(256)
     if (st->done) return;
     unsigned id = blockIdx.x;  // consecutive blocks on one XCD
     if ((gridDim.x & 7u) == 0) id = (id & 7u) * (gridDim.x >> 3) + (id >> 3);
-    const int tp = (int)(id * 256u + threadIdx.x);
+    const int tp = (int)(id * (unsigned)kOpPointThreads + threadIdx.x);
     const bool own = tp < npairs;  // (the last block's idle threads follow the last pair)
     const int t = own ? tp : npairs - 1;
     const int nx = L.nx, ny = L.ny, nz = L.nz, hx = nx >> 1;
@@ -494,26 +497,6 @@ __global__ void k_psi_last(size_t ncell, double* __restrict__ psi, const double*
     const double* d = (it & 1) ? d1 : d0;
     const size_t stride = (size_t)gridDim.x * blockDim.x;
     for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < ncell; t += stride) psi[t] = psi[t] + alpha * d[t];
-}
-
-__global__ void k_fin_alpha(unsigned nblocks, PcgState* st, Reducer red)
-{
-    // (the state and the partials are loaded together, here and in the kernels below: each
-    // wait of a one-block kernel is some 0.7 us of nothing else)
-    const int done = st->done;
-    const double delta = st->delta;
-    double tot[1];
-    final_sum<1>(red, nblocks, tot);
-    if (threadIdx.x == 0 && !done) {
-        const double den = tot[0];
-        if (!(den != 0.0) || !isfinite(den) || !isfinite(delta)) {
-            st->done = 1;
-            st->status = TBFG_ENUMERIC;
-            st->alpha = 0.0;
-        } else {
-            st->alpha = delta / den;
-        }
-    }
 }
 
 // r = q - A psi with ||r||^2, ||q||^2 (computeResiduals, rbgs.f90:276-333, used at pcg.f90:116).
@@ -701,17 +684,37 @@ __global__ void k_fin_init(unsigned nblocks, PcgState* st, Reducer red)
 }
 
 // psi += alpha d; r -= alpha qv; ||r|| and the stop test (pcg.f90:228-262,331-355,359-429).
+// alpha = delta / d.Ad first, by every workgroup from the operator pass's nop partials (in one
+// order, so all find the same value): a finalize kernel of its own took 3 to 4.5 us, where
+// the sum here costs 1 to 2.
 template <class TR>
-__global__ void k_pcg_update(size_t ncell, double* __restrict__ psi, double* __restrict__ r, TR* __restrict__ r32,
-                             const double* __restrict__ d, const double* __restrict__ qv, PcgState* st, Reducer red)
+__global__ void __launch_bounds__(256)
+    k_pcg_update(size_t ncell, double* __restrict__ psi, double* __restrict__ r, TR* __restrict__ r32,
+                 const double* __restrict__ d, const double* __restrict__ qv, PcgState* st,
+                 const double* __restrict__ pop, unsigned nop, Reducer red)
 {
     if (st->done) return;
-    const double alpha = st->alpha;
+    const double delta = st->delta;
+    const size_t stride = (size_t)gridDim.x * blockDim.x, t0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    // the first cell's values in flight meanwhile
+    const size_t c0 = t0 < ncell ? t0 : 0;
+    double rc = r[c0], qc = qv[c0];
+    const double den = sum_by_1024(pop, nop);
+    const bool bad = !(den != 0.0) || !isfinite(den) || !isfinite(delta);
+    const double alpha = bad ? 0.0 : delta / den;
+    if (t0 == 0) {
+        if (bad) {
+            st->done = 1;
+            st->status = TBFG_ENUMERIC;
+        }
+        st->alpha = alpha;
+    }
+    if (bad) return;
     double v[1] = {0.0};
-    const size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < ncell; t += stride) {
+    for (size_t t = t0; t < ncell; t += stride) {
+        if (t != t0) rc = r[t], qc = qv[t];
         if (psi) psi[t] = psi[t] + alpha * d[t];  // (NULL: deferred to the next operator pass)
-        const double rn = r[t] - alpha * qv[t];
+        const double rn = rc - alpha * qc;
         r[t] = rn;
         if (r32) r32[t] = store_as<TR>((float)rn);
         v[0] += rn * rn;
@@ -719,29 +722,7 @@ __global__ void k_pcg_update(size_t ncell, double* __restrict__ psi, double* __r
     block_partial<1>(v, red);
 }
 
-__global__ void k_fin_update(unsigned nblocks, PcgState* st, Reducer red)
-{
-    const int done = st->done, iter = st->iter + 1, max_iter = st->max_iter;
-    const double qq = st->qq, tol = st->tol;
-    double tot[1];
-    final_sum<1>(red, nblocks, tot);
-    if (threadIdx.x == 0 && !done) {
-        st->rr = tot[0];
-        st->iter = iter;
-        const double res = sqrt(tot[0]) / sqrt(qq + 2.2250738585072014e-308);
-        st->res = res;
-        if (!isfinite(res)) {
-            st->done = 1;
-            st->status = TBFG_ENUMERIC;
-        } else if (res <= tol) {
-            st->done = 1;
-            st->status = TBFG_OK;
-        } else if (iter >= max_iter) {
-            st->done = 1;
-            st->status = TBFG_ENOTCONVERGED;
-        }
-    }
-}
+__global__ void __launch_bounds__(256) k_fin_update(FinUpdate f) { fin_update(f); }
 
 // r.z, qv.z, sum z, sum r, sum qv in one pass; the preconditioned residual is
 // used with its arithmetic mean removed (rbgs.f90:403-446 leaves z mean-free):
@@ -961,8 +942,8 @@ __global__ void k_resid_restrict(LevelDev<T> L, const TB* __restrict__ beta, con
 
 // The same, a thread per coarse cell with its 16 rows of p and beta and 8 of q loaded at once:
 // a small level's time is the rounds of loads that wait for one another (four of them
-// above), not its bytes.  Per launch, FP64: 2 M cells 10.9 -> 10.3 us, 393 K 7.0 -> 5.7, 49 K
-// 6.7 -> 4.4, 6 K 6.8 -> 3.7; FP32: 1.6 M 8.6 -> 7.5, 161 K 6.7 -> 4.3.  Above 2 M cells, where
+// above), not its bytes.  Per launch, FP64: 2 M cells 10.9 -> 10.3 us, 590 K 7.0 -> 5.7, 74 K
+// 6.7 -> 4.4, 9 K 6.8 -> 3.7; FP32: 1.6 M 8.6 -> 7.5, 161 K 6.7 -> 4.3.  Above 2 M cells, where
 // the planes it reads twice count (12.6 M cells in bf16: 26.9 and 29.2 us), the segments stay.
 template <class T, class TQ, class TB>
 __global__ void __launch_bounds__(256)
@@ -1080,7 +1061,7 @@ __device__ __forceinline__ void prolong_cell(const LV& L, int ncx, int ncy, int 
 }
 
 // One thread per coarse cell: its 2x2x2 fine children all interpolate from the
-// 3x3x3 coarse neighbourhood, loaded once together with p and the weights (FP64, 6 K cells:
+// 3x3x3 coarse neighbourhood, loaded once together with p and the weights (FP64, 9 K cells:
 // 4.4 -> 3.5 us, 2 M 9.3 -> 8.8; the weights and the order of the
 // arithmetic are prolong_cell's), and each pair of x-children is one vector
 // access.
@@ -2245,7 +2226,7 @@ OpPlan op_plan(const LevelDev<double>& L)
     const uint64_t cells = (uint64_t)L.nx * L.ny * L.nz;
     if (!env && L.nx % 2 == 0 && cells < kOpPointCells && cells / 2 * (uint64_t)std::max(L.nx / 2, L.ny) < ((uint64_t)1 << 32)) {
         m.point = true;
-        m.pblocks = ceil_div((size_t)(cells / 2), 256);
+        m.pblocks = ceil_div((size_t)(cells / 2), kOpPointThreads);
     }
     // 256-thread tiles first: with long marches they measured fastest (256x192x256:
     // 64x256 tiles 136 us, 32x256 138 us, 128x512 152 us, all with 64-plane chunks)
@@ -2298,12 +2279,12 @@ size_t reduction_slots(const LevelDev<double>& L, const OpPlan& plan)
 }
 
 int launch_op_dot(const LevelDev<double>& L, const OpPlan& m, const double* beta, const double* d, double* qv,
-                  PcgState* st, const Reducer& red, void* stream)
+                  PcgState* st, const Reducer& red, unsigned* nop, void* stream)
 {
     if (m.point) {
-        hipLaunchKernelGGL((k_op_point<double, false>), dim3(m.pblocks), dim3(256), 0, S(stream), L, beta, d, qv, st, red,
+        hipLaunchKernelGGL((k_op_point<double, false>), dim3(m.pblocks), dim3(kOpPointThreads), 0, S(stream), L, beta, d, qv, st, red,
                            magic32(L.nx / 2), magic32(L.ny), (L.nx / 2) * L.ny * L.nz, OpDir<double>{});
-        hipLaunchKernelGGL(k_fin_alpha, dim3(1), dim3(1024), 0, S(stream), m.pblocks, st, red);
+        *nop = m.pblocks;
         TBFG_HIP(hipGetLastError());
         return TBFG_OK;
     }
@@ -2317,7 +2298,7 @@ int launch_op_dot(const LevelDev<double>& L, const OpPlan& m, const double* beta
             return TBFG_EINVAL;
         }
 #undef TBFG_OPM
-        hipLaunchKernelGGL(k_fin_alpha, dim3(1), dim3(1024), 0, S(stream), m.nblocks, st, red);
+        *nop = m.nblocks;
         TBFG_HIP(hipGetLastError());
         return TBFG_OK;
     }
@@ -2325,27 +2306,27 @@ int launch_op_dot(const LevelDev<double>& L, const OpPlan& m, const double* beta
     dim3 grd = op_grid(L, blk);
     const unsigned nb = grd.x * grd.y * grd.z;
     hipLaunchKernelGGL(k_op_dot<kOpPlanes>, dim3(nb), blk, 0, S(stream), L, beta, d, qv, st, red);
-    hipLaunchKernelGGL(k_fin_alpha, dim3(1), dim3(1024), 0, S(stream), nb, st, red);
+    *nop = nb;
     TBFG_HIP(hipGetLastError());
     return TBFG_OK;
 }
 
 template <class TZ>
 int launch_op_dir(const LevelDev<double>& L, const OpPlan& m, const double* beta, const TZ* z, const double* dold,
-                  double* dnew, double* psi, int init, double* qv, PcgState* st, const Reducer& red, void* stream,
-                  const KernelEvents* kev)
+                  double* dnew, double* psi, int init, double* qv, PcgState* st, const Reducer& red, unsigned* nop,
+                  void* stream, const KernelEvents* kev)
 {
     const OpDir<TZ> od{z, dold, dnew, psi, init};
     if (m.point) {
         const int pairs = (L.nx / 2) * L.ny * L.nz;
         if (kev)
-            hipExtLaunchKernelGGL((k_op_point<TZ, true>), dim3(m.pblocks), dim3(256), 0, S(stream), kev->start,
+            hipExtLaunchKernelGGL((k_op_point<TZ, true>), dim3(m.pblocks), dim3(kOpPointThreads), 0, S(stream), kev->start,
                                   kev->stop, 0, L, beta, nullptr, qv, st, red, magic32(L.nx / 2), magic32(L.ny), pairs,
                                   od);
         else
-            hipLaunchKernelGGL((k_op_point<TZ, true>), dim3(m.pblocks), dim3(256), 0, S(stream), L, beta, nullptr, qv, st,
+            hipLaunchKernelGGL((k_op_point<TZ, true>), dim3(m.pblocks), dim3(kOpPointThreads), 0, S(stream), L, beta, nullptr, qv, st,
                                red, magic32(L.nx / 2), magic32(L.ny), pairs, od);
-        hipLaunchKernelGGL(k_fin_alpha, dim3(1), dim3(1024), 0, S(stream), m.pblocks, st, red);
+        *nop = m.pblocks;
         TBFG_HIP(hipGetLastError());
         return TBFG_OK;
     }
@@ -2365,15 +2346,15 @@ int launch_op_dir(const LevelDev<double>& L, const OpPlan& m, const double* beta
         return TBFG_EINVAL;
     }
 #undef TBFG_OPD
-    hipLaunchKernelGGL(k_fin_alpha, dim3(1), dim3(1024), 0, S(stream), m.nblocks, st, red);
+    *nop = m.nblocks;
     TBFG_HIP(hipGetLastError());
     return TBFG_OK;
 }
 template int launch_op_dir<float>(const LevelDev<double>&, const OpPlan&, const double*, const float*, const double*,
-                                  double*, double*, int, double*, PcgState*, const Reducer&, void*,
+                                  double*, double*, int, double*, PcgState*, const Reducer&, unsigned*, void*,
                                   const KernelEvents*);
 template int launch_op_dir<double>(const LevelDev<double>&, const OpPlan&, const double*, const double*,
-                                   const double*, double*, double*, int, double*, PcgState*, const Reducer&, void*,
+                                   const double*, double*, double*, int, double*, PcgState*, const Reducer&, unsigned*, void*,
                                    const KernelEvents*);
 
 int launch_state_init(PcgState* st, double tol, int32_t max_iter, int32_t flexible, void* stream)
@@ -2418,11 +2399,19 @@ int launch_residual_init(const LevelDev<double>& L, const OpPlan& m, const doubl
 
 template <class TR>
 int launch_pcg_update(size_t n, double* psi, double* r, TR* r32, const double* d, const double* qv,
-                      PcgState* st, const Reducer& red, void* stream)
+                      PcgState* st, const Reducer& op, unsigned nop, const Reducer& red, FinUpdate* fin, void* stream)
 {
-    const unsigned nb = red_blocks1(n);
-    hipLaunchKernelGGL(k_pcg_update<TR>, dim3(nb), dim3(256), 0, S(stream), n, psi, r, r32, d, qv, st, red);
-    hipLaunchKernelGGL(k_fin_update, dim3(1), dim3(256), 0, S(stream), nb, st, red);
+    // two cells a thread: half as many workgroups sum the operator's partials
+    const unsigned nb = std::min<unsigned>(ceil_div(n, 512), kRedBlocks);
+    hipLaunchKernelGGL(k_pcg_update<TR>, dim3(nb), dim3(256), 0, S(stream), n, psi, r, r32, d, qv, st, op.partials, nop,
+                       red);
+    TBFG_HIP(hipGetLastError());
+    *fin = FinUpdate{st, red.partials, nb};
+    return TBFG_OK;
+}
+int launch_fin_update(const FinUpdate& f, void* stream)
+{
+    hipLaunchKernelGGL(k_fin_update, dim3(1), dim3(256), 0, S(stream), f);
     TBFG_HIP(hipGetLastError());
     return TBFG_OK;
 }
@@ -2571,9 +2560,9 @@ template int launch_residual_init<float>(const LevelDev<double>&, const OpPlan&,
 template int launch_residual_init<bf16s>(const LevelDev<double>&, const OpPlan&, const double*, const double*,
                                          const double*, double*, bf16s*, PcgState*, const Reducer&, void*);
 template int launch_pcg_update<float>(size_t, double*, double*, float*, const double*, const double*, PcgState*,
-                                      const Reducer&, void*);
+                                      const Reducer&, unsigned, const Reducer&, FinUpdate*, void*);
 template int launch_pcg_update<bf16s>(size_t, double*, double*, bf16s*, const double*, const double*, PcgState*,
-                                      const Reducer&, void*);
+                                      const Reducer&, unsigned, const Reducer&, FinUpdate*, void*);
 template int launch_tail<double>(const TailPlan<double>*, size_t, int, const int*, size_t, void*);
 template int launch_tail<float>(const TailPlan<float>*, size_t, int, const int*, size_t, void*);
 

@@ -97,6 +97,14 @@ struct Reducer {
     double* partials;    // >= blocks * NV
 };
 
+// the residual norm's partials and the stop test that they end in (fin_update): carried out by
+// a workgroup of the next sweep, or by a launch of its own
+struct FinUpdate {
+    PcgState* st = nullptr;
+    const double* partials = nullptr;
+    unsigned n = 0;  // 0: nothing to do
+};
+
 template <class T>
 struct TailLevel {
     LevelDev<T> geo;

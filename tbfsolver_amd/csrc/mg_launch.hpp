@@ -11,7 +11,7 @@ namespace tbfg {
 struct OpPlan {
     int tx = 0, nt = 0, tiles_x = 0, ntiles = 0, kc = 0;
     unsigned nblocks = 0;
-    bool point = false;     // launch_op_dir by a thread per x pair (pblocks of 256) instead
+    bool point = false;     // launch_op_dir by a thread per x pair (pblocks workgroups) instead
     unsigned pblocks = 0;
 };
 OpPlan op_plan(const LevelDev<double>& L);
@@ -20,14 +20,14 @@ size_t reduction_slots(const LevelDev<double>& L, const OpPlan& plan);
 
 int launch_apply_op(const LevelDev<double>& L, const double* beta, const double* p, double* q, void* stream);
 int launch_op_dot(const LevelDev<double>& L, const OpPlan& plan, const double* beta, const double* d, double* qv,
-                  PcgState* st, const Reducer& red, void* stream);
+                  PcgState* st, const Reducer& red, unsigned* nop, void* stream);
 // the direction d = (z - m) + gamma d_old into dnew, qv = A d, d.qv and psi +=
 // alpha_prev d_old in one pass (plan.point, or plane-marching tiles: plan.tx != 0)
 struct KernelEvents;
 template <class TZ>
 int launch_op_dir(const LevelDev<double>& L, const OpPlan& plan, const double* beta, const TZ* z, const double* dold,
-                  double* dnew, double* psi, int init, double* qv, PcgState* st, const Reducer& red, void* stream,
-                  const KernelEvents* kev = nullptr);
+                  double* dnew, double* psi, int init, double* qv, PcgState* st, const Reducer& red, unsigned* nop,
+                  void* stream, const KernelEvents* kev = nullptr);
 // psi += alpha d of the last iteration that ran (d in d0 or d1 by its parity)
 int launch_psi_last(size_t n, double* psi, const double* d0, const double* d1, const PcgState* st, void* stream);
 // the state of a new solve: zero but tol, max_iter and flexible
@@ -39,7 +39,9 @@ int launch_residual_init(const LevelDev<double>& L, const OpPlan& plan, const do
                          const double* psi, double* r, TR* r32, PcgState* st, const Reducer& red, void* stream);
 template <class TR>
 int launch_pcg_update(size_t n, double* psi, double* r, TR* r32, const double* d, const double* qv,
-                      PcgState* st, const Reducer& red, void* stream);
+                      PcgState* st, const Reducer& op, unsigned nop, const Reducer& red, FinUpdate* fin, void* stream);
+// the stop test that launch_pcg_update leaves in *fin
+int launch_fin_update(const FinUpdate& f, void* stream);
 template <class TZ>
 int launch_pcg_dots(size_t n, const double* r, const TZ* z, const double* qv, int init, PcgState* st,
                     const Reducer& red, int32_t* host_done, void* stream);
@@ -58,6 +60,7 @@ struct SweepDots {
     int init = 0;
     Reducer red{nullptr};
     size_t capacity = 0;  // doubles of red.partials
+    FinUpdate fin{};      // with r NULL, in a sweep from zero: the stop test, by a workgroup more
 };
 // events that a timed launch records around the kernel itself (the
 // dispatch's own begin and end, hipExtLaunchKernel)

@@ -430,7 +430,8 @@ int pcg_create(const tbfg_grid_desc* g, const tbfg_pcg_params* prm_in, tbfg_pcg*
     h->opp = op_plan(h->tabd[0]->view);
     h->fuse_op = (h->opp.tx != 0 || h->opp.point) && !std::getenv("TBFG_UNFUSED_OP");
     if (h->fuse_op) TBFG_TRY(h->d2.alloc(h->n0 * 8));
-    TBFG_TRY(h->partials.alloc(reduction_slots(h->tabd[0]->view, h->opp) * sizeof(double)));
+    // (two halves: the residual update reads the operator's partials and writes its own)
+    TBFG_TRY(h->partials.alloc(2 * reduction_slots(h->tabd[0]->view, h->opp) * sizeof(double)));
     TBFG_TRY(h->counter.alloc(256));
     TBFG_TRY(memset_sync(h->counter.p, 0, 256));
     // dense bottom operator
@@ -532,12 +533,14 @@ static int setup_levels(tbfg_pcg* h, const double* beta0, void* stream)
 // starts from p = 0.  Levels with the full-sweep kernel alternate between
 // their two buffers, so p (and alt) may be swapped on return.
 // last_dots: the dot products of the PCG are formed by the last sweep (see
-// launch_sweep); *nb_out receives its partial count.
+// launch_sweep); *nb_out receives its partial count.  fin: the stop test that the first sweep
+// carries out too (folds_stop_test).
 // (T0: the storage type of the level's q and beta, T or bf16s; bf16s only
 // where the plane march smooths the level)
 template <class T, class T0 = T>
 static int smooth(tbfg_pcg* h, int l, const T0* b, const T0* q, T*& p, T*& alt, int nsweeps, bool first,
-                  const int* done, void* stream, const SweepDots* last_dots = nullptr, unsigned* nb_out = nullptr)
+                  const int* done, void* stream, const SweepDots* last_dots = nullptr, unsigned* nb_out = nullptr,
+                  const SweepDots* fin = nullptr)
 {
     const LevelDev<T>& L = geo<T>(h, l);
     constexpr bool narrow = !std::is_same<T0, T>::value;
@@ -549,6 +552,7 @@ static int smooth(tbfg_pcg* h, int l, const T0* b, const T0* q, T*& p, T*& alt, 
         const bool f0 = first && s == 0;
         const bool last = s == nsweeps - 1;
         const SweepDots* dots = last ? last_dots : nullptr;
+        const SweepDots* with = f0 && fin ? fin : dots;
         unsigned* nb = last ? nb_out : nullptr;
         if (h->fused[l] == 1 || h->fused[l] == 3) {
             // the timed finest-level sweep: from a non-zero start, without the dot products
@@ -561,13 +565,13 @@ static int smooth(tbfg_pcg* h, int l, const T0* b, const T0* q, T*& p, T*& alt, 
             if (h->fused[l] == 1 && (!row_supported<T>(L) || sweep_named<T>(L, !f0 && !dots) || (h->b16 && dots)))
                 TBFG_TRY(launch_sweep<T, T0, T0>(L, b, q, p, alt, f0, done, stream, dots, nb, ps.events()));
             else
-                TBFG_TRY(launch_row_sweep<T, T0, T0>(L, b, q, p, alt, f0, h->b16 && h->fused[l] == 1, done, stream, dots,
+                TBFG_TRY(launch_row_sweep<T, T0, T0>(L, b, q, p, alt, f0, h->b16 && h->fused[l] == 1, done, stream, with,
                                                      nb, ps.events()));
             std::swap(p, alt);
         } else if constexpr (!narrow) {
             ProfScope ps(h, l == 0 ? 0 : -1, stream);
             if (h->fused[l] == 2) {
-                TBFG_TRY(launch_point_sweep<T, T>(L, b, q, p, alt, f0, done, stream, dots, nb));
+                TBFG_TRY(launch_point_sweep<T, T>(L, b, q, p, alt, f0, done, stream, with, nb));
                 std::swap(p, alt);
             } else {
                 TBFG_TRY(launch_rbgs<T, T>(L, b, q, p, RED, f0, done, stream));
@@ -576,6 +580,19 @@ static int smooth(tbfg_pcg* h, int l, const T0* b, const T0* q, T*& p, T*& alt, 
         }
     }
     return TBFG_OK;
+}
+
+// Whether the finest level's sweep from zero can carry out the stop test of the iteration
+// before (a workgroup more of it): k_point_sweep and k_row_sweep do.  The sweep itself then
+// runs once more after convergence; a launch of its own for the test took 4.5 us of every
+// iteration.
+template <class T>
+static bool folds_stop_test(const tbfg_pcg* h)
+{
+    const LevelDev<T>& L = geo<T>(const_cast<tbfg_pcg*>(h), 0);
+    if (h->prm.n_pre < 1 || (h->kin >= 0 ? h->kin : h->t0) < 1) return false;
+    if (h->fused[0] == 1) return row_supported<T>(L) && !sweep_named<T>(L, false);
+    return h->fused[0] == 2 || h->fused[0] == 3;
 }
 
 // The inner V-cycle of the coarsest-level solve on level kin (the tail's
@@ -675,7 +692,8 @@ static int inner_solve(tbfg_pcg* h, void* stream)
 // tells whether it could.
 template <class T, class T0 = T>
 static int vcycle(tbfg_pcg* h, const T0* r0, T** z, const T0* beta0, const int* done, void* stream,
-                  int dots_init = -1, bool* dots_done = nullptr, int32_t* host_done = nullptr)
+                  int dots_init = -1, bool* dots_done = nullptr, int32_t* host_done = nullptr,
+                  const FinUpdate* fin = nullptr)
 {
     if (dots_done) *dots_done = false;
     // solveMG's loop (mg_tol > 0): after every cycle the finest residual is
@@ -693,7 +711,7 @@ static int vcycle(tbfg_pcg* h, const T0* r0, T** z, const T0* beta0, const int* 
         sd.qv = h->qv.as<double>();
         sd.init = dots_init;
         sd.red = Reducer{h->partials.as<double>()};
-        sd.capacity = h->partials.bytes / sizeof(double);
+        sd.capacity = h->partials.bytes / sizeof(double) / 2;
     }
     // levels smoothed here; below them the tail, or the multi-workgroup solve of level kin
     const int t0 = h->kin >= 0 ? h->kin : h->t0;
@@ -713,7 +731,10 @@ static int vcycle(tbfg_pcg* h, const T0* r0, T** z, const T0* beta0, const int* 
             if (h->prm.n_pre == 0 && first)
                 TBFG_HIP(hipMemsetAsync(cur[l], 0, h->hl[l].cells() * sizeof(T), (hipStream_t)stream));
             if (l == 0) {
-                TBFG_TRY(smooth<T, T0>(h, 0, beta0, r0, cur[0], alt[0], h->prm.n_pre, first, done, stream));
+                SweepDots sf;
+                if (fin) sf.fin = *fin;
+                TBFG_TRY(smooth<T, T0>(h, 0, beta0, r0, cur[0], alt[0], h->prm.n_pre, first, done, stream, nullptr,
+                                       nullptr, fin ? &sf : nullptr));
                 ProfScope ps(h, 1, stream);
                 TBFG_TRY(launch_resid_restrict<T, T0, T0>(geo<T>(h, 0), beta0, r0, cur[0], h->q[1].as<T>(), done,
                                                           stream));
@@ -840,22 +861,25 @@ static int solve_t(tbfg_pcg* h, double* psi, const double* beta, const double* q
         r0 = r32;
     else
         r0 = r;
+    const Reducer red2{red.partials + h->partials.bytes / sizeof(double) / 2};
+    bool fold = false;
+    if constexpr (!FFT) fold = folds_stop_test<T>(h);
     // z = M r and the dot products of z (pcg.f90:118-139, 294-327)
     bool dots_done = false;
-    auto precondition = [&](int init, int32_t* host_done) -> int {
+    auto precondition = [&](int init, int32_t* host_done, const FinUpdate* fin) -> int {
         if constexpr (FFT) {
             z = h->zfft.as<double>();
             TBFG_TRY(fps_solve_dev(h->fps, r, z, stream));
             TBFG_TRY(launch_pcg_dots<double>(n, r, z, qv, init, st, red, host_done, stream));
         } else {
             TBFG_TRY(vcycle<T, T0>(h, r0, &z, beta0, done, stream, h->fuse_dots ? init : -1, &dots_done,
-                                   host_done));
+                                   host_done, fin));
             if (!dots_done) TBFG_TRY(launch_pcg_dots<T>(n, r, z, qv, init, st, red, host_done, stream));
         }
         return TBFG_OK;
     };
     TBFG_TRY(launch_residual_init(L0, h->opp, beta, q, psi, r, r32, st, red, stream));
-    TBFG_TRY(precondition(1, queue > 0 ? nullptr : &h->hring[0].done));
+    TBFG_TRY(precondition(1, queue > 0 ? nullptr : &h->hring[0].done, nullptr));
     // one iteration (pcg.f90:142-290): d = (z - m) + gamma d, qv = A d, alpha,
     // psi += alpha d, r -= alpha qv, the stop test, z = M r, the dot products.
     // Fused form: iteration j writes its direction to dbuf[j & 1] from
@@ -865,25 +889,28 @@ static int solve_t(tbfg_pcg* h, double* psi, const double* beta, const double* q
     int j = 0;
     auto iteration = [&](int init, int32_t* host_done) -> int {
         ++j;
+        unsigned nop = 0;
+        FinUpdate fin;
         if (h->fuse_op) {
             double* dj = dbuf[j & 1];
             {
                 ProfScope ps(h, 2, stream, true);  // the operator pass alone (not its finalize)
                 TBFG_TRY(launch_op_dir<TZ>(L0, h->opp, beta, z, dbuf[(j - 1) & 1], dj, psi, init, qv, st, red,
-                                           stream, ps.events()));
+                                           &nop, stream, ps.events()));
             }
             ProfScope ps(h, 3, stream);
-            TBFG_TRY(launch_pcg_update(n, nullptr, r, r32, dj, qv, st, red, stream));
+            TBFG_TRY(launch_pcg_update(n, nullptr, r, r32, dj, qv, st, red, nop, red2, &fin, stream));
         } else {
             TBFG_TRY(launch_pcg_dir<TZ>(n, z, d, init, st, stream));
             {
                 ProfScope ps(h, 2, stream);
-                TBFG_TRY(launch_op_dot(L0, h->opp, beta, d, qv, st, red, stream));
+                TBFG_TRY(launch_op_dot(L0, h->opp, beta, d, qv, st, red, &nop, stream));
             }
             ProfScope ps(h, 3, stream);
-            TBFG_TRY(launch_pcg_update(n, psi, r, r32, d, qv, st, red, stream));
+            TBFG_TRY(launch_pcg_update(n, psi, r, r32, d, qv, st, red, nop, red2, &fin, stream));
         }
-        TBFG_TRY(precondition(0, host_done));
+        if (!fold) TBFG_TRY(launch_fin_update(fin, stream));
+        TBFG_TRY(precondition(0, host_done, fold ? &fin : nullptr));
         return TBFG_OK;
     };
     // The stop flag after each iteration goes to a pinned slot from the kernel that ends it

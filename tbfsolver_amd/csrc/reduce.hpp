@@ -81,6 +81,73 @@ __device__ __forceinline__ void final_sum(const Reducer& red, unsigned nblocks, 
         for (int q = 0; q < NV; ++q) tot[q] = acc[q];
 }
 
+// The sum of n partials in every thread of a 256-thread workgroup, in the order in which 1024
+// threads and their 16 wavefronts add them.
+__device__ __forceinline__ double sum_by_1024(const double* __restrict__ partials, unsigned n)
+{
+    __shared__ double lds[16];
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    for (unsigned b = 0; b < n; b += 1024) {
+        double x[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const unsigned e = b + u * 256 + threadIdx.x;
+            x[u] = partials[e < n ? e : 0];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) acc[u] += b + u * 256 + threadIdx.x < n ? x[u] : 0.0;
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) acc[u] += __shfl_down(acc[u], off, 64);
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) lds[4 * u + (threadIdx.x >> 6)] = acc[u];
+    __syncthreads();
+    double s = 0.0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) s += lds[w];
+    return s;
+}
+
+// ||r|| and the stop test (pcg.f90:331-355,359-429), by one workgroup of at least 256 threads
+__device__ __forceinline__ void fin_update(const FinUpdate& f)
+{
+    __shared__ double lds[32];
+    PcgState* st = f.st;
+    const int done = st->done, iter = st->iter + 1, max_iter = st->max_iter;
+    const double qq = st->qq, tol = st->tol;
+    double tot[1] = {0.0};
+    for (unsigned b0 = 0; b0 < f.n; b0 += 2048) {  // the order of 256 threads
+        double x[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const unsigned e = b0 + u * 256 + threadIdx.x;
+            x[u] = f.partials[e < f.n ? e : 0];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) tot[0] += threadIdx.x < 256 && b0 + u * 256 + threadIdx.x < f.n ? x[u] : 0.0;
+    }
+    block_sum<1>(tot, lds);
+    if (threadIdx.x == 0 && !done) {
+        st->rr = tot[0];
+        st->iter = iter;
+        const double res = sqrt(tot[0]) / sqrt(qq + 2.2250738585072014e-308);
+        st->res = res;
+        if (!isfinite(res)) {
+            st->done = 1;
+            st->status = TBFG_ENUMERIC;
+        } else if (res <= tol) {
+            st->done = 1;
+            st->status = TBFG_OK;
+        } else if (iter >= max_iter) {
+            st->done = 1;
+            st->status = TBFG_ENOTCONVERGED;
+        }
+    }
+}
+
 // The scalars of the next direction from the sums of the dot products (pcg.f90:294-327), by
 // one workgroup.  host_done (pinned host memory, may be NULL) receives the stop flag: the
 // host's stop test of the iteration that ends here, without a copy in the stream.

@@ -466,8 +466,15 @@ __global__ void __launch_bounds__(256)
                   T* __restrict__ pout, uint32_t m_hx, uint32_t m_ny, int npairs, const int* done, SweepDots dots)
 {
     if (done && *done) return;
-    unsigned id = blockIdx.x;  // consecutive blocks on one XCD
-    if ((gridDim.x & 7u) == 0) id = (id & 7u) * (gridDim.x >> 3) + (id >> 3);
+    unsigned id = blockIdx.x, nblk = gridDim.x;  // consecutive blocks on one XCD
+    if (FIRST && dots.fin.n) {
+        if (id == 0) {
+            fin_update(dots.fin);
+            return;
+        }
+        --id, --nblk;
+    }
+    if ((nblk & 7u) == 0) id = (id & 7u) * (nblk >> 3) + (id >> 3);
     const int tp = (int)(id * 256u + threadIdx.x);
     const bool own = tp < npairs;  // (the last block's idle threads follow the last pair)
     const int t = own ? tp : npairs - 1;
@@ -518,7 +525,7 @@ __global__ void __launch_bounds__(256)
     const T zpf = half * L.a[2].ip[kf], zmf = half * L.a[2].im[kf], zpb = half * L.a[2].ip[kb], zmb = half * L.a[2].im[kb];
 
     // every load above before the arithmetic: the compiler otherwise saves registers by
-    // loading in rounds that each wait (FP64, 49 K cells: 5.4 -> 4.9 us)
+    // loading in rounds that each wait (FP64, 74 K cells: 5.4 -> 4.9 us)
     __builtin_amdgcn_sched_barrier(0);
 
     const std::true_type red;
@@ -642,8 +649,15 @@ __global__ void __launch_bounds__(64 * (row_waves<T>() + 2))
     constexpr int kSlot = 2 * 64 * (NW + 2);
     __shared__ T sR[(TILES ? 4 : 2) * kSlot];  // red values, rows -1 .. NW rw of 2 lr; as seen across a tile's edge
     if (done && *done) return;
-    unsigned id = blockIdx.x;  // consecutive tiles of a chunk on one XCD
-    if ((gridDim.x & 7u) == 0) id = (id & 7u) * (gridDim.x >> 3) + (id >> 3);
+    unsigned id = blockIdx.x, nblk = gridDim.x;  // consecutive tiles of a chunk on one XCD
+    if (FIRST && dots.fin.n) {
+        if (id == 0) {
+            fin_update(dots.fin);
+            return;
+        }
+        --id, --nblk;
+    }
+    if ((nblk & 7u) == 0) id = (id & 7u) * (nblk >> 3) + (id >> 3);
     const int nx = L.nx, ny = L.ny, nz = L.nz;
     const int k0 = (int)(id / (unsigned)ntiles) * kc, k1 = min(nz, k0 + kc);
     const int ty0 = (int)(id % (unsigned)ntiles) * NW * rw;
@@ -856,21 +870,23 @@ template <class T, class TQ>
 int launch_point_sweep(const LevelDev<T>& L, const T* beta, const TQ* q, const T* pin, T* pout, bool first,
                        const int* done, void* stream, const SweepDots* dots, unsigned* nblocks_out)
 {
-    if (!point_supported(L) || (dots && first)) {
+    const bool wd = dots && dots->r;
+    if (!point_supported(L) || (wd && first)) {
         set_error("launch_point_sweep: level %dx%dx%d not supported", L.nx, L.ny, L.nz);
         return TBFG_EINVAL;
     }
     auto magic = [](int d) { return d <= 1 ? 0u : (uint32_t)((((uint64_t)1 << 32) + (uint64_t)d - 1) / (uint64_t)d); };
     const int pairs = (L.nx / 2) * L.ny * L.nz;
     const unsigned nblocks = ceil_div((size_t)pairs, 256);
-    if (dots && (size_t)nblocks * 5 > dots->capacity) {
+    if (wd && (size_t)nblocks * 5 > dots->capacity) {
         set_error("launch_point_sweep: %u workgroups exceed the reduction scratch", nblocks);
         return TBFG_EINVAL;
     }
-    auto k = dots    ? k_point_sweep<T, TQ, false, true>
+    auto k = wd      ? k_point_sweep<T, TQ, false, true>
              : first ? k_point_sweep<T, TQ, true, false>
                      : k_point_sweep<T, TQ, false, false>;
-    hipLaunchKernelGGL(k, dim3(nblocks), dim3(256), 0, (hipStream_t)stream, L, beta, q, pin, pout, magic(L.nx / 2),
+    const unsigned fin = first && dots && dots->fin.n ? 1 : 0;
+    hipLaunchKernelGGL(k, dim3(nblocks + fin), dim3(256), 0, (hipStream_t)stream, L, beta, q, pin, pout, magic(L.nx / 2),
                        magic(L.ny), pairs, done, dots ? *dots : SweepDots{});
     TBFG_HIP(hipGetLastError());
     if (nblocks_out) *nblocks_out = nblocks;
@@ -919,12 +935,12 @@ static int launch_row_form(const LevelDev<T>& L, const TB* beta, const TQ* q, co
         set_error("launch_row_sweep: %u workgroups exceed the reduction scratch", nblocks);
         return TBFG_EINVAL;
     }
-    const dim3 blk(64 * (row_waves<T>() + 2));
+    const dim3 blk(64 * (row_waves<T>() + 2)), grd(nblocks + (FIRST && dots.fin.n ? 1 : 0));
     if (kev)
-        hipExtLaunchKernelGGL(k, dim3(nblocks), blk, 0, (hipStream_t)stream, kev->start, kev->stop, 0, L, beta, q, pin,
+        hipExtLaunchKernelGGL(k, grd, blk, 0, (hipStream_t)stream, kev->start, kev->stop, 0, L, beta, q, pin,
                               pout, kc, lr, rw, ntiles, c.tx, c.ty, done, dots);
     else
-        hipLaunchKernelGGL(k, dim3(nblocks), blk, 0, (hipStream_t)stream, L, beta, q, pin, pout, kc, lr, rw, ntiles, c.tx,
+        hipLaunchKernelGGL(k, grd, blk, 0, (hipStream_t)stream, L, beta, q, pin, pout, kc, lr, rw, ntiles, c.tx,
                            c.ty, done, dots);
     TBFG_HIP(hipGetLastError());
     if (nblocks_out) *nblocks_out = nblocks;
@@ -992,7 +1008,7 @@ int launch_row_sweep(const LevelDev<T>& L, const TB* beta, const TQ* q, const T*
                      const KernelEvents* kev)
 {
     SweepCfg c{0, 0, 0};
-    if (!row_supported(L) || (dots && first) || (tiles && (dots || !pick_shape(L, c, !first)))) {
+    if (!row_supported(L) || (dots && dots->r && first) || (tiles && ((dots && dots->r) || !pick_shape(L, c, !first)))) {
         set_error("launch_row_sweep: level %dx%dx%d not supported", L.nx, L.ny, L.nz);
         return TBFG_EINVAL;
     }
