@@ -165,7 +165,7 @@ __global__ void __launch_bounds__(512) k_op_dot(LevelDev<double> L, const double
         double dcol[kOpPlanes + 2], bcol[kOpPlanes + 2];
 #pragma unroll
         for (int u = 0; u < kOpPlanes + 2; ++u) {
-            int k = k0 - 1 + u;
+            int k = min(k0 - 1 + u, nz);  // (planes past the ghost of the last: that one again)
             k = k < 0 ? k + nz : (k >= nz ? k - nz : k);
             dcol[u] = d[plane * k + col];
             bcol[u] = beta[plane * k + col];
@@ -893,7 +893,7 @@ __global__ void k_resid_restrict(LevelDev<T> L, const TB* __restrict__ beta, con
     T P[NF][4], B[NF][4];
 #pragma unroll
     for (int u = 0; u < NF; ++u) {
-        int k = 2 * K0 - 1 + u;
+        int k = min(2 * K0 - 1 + u, nz);  // (past the ghost of the last plane: that one again)
         k = k < 0 ? k + nz : (k >= nz ? k - nz : k);
         const size_t pk = plane * k;
         P[u][0] = p[pk + c00], P[u][1] = p[pk + c10], P[u][2] = p[pk + c01], P[u][3] = p[pk + c11];
