@@ -474,7 +474,7 @@ def main():
         if prof32[0] > 0:
             us32 = prof32[1] / prof32[0] * 1e3
             out["mixed_fp32_storage"]["sweep_fine"] = {
-                "kernel": "k_sweep<float, float, float, 32, 16, 256, false, false, 4> (16 B per cell)",
+                "kernel": "k_row_sweep<float, float, float, false, false, false> (16 B per cell)",
                 "avg_us": round(us32, 2), "achieved_gbs": round(prof32[2] / us32 / 1e3, 1),
                 "frac": round(prof32[2] / us32 / 1e3 / HBM_PEAK_GBS, 4)}
         log("mixed, FP32 storage: %.2f solves/s, iterations %s" % (args.steps / tot32, sorted(set(it32))))
@@ -649,8 +649,8 @@ def main():
         achieved = bytes_per / avg_s / 1e9
         out["roofline_sweep_fine"] = {
             "bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-            "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic_of("sweep_fine_traffic.json"),
-            "kernel": "k_sweep<float, bf16s, bf16s, 32, 16, 256, false, false, 4>: finest-level red/black sweep "
+            "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None,  # (counted for the tiled sweep only)
+            "kernel": "k_row_sweep<float, bf16s, bf16s, false, false, true>: finest-level red/black sweep "
                       "from a non-zero start, out of place (p FP32 in and out, q and beta bf16 in: 12 B per cell)",
             "avg_us": round(avg_s * 1e6, 2), "launches": launches, "algorithmic_bytes_per_launch": bytes_per}
         log("operator pass: %d launches, avg %.1f us, %.0f GB/s algorithmic; sweep fine: %d launches, avg %.1f us, "
