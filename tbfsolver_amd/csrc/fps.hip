@@ -1206,10 +1206,20 @@ struct TriTables {
     double inv_ly;
 };
 
+// The volume-weighted mean of the refinement residual's pressure from that kernel's n
+// partials, by one workgroup more of the y solve: the inverse x pass subtracts it, and a
+// kernel of its own cost 3.7 us of the chain (128x96x128: 116.3 -> 111 us a solve).
+struct MeanArgs {
+    const double* partials = nullptr;
+    unsigned n = 0;  // 0: no mean is due
+    double inv_vg = 0.0;
+    double* out = nullptr;
+};
+
 template <class T, int MR, bool EXACT>
-__global__ void __launch_bounds__(256) k_ysolve(int nh, int ny, int nz, TriTables tt, C2<T>* __restrict__ B)
+__device__ __forceinline__ void ysolve(int block, int nh, int ny, int nz, const TriTables& tt, C2<T>* __restrict__ B)
 {
-    const int sys = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int sys = block * 4 + (threadIdx.x >> 6);
     if (sys >= nh * nz) return;
     const int m = sys / nz, kz = sys - m * nz;  // B is [kx][kz][j]
     C2<T>* col = B + (size_t)sys * ny;
@@ -1220,6 +1230,19 @@ __global__ void __launch_bounds__(256) k_ysolve(int nh, int ny, int nz, TriTable
     } else {
         tri_wave<float, MR, T, EXACT>(col, ny, tt.amf, tt.apf, (float)lam, false, tt.dyff, (float)tt.inv_ly);
     }
+}
+template <class T, int MR, bool EXACT>
+__global__ void __launch_bounds__(256) k_ysolve(int nh, int ny, int nz, TriTables tt, C2<T>* __restrict__ B)
+{
+    ysolve<T, MR, EXACT>(blockIdx.x, nh, ny, nz, tt, B);
+}
+template <class T, int MR, bool EXACT>
+__global__ void __launch_bounds__(256)
+    k_ysolve_mean(int nh, int ny, int nz, TriTables tt, C2<T>* __restrict__ B, MeanArgs mean)
+{
+    if (blockIdx.x > 0) return ysolve<T, MR, EXACT>(blockIdx.x - 1, nh, ny, nz, tt, B);
+    const double sum = sum_by_1024(mean.partials, mean.n);
+    if (threadIdx.x == 0) mean.out[0] = sum * mean.inv_vg;
 }
 
 // ----------------------------------------------------- refinement residual
@@ -1271,13 +1294,6 @@ __global__ void __launch_bounds__(256)
         }
     }
     block_partial<1>(v, red);
-}
-
-__global__ void k_fin_mean(unsigned nblocks, double inv_vg, double* __restrict__ out_mean, Reducer red)
-{
-    double tot[1];
-    final_sum<1>(red, nblocks, tot);
-    if (threadIdx.x == 0) out_mean[0] = tot[0] * inv_vg;
 }
 
 __global__ void k_fft_operator(OpTables o, const double* __restrict__ p, double* __restrict__ q)
@@ -1548,20 +1564,24 @@ int fps_create(const tbfg_grid_desc* g, const tbfg_fps_opts* o, tbfg_fps** out)
 }
 
 template <class T, int MR>
-static void launch_ysolve(tbfg_fps* h, C2<T>* B, hipStream_t s)
+static void launch_ysolve(tbfg_fps* h, C2<T>* B, const MeanArgs& mean, hipStream_t s)
 {
-    const int nsys = h->nh * h->nz;
+    const unsigned nblk = ceil_div(h->nh * h->nz, 4);
+    if constexpr (sizeof(T) == 4)
+        if (mean.n) {
+            auto k = h->ny == 64 * MR ? k_ysolve_mean<T, MR, true> : k_ysolve_mean<T, MR, false>;
+            hipLaunchKernelGGL(k, dim3(nblk + 1), dim3(256), 0, s, h->nh, h->ny, h->nz, h->tt, B, mean);
+            return;
+        }
     if (h->ny == 64 * MR)
-        hipLaunchKernelGGL((k_ysolve<T, MR, true>), dim3(ceil_div(nsys, 4)), dim3(256), 0, s, h->nh, h->ny, h->nz,
-                           h->tt, B);
+        hipLaunchKernelGGL((k_ysolve<T, MR, true>), dim3(nblk), dim3(256), 0, s, h->nh, h->ny, h->nz, h->tt, B);
     else
-        hipLaunchKernelGGL((k_ysolve<T, MR, false>), dim3(ceil_div(nsys, 4)), dim3(256), 0, s, h->nh, h->ny, h->nz,
-                           h->tt, B);
+        hipLaunchKernelGGL((k_ysolve<T, MR, false>), dim3(nblk), dim3(256), 0, s, h->nh, h->ny, h->nz, h->tt, B);
 }
 
 // one spectral solve: in (double) -> p (double), mode 0 write / 1 accumulate
 template <class T, class TIN>
-static int spectral_solve(tbfg_fps* h, const TIN* in, double* p, int mode, hipStream_t s)
+static int spectral_solve(tbfg_fps* h, const TIN* in, double* p, int mode, hipStream_t s, const MeanArgs& mean = {})
 {
     const int nx = h->nx, ny = h->ny, nz = h->nz, nh = h->nh;
     C2<T>* A = h->A.as<C2<T>>();
@@ -1591,12 +1611,12 @@ static int spectral_solve(tbfg_fps* h, const TIN* in, double* p, int mode, hipSt
         hipLaunchKernelGGL((k_zfwd<T>), dim3((ny / h->JT) * nh), dim3(kFftThreads), ldz, s, ny, nz, h->JT, h->pz, twz,
                            A, B);
     switch (h->MR) {
-        case 1: launch_ysolve<T, 1>(h, B, s); break;
-        case 2: launch_ysolve<T, 2>(h, B, s); break;
-        case 3: launch_ysolve<T, 3>(h, B, s); break;
-        case 4: launch_ysolve<T, 4>(h, B, s); break;
-        case 8: launch_ysolve<T, 8>(h, B, s); break;
-        default: launch_ysolve<T, 16>(h, B, s); break;
+        case 1: launch_ysolve<T, 1>(h, B, mean, s); break;
+        case 2: launch_ysolve<T, 2>(h, B, mean, s); break;
+        case 3: launch_ysolve<T, 3>(h, B, mean, s); break;
+        case 4: launch_ysolve<T, 4>(h, B, mean, s); break;
+        case 8: launch_ysolve<T, 8>(h, B, mean, s); break;
+        default: launch_ysolve<T, 16>(h, B, mean, s); break;
     }
     if (h->tlz)
         tl_dispatch(nz, [&](auto a, auto b) {
@@ -1635,9 +1655,8 @@ int fps_solve_dev(tbfg_fps* h, const double* s, double* p, void* stream)
         int kc = 0;
         const dim3 grd = residual_grid(h->nx, h->ny, h->nz, kc);
         hipLaunchKernelGGL(k_fft_residual, grd, dim3(64, 4), 0, st, h->ot, s, p, h->r.as<double>(), kc, red);
-        hipLaunchKernelGGL(k_fin_mean, dim3(1), dim3(1024), 0, st, grd.x * grd.y * grd.z, h->inv_vg,
-                           h->mean.as<double>(), red);
-        TBFG_TRY((spectral_solve<float, double>(h, h->r.as<double>(), p, 1, st)));
+        const MeanArgs mean{red.partials, grd.x * grd.y * grd.z, h->inv_vg, h->mean.as<double>()};
+        TBFG_TRY((spectral_solve<float, double>(h, h->r.as<double>(), p, 1, st, mean)));
     }
     return TBFG_OK;
 }
