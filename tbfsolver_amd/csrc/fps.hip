@@ -1056,15 +1056,23 @@ __device__ void tri_wave(C2<TS>* __restrict__ col, int ny, const TC* __restrict_
     const int m = EXACT ? MR : (ny + 63) / 64;
     TC a[MR], b[MR], c[MR];
     C2<TC> d[MR];
+    // every row's loads at once, unconditionally (rows past the last: that one): each load
+    // under its row's condition was a branch that waited for it.  256x192x256: 42.9 -> 39.1 us
+    C2<TS> col_r[MR];
+#pragma unroll
+    for (int r = 0; r < MR; ++r) {
+        const int row = EXACT ? lane * m + r : min(lane * m + min(r, m - 1), ny - 1);
+        a[r] = am[row];
+        c[r] = ap[row];
+        col_r[r] = col[row];
+    }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int r = 0; r < MR; ++r) {
         const int row = lane * m + r;
         if (r < m && (EXACT || row < ny) && !(pinned && row == ny - 1)) {
-            a[r] = am[row];
-            c[r] = ap[row];
             b[r] = lam - a[r] - c[r];
-            const C2<TS> v = col[row];
-            d[r] = C2<TC>{(TC)v.x, (TC)v.y};
+            d[r] = C2<TC>{(TC)col_r[r].x, (TC)col_r[r].y};
         } else {
             a[r] = 0;
             c[r] = 0;
