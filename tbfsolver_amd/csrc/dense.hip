@@ -316,10 +316,12 @@ __global__ void __launch_bounds__(256)
 // the MALL after the first application): 1152 cells, 10.6 MB.
 __global__ void __launch_bounds__(256)
     k_dense_apply(int n, const double* __restrict__ G, const double* __restrict__ q, double* __restrict__ x,
-                  const int* done)
+                  PcgState* st, const int* done)
 {
     __shared__ double sq[kDenseDirectCells];
-    if (done && *done) return;
+    const bool run = !(done && *done);
+    if (blockIdx.x == 0 && threadIdx.x == 0) st->coarse_due = run ? 1 : 0;
+    if (!run) return;
     for (int c = threadIdx.x; c < n; c += 256) sq[c] = q[c];
     __syncthreads();
     const int lane = threadIdx.x & 63, r = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -387,14 +389,15 @@ __global__ void __launch_bounds__(1024) k_dense_check(DenseCheck a, PcgState* st
 
 // k_fin_dots with the check beside it, in a second workgroup: nothing reads the diagnostics
 // before the solve ends, and as a launch of its own the check cost 7.3 us of the 186 that an
-// iteration takes at 96x64x96.
+// iteration takes at 96x64x96.  The first workgroup may set done, so the second goes by
+// whether the solve it checks ran.
 __global__ void __launch_bounds__(1024)
     k_fin_dots_check(unsigned nblocks, size_t ncell, int init, PcgState* st, Reducer red, int32_t* host_done,
                      DenseCheck a)
 {
     if (blockIdx.x == 0)
         fin_dots(nblocks, ncell, init, st, red, host_done);
-    else if (!st->done)
+    else if (st->coarse_due)
         dense_check(a, st);
 }
 
@@ -441,7 +444,7 @@ int launch_dense_solve(const DenseCheck& a, const double* G, double* x, bool che
         set_error("launch_dense_solve: %d cells (at most %d)", n, kDenseDirectCells);
         return TBFG_EINVAL;
     }
-    hipLaunchKernelGGL(k_dense_apply, dim3(ceil_div(n, 4)), dim3(256), 0, s, n, G, a.q, x, done);
+    hipLaunchKernelGGL(k_dense_apply, dim3(ceil_div(n, 4)), dim3(256), 0, s, n, G, a.q, x, st, done);
     if (check) hipLaunchKernelGGL(k_dense_check, dim3(1), dim3(1024), 0, s, a, st, done);
     TBFG_HIP(hipGetLastError());
     return TBFG_OK;

@@ -693,7 +693,7 @@ __global__ void __launch_bounds__(256)
                  const double* __restrict__ d, const double* __restrict__ qv, PcgState* st,
                  const double* __restrict__ pop, unsigned nop, Reducer red)
 {
-    if (st->done) return;
+    if (st->halted) return;  // (not done, which this kernel sets)
     const double delta = st->delta;
     const size_t stride = (size_t)gridDim.x * blockDim.x, t0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     // the first cell's values in flight meanwhile

@@ -63,12 +63,16 @@ struct PcgState {
     int32_t done;      // 1: stop (converged, max_iter, or numeric failure)
     int32_t status;    // TBFG_OK / TBFG_ENOTCONVERGED / TBFG_ENUMERIC
     int32_t flexible;  // 0 Fletcher-Reeves, 1 Polak-Ribiere
-    int32_t pad;
+    // done when the last iteration ended: written by fin_dots only.  A kernel that sets done
+    // itself tests this one (the residual update; a sweep that carries out the stop test):
+    // done could change while its wavefronts start, and some of a workgroup would leave
+    // ahead of the barriers that the others sum at
+    int32_t halted;
     // coarsest-level solves of this PCG solve (diagnostics)
     int32_t coarse_calls;
     int32_t coarse_iters;     // inner iterations summed over calls
     int32_t coarse_iters_max;
-    int32_t pad2;
+    int32_t coarse_due;       // the last dense solve ran (k_dense_apply): its diagnostics are due
     double coarse_res_max;    // worst final relative residual
     // V-cycles per preconditioner application under a residual target (tolMG)
     int32_t mg_stop;       // 1: no further cycle in this application

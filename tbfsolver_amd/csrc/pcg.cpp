@@ -553,6 +553,8 @@ static int smooth(tbfg_pcg* h, int l, const T0* b, const T0* q, T*& p, T*& alt, 
         const bool last = s == nsweeps - 1;
         const SweepDots* dots = last ? last_dots : nullptr;
         const SweepDots* with = f0 && fin ? fin : dots;
+        // (a sweep with the stop test sets done: its workgroups go by the iteration's start)
+        const int* stop = f0 && fin ? &fin->fin.st->halted : done;
         unsigned* nb = last ? nb_out : nullptr;
         if (h->fused[l] == 1 || h->fused[l] == 3) {
             // the timed finest-level sweep: from a non-zero start, without the dot products
@@ -565,13 +567,13 @@ static int smooth(tbfg_pcg* h, int l, const T0* b, const T0* q, T*& p, T*& alt, 
             if (h->fused[l] == 1 && (!row_supported<T>(L) || sweep_named<T>(L, !f0 && !dots) || (h->b16 && dots)))
                 TBFG_TRY(launch_sweep<T, T0, T0>(L, b, q, p, alt, f0, done, stream, dots, nb, ps.events()));
             else
-                TBFG_TRY(launch_row_sweep<T, T0, T0>(L, b, q, p, alt, f0, h->b16 && h->fused[l] == 1, done, stream, with,
+                TBFG_TRY(launch_row_sweep<T, T0, T0>(L, b, q, p, alt, f0, h->b16 && h->fused[l] == 1, stop, stream, with,
                                                      nb, ps.events()));
             std::swap(p, alt);
         } else if constexpr (!narrow) {
             ProfScope ps(h, l == 0 ? 0 : -1, stream);
             if (h->fused[l] == 2) {
-                TBFG_TRY(launch_point_sweep<T, T>(L, b, q, p, alt, f0, done, stream, with, nb));
+                TBFG_TRY(launch_point_sweep<T, T>(L, b, q, p, alt, f0, stop, stream, with, nb));
                 std::swap(p, alt);
             } else {
                 TBFG_TRY(launch_rbgs<T, T>(L, b, q, p, RED, f0, done, stream));

@@ -178,6 +178,7 @@ __device__ __forceinline__ void fin_dots(unsigned nblocks, size_t ncell, int ini
                 }
             }
         }
+        st->halted = done;
         if (host_done) __hip_atomic_store(host_done, done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }

@@ -175,3 +175,40 @@ def test_pair_operator_matches_columns(torch_gpu, monkeypatch, n, precision):
     ib, b = solve(beta, torch_gpu.zeros_like(q))
     print("  iterations", ia, ib, "rel", rel(a, b), flush=True)
     assert abs(ia - ib) <= 1 and rel(a, b) < 1e-9
+
+
+@pytest.mark.parametrize("sweeps", ["pairs", "rows"])
+@pytest.mark.parametrize("unfused", [False, True], ids=["fused", "unfused"])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_breakdown_ends_the_solve_and_leaves_psi(torch_gpu, monkeypatch, precision, unfused, sweeps):
+    """A breakdown of the first step (beta zero: d.Ad is not a number) is found by every workgroup of the
+    residual update alike: the solve ends with a numeric error, blocking and queued, psi keeps its bits, and
+    the handle solves as a new one afterwards."""
+    n = (64, 48, 64)
+    print("case breakdown", precision, unfused, sweeps, flush=True)
+    if unfused:
+        monkeypatch.setenv("TBFG_UNFUSED_OP", "1")
+    monkeypatch.setenv("TBFG_SWEEP_MIN_CELLS", "0" if sweeps == "rows" else str(10 ** 12))
+    g, beta, q = case(torch_gpu, n)
+    kw = dict(nLevels=4, precision=precision, flexible=1, tolPCG=1e-8, maxIterPCG=100)
+    start = to_dev(np.random.default_rng(3).normal(size=n), torch_gpu)
+    s = T.PCG(g, **kw)
+    for queued in (False, True):
+        psi = start.clone()
+        with pytest.raises(T.TbfgError) as e:
+            if queued:
+                s.solvePCG_queued(psi, torch_gpu.zeros_like(beta), q, 3)
+                torch_gpu.cuda.synchronize()
+                s.result()
+            else:
+                s.solvePCG(psi, torch_gpu.zeros_like(beta), q)
+        assert "non-finite" in str(e.value)
+        assert torch_gpu.equal(psi, start)
+    out = []
+    for h in (s, T.PCG(g, **kw)):
+        psi = torch_gpu.zeros_like(q)
+        h.solvePCG(psi, beta, q)
+        assert h.converged
+        out.append((h.iterations, h.coarse_stats(), psi))
+        h.close()
+    assert out[0][:2] == out[1][:2] and torch_gpu.equal(out[0][2], out[1][2])
