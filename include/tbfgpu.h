@@ -307,7 +307,9 @@ int tbfg_material_props_dev(const tbfg_grid_desc* grid, double rho_l, double rho
  *   TBFG_TUNE_SWEEP_EDGE  first sweep / sweep with the dots  shape = {tx, ty, threads}
  *   TBFG_TUNE_OP          FP64 operator product (level 0)    shape = {tx, threads, 0}, {-1, 0, 0} = columns
  * A shape the level does not divide, or without a kernel, is ignored.  Sweeps
- * read the table at every launch, the operator when a handle is created.
+ * read the table at every launch (the finest level's first sweep, which carries
+ * out the stop test unless its shape is entered: when a solve starts), the
+ * operator when a handle is created.
  * shape {0, 0, 0} removes the entry; tbfg_tune_get returns {0, 0, 0} for none. */
 #define TBFG_TUNE_SWEEP 0
 #define TBFG_TUNE_SWEEP_EDGE 1

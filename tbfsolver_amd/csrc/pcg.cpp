@@ -563,8 +563,11 @@ static int smooth(tbfg_pcg* h, int l, const T0* b, const T0* q, T*& p, T*& alt, 
             // by rows, except where a tile shape is asked for.  Under bf16 storage the last bit
             // of a sweep or of a dot product becomes a few 1e-9 of the solution (1 % of its
             // error), the residual being cut to 8 bits: there the rows round as the tiles
-            // do, and the sweep that forms the dot products stays with them
-            if (h->fused[l] == 1 && (!row_supported<T>(L) || sweep_named<T>(L, !f0 && !dots) || (h->b16 && dots)))
+            // do, and the sweep that forms the dot products stays with them.  A sweep that
+            // the solve has given the stop test to takes the rows whatever the table says by
+            // now: another thread may enter a shape in the middle of a solve
+            if (h->fused[l] == 1 && !(f0 && fin) &&
+                (!row_supported<T>(L) || sweep_named<T>(L, !f0 && !dots) || (h->b16 && dots)))
                 TBFG_TRY(launch_sweep<T, T0, T0>(L, b, q, p, alt, f0, done, stream, dots, nb, ps.events()));
             else
                 TBFG_TRY(launch_row_sweep<T, T0, T0>(L, b, q, p, alt, f0, h->b16 && h->fused[l] == 1, stop, stream, with,
@@ -587,7 +590,7 @@ static int smooth(tbfg_pcg* h, int l, const T0* b, const T0* q, T*& p, T*& alt, 
 // Whether the finest level's sweep from zero can carry out the stop test of the iteration
 // before (a workgroup more of it): k_point_sweep and k_row_sweep do.  The sweep itself then
 // runs once more after convergence; a launch of its own for the test took 4.5 us of every
-// iteration.
+// iteration.  Asked once per solve: the tuning table may change while one runs.
 template <class T>
 static bool folds_stop_test(const tbfg_pcg* h)
 {

@@ -212,3 +212,94 @@ def test_breakdown_ends_the_solve_and_leaves_psi(torch_gpu, monkeypatch, precisi
         out.append((h.iterations, h.coarse_stats(), psi))
         h.close()
     assert out[0][:2] == out[1][:2] and torch_gpu.equal(out[0][2], out[1][2])
+
+
+def _solve(torch, g, beta, q, **kw):
+    s = T.PCG(g, flexible=1, coarse_max_iter=0, **kw)
+    psi = torch.zeros_like(q)
+    s.solvePCG(psi, beta, q)
+    out = (s.iterations, s.converged, psi)
+    s.close()
+    return out
+
+
+@pytest.mark.parametrize("most", [1, 3, 200])
+def test_stop_test_in_the_sweep_ends_as_its_own_launch(torch_gpu, most):
+    """bf16 storage, where the rows round as the tiles do: with the first sweep's tile shape entered in the
+    tuning table the stop test is a launch of its own, without it a workgroup of that sweep.  Converged or at
+    the iteration limit, the iterations and the bits of psi are the same."""
+    from tbfsolver_amd import tune as Tu
+
+    n = (128, 64, 128)
+    print("case folded stop test", most, flush=True)
+    g, beta, q = case(torch_gpu, n)
+    kw = dict(nLevels=4, precision="mixed-bf16", tolPCG=1e-8, maxIterPCG=most)
+    Tu.clear()
+    try:
+        a = _solve(torch_gpu, g, beta, q, **kw)
+        Tu.set_entry("sweep_edge", n, "mixed", (64, 8, 256))  # the built-in choice, by name
+        b = _solve(torch_gpu, g, beta, q, **kw)
+    finally:
+        Tu.clear()
+    assert a[:2] == b[:2] and a[1] == (most == 200) and (a[1] or a[0] == most), (a[:2], b[:2])
+    assert torch_gpu.equal(a[2], b[2])
+
+
+@pytest.mark.parametrize("sweeps", ["pairs", "rows"])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_stop_test_in_pair_and_row_sweeps(torch_gpu, monkeypatch, precision, sweeps):
+    """The same on levels smoothed by pairs and rows, against the half-sweep launches (which leave the stop
+    test to its own launch): the iterations, at the limit and converged; psi to ten times the residual bound."""
+    n = (48, 32, 64)
+    print("case folded stop test", precision, sweeps, flush=True)
+    monkeypatch.setenv("TBFG_SWEEP_MIN_CELLS", "0" if sweeps == "rows" else str(10 ** 12))
+    g, beta, q = case(torch_gpu, n)
+    for most in (1, 2, 5, 200):
+        kw = dict(nLevels=3, precision=precision, tolPCG=1e-10, maxIterPCG=most)
+        monkeypatch.delenv("TBFG_HALF_SWEEPS", raising=False)
+        a = _solve(torch_gpu, g, beta, q, **kw)
+        monkeypatch.setenv("TBFG_HALF_SWEEPS", "1")
+        b = _solve(torch_gpu, g, beta, q, **kw)
+        assert a[1] == b[1] == (most == 200)
+        if most < 200:
+            assert a[0] == b[0] == most
+        else:
+            assert abs(a[0] - b[0]) <= 1
+            assert rel(to_host(a[2] - a[2].mean()), to_host(b[2] - b[2].mean())) < 1e-9
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed", "mixed-bf16"])
+def test_shapes_entered_while_solves_run(torch_gpu, precision):
+    """Another thread enters and removes the first sweep's tile shape all the while: the stop test is neither
+    lost nor made twice.  Iterations within one (the shapes round differently), converged to the same psi."""
+    import threading
+
+    from tbfsolver_amd import tune as Tu
+
+    n = (128, 64, 128)
+    print("case tuning during solves", precision, flush=True)
+    g, beta, q = case(torch_gpu, n)
+    kw = dict(nLevels=4, precision=precision, tolPCG=1e-8, maxIterPCG=200)
+    key, shape = ("fp64", (64, 4, 128)) if precision == "fp64" else ("mixed", (64, 8, 256))
+    Tu.clear()
+    stop, turns = threading.Event(), [0]
+
+    def toggle():
+        while not stop.is_set():
+            Tu.set_entry("sweep_edge", n, key, shape)
+            Tu.set_entry("sweep_edge", n, key, (0, 0, 0))
+            turns[0] += 1
+
+    quiet = _solve(torch_gpu, g, beta, q, **kw)
+    t = threading.Thread(target=toggle)
+    t.start()
+    try:
+        out = [_solve(torch_gpu, g, beta, q, **kw) for _ in range(5)]
+    finally:
+        stop.set()
+        t.join()
+        Tu.clear()
+    assert quiet[1] and turns[0] > 0
+    for it, converged, psi in out:
+        assert converged and abs(it - quiet[0]) <= 1
+        assert rel(to_host(psi - psi.mean()), to_host(quiet[2] - quiet[2].mean())) < 1e-6
