@@ -2222,29 +2222,31 @@ OpPlan op_plan(const LevelDev<double>& L)
 {
     OpPlan m;
     const char* env = std::getenv("TBFG_OP_TILE");
-    // pairs below 1 M cells whatever the tiles (the index divisions in 32 bits, as point_supported)
-    const uint64_t cells = (uint64_t)L.nx * L.ny * L.nz;
-    if (!env && L.nx % 2 == 0 && cells < kOpPointCells && cells / 2 * (uint64_t)std::max(L.nx / 2, L.ny) < ((uint64_t)1 << 32)) {
-        m.point = true;
-        m.pblocks = ceil_div((size_t)(cells / 2), kOpPointThreads);
-    }
+    auto fits = [&](int tx, int nt) { return L.nx % tx == 0 && L.ny % (nt / tx) == 0 && L.nz >= 2; };
     // 256-thread tiles first: with long marches they measured fastest (256x192x256:
     // 64x256 tiles 136 us, 32x256 138 us, 128x512 152 us, all with 64-plane chunks)
     std::vector<std::pair<int, int>> cand = {{64, 256}, {32, 256}, {128, 512}, {64, 512}};
+    bool named = false;  // a tile that the environment or the tuning table asks for
     int tuned[3];
     if (env) {
         int a = 0, b = 0;
         if (std::sscanf(env, "%dx%d", &a, &b) != 2) return m;
         cand = {{a, b}};
+        named = true;
     } else if (tune_lookup(TBFG_TUNE_OP, L.nx, L.ny, L.nz, 8, tuned)) {
         if (tuned[0] < 0) return m;  // columns
         const std::pair<int, int> t{tuned[0], tuned[1]};
-        const bool known = t == std::pair<int, int>{128, 512} || t == std::pair<int, int>{64, 512} ||
-                           t == std::pair<int, int>{32, 256} || t == std::pair<int, int>{64, 256};
-        if (known) cand.insert(cand.begin(), t);
+        named = std::find(cand.begin(), cand.end(), t) != cand.end() && fits(t.first, t.second);
+        if (named) cand.insert(cand.begin(), t);
+    }
+    // otherwise pairs below 1 M cells whatever the tiles (the index divisions in 32 bits, as point_supported)
+    const uint64_t cells = (uint64_t)L.nx * L.ny * L.nz;
+    if (!named && L.nx % 2 == 0 && cells < kOpPointCells && cells / 2 * (uint64_t)std::max(L.nx / 2, L.ny) < ((uint64_t)1 << 32)) {
+        m.point = true;
+        m.pblocks = ceil_div((size_t)(cells / 2), kOpPointThreads);
     }
     for (auto [tx, nt] : cand) {
-        if (L.nx % tx == 0 && L.ny % (nt / tx) == 0 && L.nz >= 2) {
+        if (fits(tx, nt)) {
             m.tx = tx;
             m.nt = nt;
             break;

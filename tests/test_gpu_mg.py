@@ -899,3 +899,42 @@ def test_mg_tolerance_loop_cap_and_fixed_cycles(torch_gpu, monkeypatch):
         true_res = np.linalg.norm(q - O.apply_op(go, beta, to_host(psi))) / np.linalg.norm(q)
         assert true_res < 2e-8
         s.close()
+
+
+@pytest.mark.parametrize("shape,tile", [((-1, 0, 0), "columns"), ((64, 512, 0), "64x512"), ((32, 256, 0), "32x256")])
+def test_tuned_operator_below_the_pairs_limit(torch_gpu, monkeypatch, shape, tile):
+    """An operator entry of the tuning table is the operator launched below 1 M cells too, where a thread
+    per pair is the built-in choice: the bits of the same operator asked for by TBFG_OP_TILE, and for the
+    columns a handle without the second direction buffer.  An entry that does not divide the grid is ignored."""
+    from tbfsolver_amd import tune as Tu
+
+    n = (64, 48, 64)
+    print("case tuned operator", shape, flush=True)
+    g, go, rho, _, q, beta = bubble_case(n, 8, 1, 19)
+    dq, db = to_dev(q, torch_gpu), to_dev(beta, torch_gpu)
+
+    def solve():
+        s = T.PCG(g, nLevels=4, tolPCG=1e-10, maxIterPCG=200, flexible=1)
+        psi = torch_gpu.zeros_like(dq)
+        s.solvePCG(psi, db, dq)
+        out = (s.iterations, s.footprint, to_host(psi))
+        assert s.converged
+        s.close()
+        return out
+
+    Tu.clear()
+    try:
+        plain = solve()
+        Tu.set_entry("op", n, "fp64", (128, 512, 0))  # 64 cells along x: does not divide
+        ignored = solve()
+        Tu.set_entry("op", n, "fp64", shape)
+        tuned = solve()
+    finally:
+        Tu.clear()
+    monkeypatch.setenv("TBFG_OP_TILE", tile)
+    asked = solve()
+    assert ignored[:2] == plain[:2] and np.array_equal(ignored[2], plain[2])
+    assert tuned[:2] == asked[:2] and np.array_equal(tuned[2], asked[2])
+    assert not np.array_equal(tuned[2], plain[2])
+    if shape[0] < 0:
+        assert tuned[1] == plain[1] - 8 * n[0] * n[1] * n[2]
