@@ -1,12 +1,15 @@
 """Tile-shape tuner for the multigrid kernels.
 
-The library launches its sweep and operator kernels with a tile shape chosen
-per level: from the tuning table (tbfg_tune_set) when it has an entry for the
-level's cells and precision, else by a built-in order of preference.  This
-module fills the table by measurement: for the finest level of a PCG+MG
-instance it times whole solves with every candidate shape of one kernel
-family at a time (sweep from a non-zero start, first sweep / sweep with the
-dot products, FP64 operator product) and keeps the fastest.  Shapes change
+The library launches its sweep and operator kernels with a tile shape from the
+tuning table (tbfg_tune_set) when it has an entry for the level's cells and
+precision, else by its built-in choice: kernels that march whole rows, or a
+thread per pair of cells on smaller grids, and a tile where those do not apply.
+This module fills the table by measurement: for the finest level of a PCG+MG
+instance it times whole solves with the built-in choice and with every candidate
+shape of one kernel family at a time (sweep from a non-zero start, first sweep /
+sweep with the dot products, FP64 operator product) and enters the fastest shape
+where it beats the built-in choice by more than 1 % and by more than the two
+timings of that choice, before and after the shapes, differ.  Shapes change
 only how cells are grouped into workgroups: the sweep results agree to
 round-off (a cell recomputed in a tile's ring may round differently from the
 same cell inside a tile), the operator's dot product differs in its summation
@@ -15,7 +18,7 @@ order only.
   candidates(kind, dims, precision)     shapes with a kernel that tile the level
   tune_instance(dims, precision, reps)  measure one instance size, enter the winners
   autotune(sizes, precision, reps)      every distinct size; returns the table
-  save(table, path) / load(path)        JSON; load enters the entries
+  save(table, path) / load(path)        JSON; load enters the entries (shape 0,0,0: the built-in choice)
 
   python -m tbfsolver_amd.tune --config3 --out table.json   (the 64-instance workload's sizes)
 """
@@ -33,6 +36,8 @@ SWEEP_F = [(64, 8, 256), (32, 16, 256), (64, 16, 512), (32, 8, 128)]
 SWEEP_D = [(64, 4, 128), (64, 8, 256), (32, 8, 128)]
 OP = [(128, 512, 0), (64, 512, 0), (32, 256, 0), (64, 256, 0), (-1, 0, 0)]  # (-1, 0, 0): column segments
 PLANE_MARCH_MIN_CELLS = 1 << 20  # smallest level smoothed by the plane-march sweep
+BUILT_IN = (0, 0, 0)  # no entry
+MARGIN = 0.01
 
 
 def _i3(v):
@@ -109,26 +114,39 @@ def _time_solves(g, q, beta, precision, reps):
 
 
 def tune_instance(dims, precision="mixed", reps=3, log=None):
-    """Times each candidate of each family on a PCG+MG instance of these cells
-    (the other families at their current choice) and enters the fastest.
-    Returns {kind: {"shape": [...], "ms": t, "tried": {shape: ms}}}."""
+    """Times the built-in choice and each candidate of each family on a PCG+MG instance of these
+    cells (the other families at their current choice) and enters the fastest candidate, or removes
+    the entry where none beats the built-in choice.
+    Returns {kind: {"shape": [...], "ms": t, "tried": {shape: ms}}}, shape [0, 0, 0] for the built-in
+    choice; the operator, FP64 in every form, with "precision": "fp64" (its key in the table)."""
     dims = tuple(int(v) for v in dims)
     g, q, beta = _case(dims)
     out = {}
     for kind in ("op", "sweep", "sweep_edge"):
+        key = "fp64" if kind == "op" else precision
         cands = candidates(kind, dims, precision)
-        if len(cands) < 2:
+        if not cands:
             continue
-        tried = {}
-        for shape in cands:
-            set_entry(kind, dims, precision, shape)
-            tried[shape] = _time_solves(g, q, beta, precision, reps)
+
+        def timed(shape):
+            set_entry(kind, dims, key, shape)
+            return _time_solves(g, q, beta, precision, reps)
+
+        first = timed(BUILT_IN)
+        tried = {shape: timed(shape) for shape in cands}
+        base = sorted((first, timed(BUILT_IN)))
         best = min(tried, key=tried.get)
-        set_entry(kind, dims, precision, best)
+        if tried[best] >= base[0] - max(MARGIN * base[0], base[1] - base[0]):
+            best = BUILT_IN
+        tried[BUILT_IN] = base[0]
+        set_entry(kind, dims, key, best)
         out[kind] = {"shape": list(best), "ms": round(tried[best], 4),
                      "tried": {"x".join(str(v) for v in k): round(t, 4) for k, t in tried.items()}}
+        if key != precision:
+            out[kind]["precision"] = key
         if log:
-            log("tune %s %s %s: %s (%.3f ms; %s)" % ("x".join(map(str, dims)), precision, kind, best, tried[best],
+            log("tune %s %s %s: %s (%.3f ms; %s)" % ("x".join(map(str, dims)), precision, kind,
+                                                    "built-in" if best == BUILT_IN else best, tried[best],
                                                     ", ".join("%s %.3f" % (k, t) for k, t in tried.items())))
     return out
 
@@ -155,7 +173,7 @@ def load(path, apply=True):
         for key, kinds in table["entries"].items():
             dims = tuple(int(v) for v in key.split(","))
             for kind, e in kinds.items():
-                set_entry(kind, dims, prec, e["shape"])
+                set_entry(kind, dims, e.get("precision", prec), e["shape"])
     return table
 
 

@@ -44,3 +44,59 @@ def test_json_tables(tmp_path):
     assert Tu.get_entry("op", (128, 96, 128), "mixed") == (64, 512, 0)
     assert Tu.get_entry("sweep", (128, 96, 128), "mixed") == (32, 16, 256)
     Tu.clear()
+
+
+@pytest.mark.parametrize("precision", ["mixed", "fp64"])
+@pytest.mark.parametrize("wins", [False, True], ids=["built-in", "shapes"])
+def test_tuner_enters_what_beats_the_built_in_choice(monkeypatch, tmp_path, precision, wins):
+    """With every shape 5 % slower than the built-in choice nothing is entered; with the 32-cell tiles 5 % faster
+    they are, the operator's under the FP64 key that handles of every precision look up, also from a saved table."""
+    dims = (192, 96, 128)
+    monkeypatch.setattr(Tu, "_case", lambda d: (None, None, None))
+    families = (("op", "fp64"), ("sweep", precision), ("sweep_edge", precision))
+
+    def time_solves(*_):
+        ms = 1.0
+        for kind, key in families:
+            shape = Tu.get_entry(kind, dims, key)
+            if shape != Tu.BUILT_IN:
+                ms += -0.05 if wins and shape[0] == 32 else 0.05
+        return ms
+
+    monkeypatch.setattr(Tu, "_time_solves", time_solves)
+    Tu.clear()
+    try:
+        table = Tu.autotune([dims], precision)
+        got = {kind: Tu.get_entry(kind, dims, key) for kind, key in families}
+        assert set(table["entries"]["192,96,128"]) == {"op", "sweep", "sweep_edge"}
+        for shape in got.values():
+            assert (shape[0] == 32) if wins else shape == Tu.BUILT_IN
+        path = str(tmp_path / "t.json")
+        Tu.save(table, path)
+        Tu.clear()
+        Tu.load(path)
+        assert {kind: Tu.get_entry(kind, dims, key) for kind, key in families} == got
+    finally:
+        Tu.clear()
+
+
+def test_tuner_does_not_enter_noise(monkeypatch):
+    """A shape ahead by less than 1 %, or by less than the built-in choice differs from itself, is noise."""
+    dims = (192, 96, 128)
+    monkeypatch.setattr(Tu, "_case", lambda d: (None, None, None))
+    Tu.clear()
+    try:
+        for base, other in ((lambda n: 1.0, 0.995), (lambda n: 1.0 + 0.04 * (n % 2), 0.97)):
+            calls = [0]
+
+            def time_solves(*_):
+                if all(Tu.get_entry(k, dims, p) == Tu.BUILT_IN for k in Tu.KINDS for p in ("mixed", "fp64")):
+                    calls[0] += 1
+                    return base(calls[0])
+                return other
+
+            monkeypatch.setattr(Tu, "_time_solves", time_solves)
+            Tu.tune_instance(dims, "mixed")
+            assert all(Tu.get_entry(k, dims, p) == Tu.BUILT_IN for k in Tu.KINDS for p in ("mixed", "fp64"))
+    finally:
+        Tu.clear()
