@@ -121,8 +121,12 @@ int copy_in(HostRing& ring, const double* src, const FArr& f, const int32_t* n, 
         const int sl = c % HostRing::kSlots;
         const int64_t kb = k + planes <= n[2] + 1 ? k + planes : n[2] + 1;
         TBFG_TRY(ring.wait(sl));
-        double* pin = ring.pin + (size_t)sl * ring.slot;
+        double* pin = ring.at(sl);
         gather(src, f, n, k, kb, pin);
+        if (!ring.pin) {  // (one chunk)
+            TBFG_HIP(hipMemcpy(dev, pin, plane * (size_t)n[2] * 8, hipMemcpyHostToDevice));
+            return TBFG_OK;
+        }
         TBFG_HIP(hipMemcpyAsync(dev + plane * (size_t)(k - 1), pin, plane * (size_t)(kb - k) * 8, hipMemcpyHostToDevice,
                                 nullptr));
         TBFG_TRY(ring.record(sl));
@@ -136,11 +140,17 @@ int copy_out(HostRing& ring, const double* dev, const FArr& f, const int32_t* n,
     const size_t plane = (size_t)n[0] * n[1];
     const int64_t planes = std::min<int64_t>(n[2], (int64_t)(ring.slot / plane));
     const int64_t chunks = (n[2] + planes - 1) / planes;
+    if (chunks == 1) {  // (a blocking copy: after one that an event ends, the next wait for the device takes 30 us)
+        TBFG_HIP(hipMemcpy(ring.at(0), dev, plane * (size_t)n[2] * 8, hipMemcpyDeviceToHost));
+        scatter_planes(ring.at(0), f, n, 1, (int64_t)n[2] + 1, dst);
+        scatter_z_halo(f, n, dst);
+        return TBFG_OK;
+    }
     auto first = [&](int64_t c) { return 1 + c * planes; };
     auto end = [&](int64_t c) { return c + 1 < chunks ? 1 + (c + 1) * planes : (int64_t)n[2] + 1; };
     auto start = [&](int64_t c) -> int {
         const int sl = (int)(c % HostRing::kSlots);
-        TBFG_HIP(hipMemcpyAsync(ring.pin + (size_t)sl * ring.slot, dev + plane * (size_t)(first(c) - 1),
+        TBFG_HIP(hipMemcpyAsync(ring.at(sl), dev + plane * (size_t)(first(c) - 1),
                                 plane * (size_t)(end(c) - first(c)) * 8, hipMemcpyDeviceToHost, nullptr));
         return ring.record(sl);  // (after the slot's last use: the same stream)
     };
@@ -148,7 +158,7 @@ int copy_out(HostRing& ring, const double* dev, const FArr& f, const int32_t* n,
     for (int64_t c = 0; c < chunks; ++c) {
         const int sl = (int)(c % HostRing::kSlots);
         TBFG_TRY(ring.wait(sl));
-        scatter_planes(ring.pin + (size_t)sl * ring.slot, f, n, first(c), end(c), dst);
+        scatter_planes(ring.at(sl), f, n, first(c), end(c), dst);
         if (c + HostRing::kSlots < chunks) TBFG_TRY(start(c + HostRing::kSlots));
     }
     scatter_z_halo(f, n, dst);

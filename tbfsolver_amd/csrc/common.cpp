@@ -179,6 +179,7 @@ std::mutex g_ring_mu;
 // the idle ones (never destroyed: at exit the runtime may be gone before statics)
 std::vector<std::unique_ptr<HostRing>>& g_rings = *new std::vector<std::unique_ptr<HostRing>>();
 int g_ring_users = 0;                            // live solver handles
+bool g_ring_called = false;                      // a ring was taken since there are any
 }  // namespace
 
 HostRing::~HostRing()
@@ -190,13 +191,20 @@ HostRing::~HostRing()
 
 int host_ring_take(const int32_t* n, std::unique_ptr<HostRing>& out)
 {
-    const size_t need = std::max(HostRing::kSlotBytes / 8, (size_t)n[0] * n[1]);
+    const size_t plane = (size_t)n[0] * n[1], cells = plane * (size_t)n[2];
+    const size_t slot = std::min(std::max(HostRing::kSlotBytes / 8, plane), cells);
+    const size_t chunks = ceil_div((size_t)n[2], slot / plane);
+    const size_t need = slot * std::min<size_t>(HostRing::kSlots, chunks);
     int dev = 0;
+    bool pageable = false;
     TBFG_HIP(hipGetDevice(&dev));
     {
         std::lock_guard<std::mutex> lk(g_ring_mu);
+        pageable = need * 8 <= (g_ring_called ? HostRing::kPageable : HostRing::kPageableFirst);
+        g_ring_called = true;
         for (auto& r : g_rings)
-            if (r->dev == dev && r->slot >= need) {
+            if (r->dev == dev && r->capacity >= need && (r->pin == nullptr) == pageable) {
+                r->slot = slot;
                 out = std::move(r);
                 r = std::move(g_rings.back());
                 g_rings.pop_back();
@@ -205,8 +213,14 @@ int host_ring_take(const int32_t* n, std::unique_ptr<HostRing>& out)
     }
     std::unique_ptr<HostRing> r(new HostRing());
     r->dev = dev;
-    r->slot = need;
-    TBFG_HIP(hipHostMalloc((void**)&r->pin, HostRing::kSlots * need * 8, hipHostMallocDefault));
+    r->capacity = need;
+    r->slot = slot;
+    if (pageable) {
+        r->page.resize(need);
+        out = std::move(r);
+        return TBFG_OK;
+    }
+    TBFG_HIP(hipHostMalloc((void**)&r->pin, need * 8, hipHostMallocDefault));
     for (hipEvent_t& e : r->ev) TBFG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     out = std::move(r);
     return TBFG_OK;
@@ -215,7 +229,14 @@ int host_ring_take(const int32_t* n, std::unique_ptr<HostRing>& out)
 void host_ring_give(std::unique_ptr<HostRing> r)
 {
     std::lock_guard<std::mutex> lk(g_ring_mu);
-    if (g_ring_users > 0 && g_rings.size() < (size_t)kHostRingsKept) g_rings.push_back(std::move(r));
+    if (g_ring_users == 0) return;
+    if (g_rings.size() < (size_t)kHostRingsKept) {
+        g_rings.push_back(std::move(r));
+        return;
+    }
+    auto least = std::min_element(g_rings.begin(), g_rings.end(),
+                                  [](const auto& a, const auto& b) { return a->capacity < b->capacity; });
+    if ((*least)->capacity < r->capacity) std::swap(*least, r);
 }
 
 HostRingUser::HostRingUser()
@@ -227,7 +248,10 @@ HostRingUser::HostRingUser()
 HostRingUser::~HostRingUser()
 {
     std::lock_guard<std::mutex> lk(g_ring_mu);
-    if (--g_ring_users == 0) g_rings.clear();
+    if (--g_ring_users == 0) {
+        g_rings.clear();
+        g_ring_called = false;
+    }
 }
 
 template <class T>

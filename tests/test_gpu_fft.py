@@ -470,3 +470,88 @@ def test_host_arrays_in_chunks_equal_device_solve(torch_gpu, n, precision, halo)
     ref = np.pad(np.pad(ref, ((halo, halo), (0, 0), (0, 0)), mode="wrap"), ((0, 0), (0, 0), (halo, halo)), mode="wrap")
     assert np.array_equal(p, ref)
     fs.close()
+
+
+# fields of 256 KB (ordinary memory), 608 KB (that in the first call, pinned after it), 2 MB (one pinned chunk),
+# 4.5 MB (two chunks), 9 MB (three)
+_HOST_SIZES = [(32, 32, 32), (36, 44, 48), (64, 64, 64), (128, 64, 72), (96, 96, 128)]
+
+
+def _host_case(torch, n, seed, precision="fp64"):
+    g, _ = grids(n, 1)
+    s = np.asfortranarray(np.random.default_rng(seed).standard_normal(n))
+    fs = T.FastPoissonSolver(g, precision=precision)
+    ref = torch.zeros_like(to_dev(s, torch))
+    fs.solveFPS(ref, to_dev(s, torch))
+    torch.cuda.synchronize()
+    return fs, s, to_host(ref)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_host_staging_over_sizes_and_handles(torch_gpu, precision):
+    """Staging memory passes from one handle and size to the next (a larger ring serves a smaller field and not
+    the other way round), is given back with the last handle and taken anew: each call equals the device solve
+    bit for bit, from the first on."""
+    print("case host staging", precision, flush=True)
+    order = _HOST_SIZES + _HOST_SIZES[::-1]
+    for n in _HOST_SIZES:  # each alone: staging given back in between
+        fs, s, ref = _host_case(torch_gpu, n, 5, precision)
+        for _ in range(3):
+            p = np.zeros(n, order="F")
+            fs.solveFPS(p, s)
+            assert np.array_equal(p, ref), n
+        fs.close()
+    held = [_host_case(torch_gpu, n, 7 + i, precision) for i, n in enumerate(order)]
+    for _ in range(2):
+        for fs, s, ref in held:
+            p = np.zeros_like(s)
+            fs.solveFPS(p, s)
+            assert np.array_equal(p, ref)
+    for fs, s, ref in held:
+        fs.close()
+
+
+def test_host_calls_from_threads(torch_gpu):
+    """Host calls of several handles at once, each thread in staging memory of its own, more threads than idle
+    rings are kept: every result equals the device solve bit for bit."""
+    import threading
+
+    print("case host threads", flush=True)
+    held = [_host_case(torch_gpu, _HOST_SIZES[i % 5], 20 + i) for i in range(7)]
+    bad = []
+
+    def work(fs, s, ref):
+        for _ in range(6):
+            p = np.zeros_like(s)
+            fs.solveFPS(p, s)
+            if not np.array_equal(p, ref):
+                bad.append(s.shape)
+
+    threads = [threading.Thread(target=work, args=h) for h in held]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+    for fs, _, _ in held:
+        fs.close()
+
+
+@pytest.mark.parametrize("n", [(32, 32, 32), (40, 40, 48), (64, 48, 64), (128, 64, 80)])
+def test_host_pcg_equals_device_solve(torch_gpu, n):
+    """The PCG's host call (three arrays in, one out) through each form of the staging: the device solve's bits."""
+    print("case host pcg", n, flush=True)
+    g, _ = grids(n, 1)
+    r = np.random.default_rng(11)
+    beta, q = np.asfortranarray(np.exp(r.uniform(-1, 1, n))), np.asfortranarray(r.standard_normal(n))
+    s = T.PCG(g, nLevels=2, tolPCG=1e-8, maxIterPCG=8, flexible=1, precision="mixed")
+    start = np.asfortranarray(r.standard_normal(n))
+    ref = to_dev(start, torch_gpu)
+    s.solvePCG(ref, to_dev(beta, torch_gpu), to_dev(q, torch_gpu))
+    out = (s.iterations, s.converged)
+    for _ in range(3):
+        psi = start.copy(order="F")
+        s.solvePCG(psi, beta, q)
+        assert (s.iterations, s.converged) == out
+        assert np.array_equal(psi, to_host(ref))
+    s.close()
