@@ -1699,6 +1699,6 @@ int fps_host_fields(tbfg_fps* h, double** s, double** p)
     return TBFG_OK;
 }
 
-int64_t fps_footprint(const tbfg_fps* h) { return h ? h->footprint : 0; }
+int64_t fps_footprint(const tbfg_fps* h) { return h ? h->footprint + (int64_t)(h->hs.bytes + h->hp.bytes) : 0; }
 
 }  // namespace tbfg

@@ -555,3 +555,16 @@ def test_host_pcg_equals_device_solve(torch_gpu, n):
         assert (s.iterations, s.converged) == out
         assert np.array_equal(psi, to_host(ref))
     s.close()
+
+
+@pytest.mark.parametrize("precision,fields", [("fp64", 0), ("mixed", 2)])
+def test_footprint_counts_the_host_call_fields(torch_gpu, precision, fields):
+    """The device fields that a handle keeps from its first host call on are in its footprint."""
+    n = (32, 10, 36)
+    print("case host footprint", precision, flush=True)
+    fs, s, ref = _host_case(torch_gpu, n, 2, precision)
+    before = fs.footprint
+    for _ in range(2):
+        fs.solveFPS(np.zeros_like(s), s)
+        assert fs.footprint == before + fields * 8 * n[0] * n[1] * n[2]
+    fs.close()
