@@ -938,3 +938,81 @@ def test_tuned_operator_below_the_pairs_limit(torch_gpu, monkeypatch, shape, til
     assert not np.array_equal(tuned[2], plain[2])
     if shape[0] < 0:
         assert tuned[1] == plain[1] - 8 * n[0] * n[1] * n[2]
+
+
+@pytest.mark.parametrize("precision,shape", [("fp64", "64x4x128"), ("fp64", "64x8x256"), ("fp64", "32x8x128"),
+                                             ("mixed", "64x8x256"), ("mixed", "32x16x256"), ("mixed", "64x16x512"),
+                                             ("mixed", "32x8x128")])
+def test_staged_tiles_match_half_sweeps_and_separate_dots(torch_gpu, monkeypatch, precision, shape):
+    """The staged-tile sweep in every shape it has (asked for by TBFG_SWEEP_SHAPE, or rows would take these
+    levels): the V-cycle of the half-sweep launches, and with the dot products in its last sweep the solve of
+    their separate pass.  Bounds of the same tests on the built-in choice."""
+    n = (128, 96, 64)
+    print("case staged tiles", precision, shape, flush=True)
+    monkeypatch.setenv("TBFG_SWEEP_MIN_CELLS", "0")
+    g, go, rho, _, q, beta = bubble_case(n, 8, 1, 5)
+    dq, db = to_dev(q, torch_gpu), to_dev(beta, torch_gpu)
+
+    def cycle():
+        s = T.PCG(g, nLevels=4, precision=precision)
+        z = torch_gpu.zeros_like(dq)
+        s.precondition(db, dq, z)
+        out = to_host(z)
+        s.close()
+        return out
+
+    rows = cycle()
+    monkeypatch.setenv("TBFG_SWEEP_SHAPE", shape)
+    tiles = cycle()
+    out = []
+    for unfused in (False, True):
+        if unfused:
+            monkeypatch.setenv("TBFG_UNFUSED_DOTS", "1")
+        s = T.PCG(g, nLevels=4, tolPCG=1e-10, maxIterPCG=200, precision=precision, flexible=1)
+        psi = torch_gpu.zeros_like(dq)
+        s.solvePCG(psi, db, dq)
+        assert s.converged
+        out.append((s.iterations, mean_free(to_host(psi))))
+        s.close()
+    monkeypatch.setenv("TBFG_HALF_SWEEPS", "1")
+    assert np.all(np.isfinite(tiles)) and rel(tiles, cycle()) < (1e-13 if precision == "fp64" else 1e-6)
+    assert not np.array_equal(tiles, rows)
+    assert abs(out[0][0] - out[1][0]) <= 1
+    assert rel(out[0][1], out[1][1]) < (1e-10 if precision == "fp64" else 1e-9)
+
+
+@pytest.mark.parametrize("tile", ["64x256", "32x256", "128x512", "64x512"])
+@pytest.mark.parametrize("precision,precond", [("fp64", "mg"), ("mixed", "mg"), ("mixed", "fft")])
+def test_marching_operator_with_direction_matches_separate_kernels(torch_gpu, monkeypatch, precision, precond, tile):
+    """The plane-marching operator, whose tiles are asked for here (a thread per pair takes this size otherwise):
+    with the direction and the deferred pressure update inside it gives the solve of the separate kernels bit for
+    bit, at the iteration limit, converged, from a warm start and for a zero right-hand side."""
+    n = (128, 96, 64)
+    print("case marching operator", precision, precond, tile, flush=True)
+    monkeypatch.setenv("TBFG_OP_TILE", tile)
+    g, go, rho, _, q, beta = bubble_case(n, 12, 1, 37)
+    dq, db = to_dev(q, torch_gpu), to_dev(beta, torch_gpu)
+    zero = torch_gpu.zeros_like(dq)
+
+    def run(unfused, most, rhs, start):
+        if unfused:
+            monkeypatch.setenv("TBFG_UNFUSED_OP", "1")
+        else:
+            monkeypatch.delenv("TBFG_UNFUSED_OP", raising=False)
+        s = T.PCG(g, nLevels=4, tolPCG=1e-9, maxIterPCG=most, precision=precision, flexible=1,
+                  coarse_max_iter=0, preconditioner=precond)
+        psi = start.clone()
+        s.solvePCG(psi, db, rhs)
+        out = (s.iterations, s.converged, s.res_, psi)
+        s.close()
+        return out
+
+    conv = run(False, 300, dq, zero)
+    assert conv[1]
+    for most, rhs, start in ((1, dq, zero), (3, dq, zero), (300, dq, zero), (300, dq, conv[3]), (50, zero, zero)):
+        a, b = run(False, most, rhs, start), run(True, most, rhs, start)
+        assert a[:3] == b[:3] and torch_gpu.equal(a[3], b[3])
+        if most <= 3:
+            assert a[0] == most and not a[1]
+        if start is conv[3]:
+            assert a[1] and a[0] <= 1 and (a[0] or torch_gpu.equal(a[3], start))
