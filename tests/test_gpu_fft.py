@@ -568,3 +568,31 @@ def test_footprint_counts_the_host_call_fields(torch_gpu, precision, fields):
         fs.solveFPS(np.zeros_like(s), s)
         assert fs.footprint == before + fields * 8 * n[0] * n[1] * n[2]
     fs.close()
+
+
+@pytest.mark.parametrize("n", [(64, 1, 4), (96, 2, 6), (36, 7, 2)])
+def test_fast_projection_leaves_the_wall_faces(torch_gpu, n):
+    """Wall faces of any value keep their bits (with one row in y every y face is one), interior faces follow the
+    oracle to 1e-12; the source reads the wall faces' velocity and surface tension, to 1e-13."""
+    print("case fast wall faces", n, flush=True)
+    g, go = grids(n, 1)
+    nx, ny, nz = n
+    r = np.random.default_rng(15)
+    u = [np.asfortranarray(r.standard_normal(s)) for s in ((nx, ny, nz), (nx, ny + 1, nz), (nx, ny, nz))]
+    rho = np.asfortranarray(r.uniform(0.05, 1.0, n))
+    psi, psi1, psi2 = (np.asfortranarray(r.standard_normal(n)) for _ in range(3))
+    st1, st2 = random_st(n), random_st(n)
+    adt, rho0 = 1e-3, 0.05
+    dev = lambda a: to_dev(a, torch_gpu)  # noqa: E731
+    du, d1, d2 = [dev(a) for a in u], tuple(dev(a) for a in st1), tuple(dev(a) for a in st2)
+    s = torch_gpu.zeros_like(dev(rho))
+    F.computeSourceFast(g, adt, rho0, dev(rho), *du, s, dev(psi1), dev(psi2), d1, d2)
+    assert rel(to_host(s), O.source_fast(go, adt, rho0, rho, *u, psi1, psi2, st1, st2)) < 1e-13
+    F.makeVelocityDivFreeFast(g, adt, rho0, dev(rho), dev(psi), *du, dev(psi1), dev(psi2), d1, d2)
+    torch_gpu.cuda.synchronize()
+    got = [to_host(a) for a in du]
+    ref = O.project_fast(go, adt, rho0, rho, psi, psi1, psi2, *u, st1, st2)
+    assert rel(got[0], ref[0]) < 1e-12 and rel(got[2], ref[2]) < 1e-12
+    assert np.array_equal(got[1][:, [0, ny]], u[1][:, [0, ny]])
+    if ny > 1:
+        assert rel(got[1][:, 1:ny], ref[1][:, 1:ny]) < 1e-12
