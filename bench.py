@@ -649,7 +649,7 @@ def main():
         achieved = bytes_per / avg_s / 1e9
         out["roofline_sweep_fine"] = {
             "bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-            "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None,  # (counted for the tiled sweep only)
+            "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic_of("sweep_fine_traffic.json"),
             "kernel": "k_row_sweep<float, bf16s, bf16s, false, false, true>: finest-level red/black sweep "
                       "from a non-zero start, out of place (p FP32 in and out, q and beta bf16 in: 12 B per cell)",
             "avg_us": round(avg_s * 1e6, 2), "launches": launches, "algorithmic_bytes_per_launch": bytes_per}
